@@ -124,7 +124,7 @@ def write_traffic(fetch_dir, write_dir, launches):
         rows.sort()
         return rows
 
-    kinds = {"fp_ratio": "fp_kernel<4, 1, 1, true>", "backproject": "bp_inc_kernel",
+    kinds = {"fp_ratio": "fp_kernel<3, 2, 1, true>", "backproject": "bp_inc_kernel",
              "rotate_update": "rot_update_kernel<false>"}
     cal_bytes = 256 << 20
     out = {}

@@ -1,8 +1,8 @@
 """Launch-shape autotuner for the projectors.
 
 The forward projector's workgroup owns planes of one ray column (one x of
-one view pair); the shape picks how many planes each thread accumulates in
-registers and how many workgroups share one column (each recomputing the
+one view pair); the shape picks whether each thread accumulates one plane or a
+run of three, and how many workgroups share one column (each recomputing the
 column's rotated samples).  The back
 projector's workgroup stages one sinogram column in LDS; its shape is the
 number of waves (voxel rows in flight) sharing that column.  Results are

@@ -381,14 +381,17 @@ extern "C" int hrrt_create(const hrrt_params *params, hrrt_ctx **out) {
     // ym of the segment and its position advanced by yr - ym (PJ:1929-1944), so the device
     // repeats the tables' float operations exactly.  Rows below ymin are skipped
     // (PJ:1920-1921); the skip rule is checked to hold for exactly the rows below a threshold.
-    std::vector<int4> fplanes;
-    int fp_fast = 1;   // positions never negative: the forward projector may take fract for zz - (int)zz
-    for (int yr = 0; yr < Z; yr++) fplanes.push_back(make_int4(yr << 8, 0, 0, 0));
+    std::vector<int4> fruns[2], fsingle;   // runs of one and of three middle planes, all other planes
+    int fp_fast = 1;   // no row skipped, positions never negative: fract for zz - (int)zz, no row test
+    int first_row = c;   // of any ray
+    for (int x = 1; x <= c; x++)
+        if (G.cyl_lo[x] != G.cyl_hi[x]) first_row = std::min(first_row, G.cyl_lo[x]);
     for (int k = 1; k <= G.K; k++) {
         const int th = 2 * k, yb = G.yr_bottom[th], yt = G.yr_top[th], ym = yb + ZS;
         int ymin = 1;
         for (int y = 1; y < c; y++)
             if (skip[(size_t)y * GM + k - 1]) ymin = y + 1;
+        if (ymin > first_row) fp_fast = 0;
         for (int y = ymin; y < c; y++)
             if (skip[(size_t)y * GM + k - 1]) {
                 delete ctx;
@@ -399,12 +402,18 @@ extern "C" int hrrt_create(const hrrt_params *params, hrrt_ctx **out) {
             const int base = end ? yr : ym, delta = end ? 0 : yr - ym;
             const float bf = (float)base;
             const float t = G.tantheta[(size_t)(k - 1) * Z + base];
-            fplanes.push_back(make_int4(k | (yr << 8) | (delta << 16), bits(bf), bits(t), ymin));
+            if (end) fsingle.push_back(make_int4(k | (yr << 8) | (1 << 16), bits(bf), bits(t), ymin << 16));
+            else
+                for (int n = 1; n <= 3; n += 2)
+                    if (delta % n == 0) {
+                        const int cnt = std::min(n, yt - ZS - yr + 1);
+                        fruns[n == 3].push_back(make_int4(k | (yr << 8) | (cnt << 16), bits(bf), bits(t), delta | (ymin << 16)));
+                    }
             // the device recomputes what the tables hold: check it on the host for every row
             for (int y = ymin; y < c; y++) {
                 const float zz1 = bf + (y - c) * t, zz2 = bf + (c - y) * t;
                 const int z1 = (int)zz1, z2 = (int)zz2;
-                if (zz1 < 0.0f || zz2 < 0.0f) fp_fast = 0;
+                if (y >= first_row && (zz1 < 0.0f || zz2 < 0.0f)) fp_fast = 0;
                 int rz, rz2;
                 float rf1, rf2;
                 const size_t li = (size_t)y * GM + k - 1;
@@ -424,6 +433,7 @@ extern "C" int hrrt_create(const hrrt_params *params, hrrt_ctx **out) {
             }
         }
     }
+    for (int yr = 0; yr < Z; yr++) fsingle.push_back(make_int4((yr << 8) | (1 << 16), 0, 0, 0));   // axial planes last
     std::vector<int16_t> pseg(G.spp, -1), plane_seg(G.segmentsize, 0);
     for (int s = 0; s < G.th_pixels; s++)
         for (int i = 0; i < G.nplanes(s); i++) {
@@ -595,7 +605,8 @@ extern "C" int hrrt_create(const hrrt_params *params, hrrt_ctx **out) {
         (r = ctx->upload(G.seg_data, d.seg_data)) || (r = ctx->upload(G.segment_offset, d.segment_offset)) ||
         (r = ctx->upload(file_seg, d.file_seg)) || (r = ctx->upload(G.bp_rescale, d.bp_rescale)) ||
         (r = ctx->upload(resc, d.rescalearray)) || (r = ctx->upload(blut, d.bp_lut)) ||
-        (r = ctx->upload(rot, d.rot)) || (r = ctx->upload(fplanes, d.fp_planes)) || (r = ctx->upload(pseg, d.pseg)) ||
+        (r = ctx->upload(rot, d.rot)) || (r = ctx->upload(fruns[0], d.fp_runs[0])) ||
+        (r = ctx->upload(fruns[1], d.fp_runs[1])) || (r = ctx->upload(fsingle, d.fp_single)) || (r = ctx->upload(pseg, d.pseg)) ||
         (r = ctx->upload(plane_seg, d.plane_seg)) || (r = ctx->upload(bp_src, d.bp_src)) ||
         (r = ctx->upload(blut2, d.bp_lut2)) || (r = ctx->upload(isrc, d.inc_src)) ||
         (r = ctx->upload(iconv, d.inc_conv)) || (r = ctx->upload(igroup, d.inc_group)) ||
@@ -603,9 +614,10 @@ extern "C" int hrrt_create(const hrrt_params *params, hrrt_ctx **out) {
         delete ctx;
         return r;
     }
-    d.fp_np = (int)fplanes.size();
+    for (int n = 0; n < 2; n++) d.fp_nr[n] = (int)fruns[n].size();
+    d.fp_ns = (int)fsingle.size();
     d.fp_fast = fp_fast;
-    d.fp_maxt = 4;
+    d.fp_maxt = 0;
     d.fp_nsplit = 0;
     d.bp_waves = 16;
     ctx->bp_threads = d.inc_ok ? 1 : 0;                                 // every pair incremental when possible
@@ -1020,8 +1032,8 @@ static int frames_subset_launch(hrrt_ctx *ctx, int nframes, float *d_images, con
     ctx->mark(0, s);
     HIP_TRY(hrrt::launch_forward(ctx->dg, b, d_images, ctx->f_ratio, io, pr.mixed ? hrrt::FP_RATIO16 : hrrt::FP_RATIO, s));
     if (pr.mixed && pr.loglik) {
-        int maxt, nsplit, threads, items;
-        hrrt::forward_shape(ctx->dg, maxt, nsplit, threads, items);
+        int run, nsplit, threads;
+        hrrt::forward_shape(ctx->dg, b.npairs * nframes, run, nsplit, threads);
         HIP_TRY(hrrt::launch_ll_reduce(ctx->ll_part, ctx->dg.c * nsplit * b.npairs, nframes, pr.loglik, s));
     }
     // the subset update back-projects under the schedule in both forms (incremental by default);
@@ -1044,8 +1056,8 @@ static int frames_check(hrrt_ctx *ctx, int nframes, const void *a, const void *b
         return fail(HRRT_ERR_ARG, "too many frames for one launch (%d)", nframes);
     int r;
     if ((r = ctx->ensure_frame_scratch(nframes))) return r;
-    int maxt, nsplit, threads, items;
-    hrrt::forward_shape(ctx->dg, maxt, nsplit, threads, items);
+    int run, nsplit, threads;
+    hrrt::forward_shape(ctx->dg, ctx->npairs() * nframes, run, nsplit, threads);
     return ctx->ensure_ll_part((size_t)ctx->dg.c * nsplit * ctx->npairs() * nframes);
 }
 

@@ -25,10 +25,12 @@ struct DevGeom {
     const int4 *bp_lut2;                 // [N][GM]: {zsa | zea << 16, LDS index of plane 0 of the shifted
                                          //  segment 2k, of segment 2k-1, bits(frac)}
     const float2 *rot;                   // [views/2][N][N] rotation sample positions (rotateimage2 order)
-    const int4 *fp_planes;               // [fp_np] forward-projector planes, axial first, then by (k, yr):
-                                         //  {k | yr << 8 | delta << 16, bits(base plane), bits(tan), ymin}
-    int fp_np;
-    int fp_fast;                         // 1: every forward position of a row the kernel projects is >= 0
+    // forward-projector planes by (k, yr): {k | yr << 8 | planes << 16, bits(base plane), bits(tan),
+    // delta | ymin << 16}; runs of one and of up to three middle planes of a group, and the end and
+    // axial (k = 0) planes one by one
+    const int4 *fp_runs[2], *fp_single;
+    int fp_nr[2], fp_ns;
+    int fp_fast;                         // 1: no ray skips a row and every forward position is >= 0
     const int16_t *pseg;                 // [spp] padded plane -> segment (-1 on guards)
     const int16_t *plane_seg;            // [S] internal plane -> segment
     const int *bp_src;                   // [bp_lds + 1] LDS entry -> pair-column plane (-1 = zero)
@@ -43,7 +45,7 @@ struct DevGeom {
     const int4 *inc_group;               // [K][4] per group: window, first-row lookups, row c+1 breakpoint
     const int4 *inc_sched;               // [n+1] breakpoints of rows c-2 down to 1, groups ascending
     const int *inc_nrow;                 // [c+1] breakpoints of row y
-    int fp_maxt, fp_nsplit;              // forward-projector launch shape (tasks/thread, workgroups/(pair,x))
+    int fp_maxt, fp_nsplit;              // forward-projector launch shape asked for (tasks/thread, workgroups/(pair,x)), 0: by rule
     int bp_waves;                        // back-projector waves per workgroup
 };
 
@@ -74,8 +76,9 @@ struct FpIO {
 
 hipError_t launch_forward(const DevGeom &g, const PairBatch &b, const float *image, float *out_paircol,
                           const FpIO &io, int mode, hipStream_t s);
-// launch shape the forward projector uses (workgroups per ray = nsplit, planes per thread = maxt)
-void forward_shape(const DevGeom &g, int &maxt, int &nsplit, int &threads, int &items);
+// launch shape the forward projector uses for npf (view pair, frame) combinations (workgroups per ray
+// = nsplit, middle planes per thread = run)
+void forward_shape(const DevGeom &g, int npf, int &run, int &nsplit, int &threads);
 // src: float pair-column, or FP16 bits when src_half; kahan: compensated accumulation over groups
 hipError_t launch_backproject(const DevGeom &g, const PairBatch &b, const void *src_paircol, int src_half,
                               int src_global, int apply_rescale, int kahan, float *bufA, float *bufB, hipStream_t s);

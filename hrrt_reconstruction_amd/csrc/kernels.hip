@@ -8,6 +8,7 @@
 // FIO = hrrt_osem3d/file_io_processor.cpp.
 #include "kernels.h"
 
+#include <algorithm>
 #include <type_traits>
 
 #pragma clang fp contract(off)
@@ -33,131 +34,33 @@ __device__ __forceinline__ void kahan_add(float &s, float &c, float x) {
     s = t;
 }
 
+// f(0), f(1), ..., f(N - 1) with the index as a constant
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void unroll(F &&f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        unroll<N, I + 1>(f);
+    }
+}
+
 __device__ __forceinline__ float lane(const float4 &v, int l) {
     return l == 0 ? v.x : (l == 1 ? v.y : (l == 2 ? v.z : v.w));
-}
-
-// Bilinear sample of the z-column chunk q (4 planes) at the rotated position of
-// (xx, yy) (PJ:1865-1892).  Returns false when the reference rejects the sample.
-__device__ __forceinline__ bool sample_chunk(const DevGeom &g, const float4 *__restrict__ image, float cosv,
-                                             float sinv, int xx, int yy, int q, float4 &out) {
-    const int c = g.c, N = g.N;
-    float xx0 = (xx - c) * cosv - (yy - c) * sinv + c;
-    float yy0 = (xx - c) * sinv + (yy - c) * cosv + c;
-    if (xx0 < 0 || xx0 > N - 2 || yy0 < 0 || xx0 > N - 2) return false;
-    int xi = (int)xx0, yi = (int)yy0;
-    float x1 = xx0 - xi, y1 = yy0 - yi;
-    float w1 = (1 - x1) * (1 - y1), w2 = x1 * (1 - y1), w3 = y1 * (1 - x1), w4 = y1 * x1;
-    const size_t NQ = g.NQ;
-    float4 r1 = image[((size_t)xi * N + yi) * NQ + q];
-    float4 r2 = image[((size_t)(xi + 1) * N + yi) * NQ + q];
-    float4 r3 = image[((size_t)xi * N + yi + 1) * NQ + q];
-    float4 r4 = image[((size_t)(xi + 1) * N + yi + 1) * NQ + q];
-    out = add4(add4(mul4(r1, w1), mul4(r2, w2)), add4(mul4(r3, w3), mul4(r4, w4)));
-    return true;
-}
-
-__device__ __forceinline__ void put_lanes(float4 *buf, int q, int lanei, float4 v, int Z) {
-    float *f = reinterpret_cast<float *>(buf);
-    int z = 4 * q;
-    if (z + 0 < Z) f[(z + 0) * 4 + lanei] = v.x;
-    if (z + 1 < Z) f[(z + 1) * 4 + lanei] = v.y;
-    if (z + 2 < Z) f[(z + 2) * 4 + lanei] = v.z;
-    if (z + 3 < Z) f[(z + 3) * 4 + lanei] = v.w;
 }
 
 // The eight symmetric sample positions of (x, y) (PJ:1856-1864).  Samples 0..3
 // feed "pam" (near half of the ray), 4..7 feed "pam2" (mirrored half).
 // i: (x, y), (N-x, y), (N-y, x), (N-y, N-x), (x, N-y), (N-x, N-y), (y, x), (y, N-x).  Bit 0
-// mirrors x, bit 1 swaps the two coordinates, bit 2 mirrors y; as selects rather than a branch
-// tree, since the sample index differs between the 16-lane rows of a wave.
-__device__ __forceinline__ void sym8(int i, int x, int y, int N, int &xx, int &yy) {
-    const int X = (i & 1) ? N - x : x;
-    const int Yd = (i & 4) ? N - y : y;   // y coordinate of the unswapped samples
-    const int Ys = (i & 4) ? y : N - y;   // x coordinate of the swapped samples
-    xx = (i & 2) ? Ys : X;
-    yy = (i & 2) ? X : Yd;
-}
-
-__device__ __forceinline__ void sample8(const DevGeom &g, const float4 *__restrict__ image, float cosv, float sinv,
-                                        int x, int y, float4 *pam, float4 *pam2) {
-    const int NQ = g.NQ, N = g.N;
-    for (int it = threadIdx.x; it < 8 * NQ; it += blockDim.x) {
-        int i = it / NQ, q = it - i * NQ;
-        int xx, yy;
-        sym8(i, x, y, N, xx, yy);
-        float4 v;
-        if (!sample_chunk(g, image, cosv, sinv, xx, yy, q, v)) v = f4(0.f);
-        put_lanes(i < 4 ? pam : pam2, q, i & 3, v, g.Z);
-    }
-}
-
-// Two-phase version of sample8 for software pipelining: issue the global loads
-// of the next y into registers, project the current y, then combine and store.
-// Each thread owns ITEMS of the 8*NQ (sample, 4-plane chunk) items.
-template <int ITEMS>
-struct SampleRegs {
-    float4 r1[ITEMS], r2[ITEMS], r3[ITEMS], r4[ITEMS];
-    float w1[ITEMS], w2[ITEMS], w3[ITEMS], w4[ITEMS];
-    bool ok[ITEMS];
-};
-
-template <int ITEMS>
-__device__ __forceinline__ void sample8_load(const DevGeom &g, const float4 *__restrict__ image, float cosv,
-                                             float sinv, int x, int y, SampleRegs<ITEMS> &s) {
-    const int NQ = g.NQ, N = g.N, c = g.c;
-#pragma unroll
-    for (int j = 0; j < ITEMS; j++) {
-        const int it = threadIdx.x + j * blockDim.x;
-        s.ok[j] = false;
-        if (it >= 8 * NQ) continue;
-        const int i = it / NQ, q = it - i * NQ;
-        int xx, yy;
-        sym8(i, x, y, N, xx, yy);
-        const float xx0 = (xx - c) * cosv - (yy - c) * sinv + c;
-        const float yy0 = (xx - c) * sinv + (yy - c) * cosv + c;
-        if (xx0 < 0 || xx0 > N - 2 || yy0 < 0 || xx0 > N - 2) continue;
-        const int xi = (int)xx0, yi = (int)yy0;
-        const float x1 = xx0 - xi, y1 = yy0 - yi;
-        s.w1[j] = (1 - x1) * (1 - y1); s.w2[j] = x1 * (1 - y1); s.w3[j] = y1 * (1 - x1); s.w4[j] = y1 * x1;
-        const float4 *p = image + ((size_t)xi * N + yi) * NQ + q;
-        s.r1[j] = p[0];
-        s.r2[j] = p[(size_t)N * NQ];
-        s.r3[j] = p[NQ];
-        s.r4[j] = p[(size_t)N * NQ + NQ];
-        s.ok[j] = true;
-    }
-}
-
-template <int ITEMS>
-__device__ __forceinline__ void sample8_store(const DevGeom &g, const SampleRegs<ITEMS> &s, float4 *pam, float4 *pam2) {
-    const int NQ = g.NQ;
-#pragma unroll
-    for (int j = 0; j < ITEMS; j++) {
-        const int it = threadIdx.x + j * blockDim.x;
-        if (it >= 8 * NQ) continue;
-        const int i = it / NQ, q = it - i * NQ;
-        const float4 v = s.ok[j] ? add4(add4(mul4(s.r1[j], s.w1[j]), mul4(s.r2[j], s.w2[j])),
-                                        add4(mul4(s.r3[j], s.w3[j]), mul4(s.r4[j], s.w4[j])))
-                                 : f4(0.f);
-        put_lanes(i < 4 ? pam : pam2, q, i & 3, v, g.Z);
-    }
-}
-
-// Transposed staging of a row (the FAST forward path).  A wave owns 16 chunks (4 planes
+// mirrors x, bit 1 swaps the two coordinates, bit 2 mirrors y.
+//
+// Transposed staging of a row.  A wave owns 16 chunks (4 planes
 // each) of one half of the row's samples: lane l samples chunk 16 b + (l & 15) of sample
 // 4 h + (l >> 4), so each row of 16 lanes loads 256 contiguous bytes of one image column.
 // A 4x4 transpose across the four 16-lane rows (two permlane32 swaps, then two permlane16
 // swaps) leaves lane l with plane 4 q + (l >> 4) of all four samples, stored with one
 // 16-byte LDS write instead of four scattered 4-byte ones.
-__device__ __forceinline__ int xpose_chunks(const DevGeom &g) { return 2 * ((g.NQ + 15) >> 4); }
-
-__device__ __forceinline__ void xpose_item(const DevGeom &g, int it, int &h, int &q, int &i) {
-    const int nq16 = (g.NQ + 15) >> 4, chunk = it >> 6, l = it & 63;
-    h = chunk >= nq16;
-    q = 16 * (chunk - h * nq16) + (l & 15);
-    i = 4 * h + (l >> 4);
-}
+// Staged planes per column: at most 256 image planes and the zero plane behind them, as a
+// constant so that every LDS read of a row takes its buffer and neighbour as immediate offsets.
+constexpr int FP_PL = 264;
 
 __device__ __forceinline__ void swap_pl32(float &a, float &b) {
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
@@ -180,60 +83,88 @@ __device__ __forceinline__ float4 xpose4(float4 v) {
     return v;
 }
 
-template <int ITEMS>
-__device__ __forceinline__ void sample8x_load(const DevGeom &g, const float4 *__restrict__ image, float cosv,
-                                              float sinv, int x, int y, SampleRegs<ITEMS> &s) {
+// One bilinear sample of a z chunk (PJ:1865-1892), its four neighbours in flight.
+struct Sample {
+    float4 r1, r2, r3, r4;
+    float x1, y1;
+    bool ok;
+};
+
+__device__ __forceinline__ void sample_load(const DevGeom &g, const float4 *__restrict__ image, float cosv, float sinv,
+                                            float dx, float dy, int q, Sample &s) {
     const int NQ = g.NQ, N = g.N, c = g.c;
-#pragma unroll
-    for (int j = 0; j < ITEMS; j++) {
-        const int it = threadIdx.x + j * blockDim.x;
-        s.ok[j] = false;
-        if ((it >> 6) >= xpose_chunks(g)) continue;
-        int h, q, i, xx, yy;
-        xpose_item(g, it, h, q, i);
-        if (q >= NQ) continue;
-        sym8(i, x, y, N, xx, yy);
-        const float xx0 = (xx - c) * cosv - (yy - c) * sinv + c;
-        const float yy0 = (xx - c) * sinv + (yy - c) * cosv + c;
-        if (xx0 < 0 || xx0 > N - 2 || yy0 < 0 || xx0 > N - 2) continue;
-        const int xi = (int)xx0, yi = (int)yy0;
-        const float x1 = xx0 - xi, y1 = yy0 - yi;
-        s.w1[j] = (1 - x1) * (1 - y1); s.w2[j] = x1 * (1 - y1); s.w3[j] = y1 * (1 - x1); s.w4[j] = y1 * x1;
-        // 32-bit chunk offsets from the uniform image base (an image holds < 2^32 chunks)
-        const unsigned o = ((unsigned)xi * (unsigned)N + (unsigned)yi) * (unsigned)NQ + (unsigned)q;
-        const unsigned dx = (unsigned)N * (unsigned)NQ;
-        s.r1[j] = image[o];
-        s.r2[j] = image[o + dx];
-        s.r3[j] = image[o + (unsigned)NQ];
-        s.r4[j] = image[o + dx + (unsigned)NQ];
-        s.ok[j] = true;
-    }
+    const float xx0 = dx * cosv - dy * sinv + c;
+    const float yy0 = dx * sinv + dy * cosv + c;
+    s.ok = q < NQ && !(xx0 < 0 || xx0 > N - 2 || yy0 < 0 || xx0 > N - 2);
+    if (!s.ok) return;
+    const int xi = (int)xx0, yi = (int)yy0;
+    s.x1 = xx0 - xi;
+    s.y1 = yy0 - yi;
+    // 32-bit chunk offsets from the uniform image base (an image holds < 2^32 chunks)
+    const unsigned o = ((unsigned)xi * (unsigned)N + (unsigned)yi) * (unsigned)NQ + (unsigned)q;
+    const unsigned nx = (unsigned)N * (unsigned)NQ;
+    s.r1 = image[o];
+    s.r2 = image[o + nx];
+    s.r3 = image[o + (unsigned)NQ];
+    s.r4 = image[o + nx + (unsigned)NQ];
 }
 
-template <int ITEMS>
-__device__ __forceinline__ void sample8x_store(const DevGeom &g, const SampleRegs<ITEMS> &s, float4 *pam,
-                                               float4 *pam2) {
-#pragma unroll
-    for (int j = 0; j < ITEMS; j++) {
-        const int it = threadIdx.x + j * blockDim.x;
-        if ((it >> 6) >= xpose_chunks(g)) continue;   // whole waves
-        int h, q, i;
-        xpose_item(g, it, h, q, i);
-        float4 v = s.ok[j] ? add4(add4(mul4(s.r1[j], s.w1[j]), mul4(s.r2[j], s.w2[j])),
-                                  add4(mul4(s.r3[j], s.w3[j]), mul4(s.r4[j], s.w4[j])))
-                           : f4(0.f);
-        v = xpose4(v);
-        const int z = 4 * q + (i & 3);
-        if (q < g.NQ && z < g.Z) (h ? pam2 : pam)[z] = v;
-    }
+// Combined and transposed: plane 4 q + (l >> 4) of the wave's four samples (every lane must call).
+__device__ __forceinline__ float4 sample_combine(const Sample &s) {
+    const float x1 = s.x1, y1 = s.y1;
+    const float w1 = (1 - x1) * (1 - y1), w2 = x1 * (1 - y1), w3 = y1 * (1 - x1), w4 = y1 * x1;
+    const float4 v = s.ok ? add4(add4(mul4(s.r1, w1), mul4(s.r2, w2)), add4(mul4(s.r3, w3), mul4(s.r4, w4))) : f4(0.f);
+    return xpose4(v);
 }
 
-// Workgroups are dispatched round-robin over the 8 XCDs (blockIdx k runs on XCD k mod 8),
-// each with its own L2.  This maps a dispatch index to a logical index such that every XCD
-// receives one contiguous range of logical indices, processed in order.
-__device__ __forceinline__ int xcd_contiguous(int bid, int nb) {
-    if (nb & 7) return bid;
-    return (bid & 7) * (nb >> 3) + (bid >> 3);
+// What a lane samples of every row: its item's position relative to the centre is linear in
+// fy = y - c (small integers, so these float operations are exact), its chunk and its LDS slot.
+struct SampleLane {
+    float kx, sx, ky, sy;
+    int q;      // chunk, NQ or more: nothing to load
+    int slot;   // float4 index in the row's two halves, negative: nothing to store
+};
+
+__device__ __forceinline__ SampleLane sample_lane(const DevGeom &g, int it, int x) {
+    SampleLane s;
+    const int nq16 = (g.NQ + 15) >> 4, chunk = it >> 6, l = it & 63;
+    const int h = chunk >= nq16 ? 1 : 0;
+    s.q = 16 * (chunk - h * nq16) + (l & 15);
+    const int i = 4 * h + (l >> 4), z = 4 * s.q + (i & 3);
+    if (chunk >= 2 * nq16) s.q = g.NQ;
+    s.slot = s.q < g.NQ && z < g.Z ? h * FP_PL + z : -1;
+    const float X = (float)((i & 1) ? g.c - x : x - g.c);       // x - c or its mirror
+    const float Yd = (i & 4) ? -1.f : 1.f, Ys = -Yd;             // coefficients of y - c
+    s.kx = (i & 2) ? 0.f : X;
+    s.sx = (i & 2) ? Ys : 0.f;
+    s.ky = (i & 2) ? X : 0.f;
+    s.sy = (i & 2) ? 0.f : Yd;
+    return s;
+}
+
+// Forward grid.  Workgroups are dispatched round-robin over the 8 XCDs (blockIdx k runs on XCD
+// k mod 8), each with its own L2.  A strip is FP_STRIP neighbouring rays of one (view pair,
+// frame), whose rotated rows share image columns; the strips of every pair and frame are ordered
+// from the centre (the longest rays) outwards and dealt to the XCDs in turn, so that an XCD
+// holds neighbouring rays at a time, all XCDs get the same work and the short rays come last (9 view
+// pairs at 256 x 256: 0.825 -> 0.783 ms against a contiguous range of rays per XCD, whose
+// longest took 520 rows of a CU's time where the mean is 434).
+constexpr int FP_STRIP = 16;
+static inline long long fp_blocks(int c, int npf, int nsplit) {
+    const long long items = (long long)((c + FP_STRIP - 1) / FP_STRIP) * npf;
+    return (items + 7) / 8 * 8 * FP_STRIP * nsplit;
+}
+__device__ __forceinline__ bool fp_block(const DevGeom &g, const PairBatch &b, int nsplit, int bid, int &frame, int &lp,
+                                         int &ray, int &split) {
+    const int npf = b.npairs * b.nframes, per = FP_STRIP * nsplit;
+    const int r = bid >> 3, k = r / per, j = r - k * per;
+    const int item = 8 * k + (bid & 7);
+    const int strip = item / npf, pf = item - strip * npf;
+    ray = strip * FP_STRIP + j / nsplit;
+    split = j % nsplit;
+    frame = pf / b.npairs;
+    lp = pf - frame * b.npairs;
+    return ray < g.c;
 }
 
 // Rotation grid: voxel column x and group of 4 rows yg.  Each XCD owns a band of row
@@ -259,86 +190,159 @@ __device__ __forceinline__ void rot_block(int bid, int N, int NYG, int &x, int &
 // S3:2493-2505) and the back-projection rescale (PJ:1638-1649).
 //
 // One workgroup per (view pair, x in [1, N/2], share of the planes).  The
-// eight rotated z-columns of each row y are staged in LDS (double buffered,
-// the next row's samples loaded into registers while the current row is
-// projected); every thread owns up to MAXT planes (consecutive planes on
-// consecutive lanes, so LDS reads are unit-stride) and accumulates each over
-// y in the reference's order.  A plane's axial positions for row y are
-// recomputed from per-plane constants with the float operations that build
-// the reference's flookup table and middle-plane positions (PJ:544-562,
-// 1929-1944), so every lane runs one code path.
+// eight rotated z-columns of each row y are staged in LDS (double buffered);
+// a thread accumulates its planes over y in the reference's order.  A plane's
+// axial positions for row y are recomputed from per-plane constants with the
+// float operations that build the reference's flookup table and middle-plane
+// positions (PJ:544-562, 1929-1944).
+//
+// The middle planes of a segment group share their positions up to the plane
+// shift, so a thread takes a run of RL of them: one position per row, and
+// 4 (RL + 1) LDS reads of 16 bytes in place of 8 RL.  End planes and axial
+// planes go one per thread (single).
+//
+// What bounds it: LDS reads and FP32 VALU, about equally (span 3, 9 view pairs at 256 x 256: 16 runs
+// and 5 singles of 64 lanes per row).  With one plane per thread slot and 8 reads per plane the LDS alone
+// took 2 of the 2.9 thousand cycles of a row.  RL = 3 is odd, so the 16 lanes of a quarter-wave read
+// 16 different bank groups, and its sums fit 128 registers with 16 waves in a CU: 0.69 -> 0.586 ms for
+// such a subset.  The samples of a step are loaded a whole step ahead and stored at its beginning,
+// so that no wave waits for memory before the barrier, and a step of 16 waves holds two
+// rows (0.70 -> 0.68 ms).
 // ---------------------------------------------------------------------------
-// Write-out of one plane of one segment for the four lanes (v, x), (v, N-x),
-// (v+90, x), (v+90, N-x) (PJ:1397-1436), optionally through the OP ratio
-// (S3:2493-2505) and the back-projection rescale (PJ:1638-1649).
-template <int MODE>
-__device__ __forceinline__ void fp_write1(const DevGeom &g, float4 acc, int seg, int yr, int x, int view, int lp,
-                                          float *__restrict__ out, const FpIO &io, double &ll) {
-    const int N = g.N;
-    const int pidx = g.seg_data[seg] + (yr - g.yb[seg]);
-    const float resc = g.bp_rescale[seg];
+// Axial sample positions of a plane in a row: LDS byte offsets of the two lower planes (the plane
+// shift included) and their fractions.
+struct FpPos {
+    int o1, o2;
+    float f1, f2;
+};
+
+template <bool FAST>
+__device__ __forceinline__ FpPos fp_pos(float base, float tan, float fy2, int dbyte) {
+    FpPos q;
+    const float pt = fy2 * tan;
+    const float zz1 = base - pt, zz2 = base + pt;
+    const int i1 = (int)zz1, i2 = (int)zz2;
+    if (FAST) {        // zz >= 0: zz - trunc(zz) = zz - floor(zz)
+        q.f1 = __builtin_amdgcn_fractf(zz1);
+        q.f2 = __builtin_amdgcn_fractf(zz2);
+    } else {
+        q.f1 = zz1 - i1;
+        q.f2 = zz2 - i2;
+    }
+    q.o1 = i1 * (int)sizeof(float4) + dbyte;
+    q.o2 = i2 * (int)sizeof(float4) + dbyte;
+    return q;
+}
+
+// PJ:1934-1944 for R consecutive planes: acc[j] += (pb[z2+1] + pa[z])*f2 + (pa[z+1] + pb[z2])*f1
+template <int RL>
+__device__ __forceinline__ void fp_add(float4 (&acc)[RL], const float4 *pa, const float4 *pb, const FpPos &q) {
+    const float4 *qa = reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(pa) + q.o1);
+    const float4 *qb = reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(pb) + q.o2);
+    float4 a[RL + 1], d[RL + 1];
+#pragma unroll
+    for (int j = 0; j <= RL; j++) a[j] = qa[j], d[j] = qb[j];
+#pragma unroll
+    for (int j = 0; j < RL; j++)
+        acc[j] = add4(acc[j], add4(mul4(add4(d[j + 1], a[j]), q.f2), mul4(add4(a[j + 1], d[j]), q.f1)));
+}
+
+// What a plane's bins need at the write-out, RL consecutive planes of one segment: the inputs of the
+// bins of the four lanes (v, x), (v, N-x), (v+90, x), (v+90, N-x).
+template <int MODE, int RL>
+struct FpBins {
+    float a[4][RL];
+    int16_t pr[4][RL];
+    uint16_t wn[4][RL];
+};
+
+template <int MODE, int RL>
+__device__ __forceinline__ void fp_bins_load(const DevGeom &g, int pidx, int cnt, int x, int view, const FpIO &io,
+                                             FpBins<MODE, RL> &b) {
+    if (MODE == FP_PLAIN) return;
 #pragma unroll
     for (int l = 0; l < 4; l++) {
-        if ((l & 1) && x == g.c) continue;   // at x == N/2 lanes 1/3 duplicate lanes 0/2
-        const int col = (l & 1) ? N - x : x, h = l >> 1;
-        float v = lane(acc, l);
-        if (MODE == FP_RATIO_W012) {   // pt_update_est_w012 S3:2436-2447
-            const size_t gi = ((size_t)(view * 2 + h) * N + col) * g.spp + pidx;
-            const float dt = static_cast<const float *>(io.add)[gi];
-            const float q = v > g.eps3 ? dt / v : 0.0f;
-            v = q * resc;
-        } else if (MODE != FP_PLAIN) {
-            const size_t gi = ((size_t)(view * 2 + h) * N + col) * g.spp + pidx;
-            const float a = MODE == FP_RATIO ? static_cast<const float *>(io.add)[gi]
-                                             : half_at(static_cast<const uint16_t *>(io.add), gi);
-            const float den = v + a;
-            const int16_t pr = io.prompt[gi];
-            float q;
-            if (pr == 0) q = 0.0f;
-            else if (den > g.eps3) q = (float)pr / den;
-            else q = 1.0f;
-            if (MODE == FP_RATIO16 && io.ll_part) {
-                // Poisson log-likelihood of the bin (without log y!) at the mean (est + add) / (N*A)
-                const float w = half_at(io.invnorm, gi);
-                if (w > 0.0f && den > g.eps3) {
-                    const double mu = (double)den * (double)w;
-                    ll += (pr > 0 ? (double)pr * log(mu) : 0.0) - mu;
-                }
-            }
-            v = q * resc;
+        const int col = ((l & 1) && x != g.c) ? g.N - x : x, h = l >> 1;
+        const size_t gi = ((size_t)(view * 2 + h) * g.N + col) * g.spp + pidx;
+#pragma unroll
+        for (int j = 0; j < RL; j++) {
+            const int jj = j < cnt ? j : 0;
+            if (MODE == FP_RATIO16) b.a[l][j] = half_at(static_cast<const uint16_t *>(io.add), gi + jj);
+            else b.a[l][j] = static_cast<const float *>(io.add)[gi + jj];
+            if (MODE != FP_RATIO_W012) b.pr[l][j] = io.prompt[gi + jj];
+            if (MODE == FP_RATIO16 && io.ll_part) b.wn[l][j] = io.invnorm[gi + jj];
         }
-        out[((size_t)(lp * 2 + h) * N + col) * g.spp + pidx] = v;
     }
 }
 
-// FAST (HRRT's 207 planes, positions checked non-negative on the host): the staged
-// column length is a compile-time constant, so every LDS read of a row takes its buffer
-// and neighbour as immediate offsets, and the axial fraction is one v_fract.
-constexpr int FP_PL_FAST = 216;
+// Write-out of RL planes of one segment for the four lanes (PJ:1397-1436), optionally through the OP
+// ratio (S3:2493-2505) and the back-projection rescale (PJ:1638-1649).
+template <int MODE, int RL>
+__device__ __forceinline__ void fp_bins_write(const DevGeom &g, const float4 (&acc)[RL], float sc, float resc, int pidx,
+                                              int cnt, int x, int lp, float *__restrict__ out, const FpIO &io,
+                                              const FpBins<MODE, RL> &b, double &ll) {
+#pragma unroll
+    for (int l = 0; l < 4; l++) {
+        if ((l & 1) && x == g.c) continue;   // at x == N/2 lanes 1/3 duplicate lanes 0/2
+        const int col = (l & 1) ? g.N - x : x, h = l >> 1;
+        float r[RL];
+#pragma unroll
+        for (int j = 0; j < RL; j++) {
+            float v = lane(acc[j], l) * sc;
+            if (MODE == FP_RATIO_W012) {   // pt_update_est_w012 S3:2436-2447
+                const float q = v > g.eps3 ? b.a[l][j] / v : 0.0f;
+                v = q * resc;
+            } else if (MODE != FP_PLAIN) {
+                const float den = v + b.a[l][j];
+                const int16_t pr = b.pr[l][j];
+                float q;
+                if (pr == 0) q = 0.0f;
+                else if (den > g.eps3) q = (float)pr / den;
+                else q = 1.0f;
+                if (MODE == FP_RATIO16 && io.ll_part && j < cnt) {
+                    // Poisson log-likelihood of the bin (without log y!) at the mean (est + add) / (N*A)
+                    const float w = __half2float(__ushort_as_half(b.wn[l][j]));
+                    if (w > 0.0f && den > g.eps3) {
+                        const double mu = (double)den * (double)w;
+                        ll += (pr > 0 ? (double)pr * log(mu) : 0.0) - mu;
+                    }
+                }
+                v = q * resc;
+            }
+            r[j] = v;
+        }
+        float *o = out + ((size_t)(lp * 2 + h) * g.N + col) * g.spp + pidx;
+        if (RL == 3 && cnt == 3) {
+            typedef float f3 __attribute__((ext_vector_type(3), aligned(4)));
+            f3 v3;
+            v3.x = r[0], v3.y = r[RL > 1 ? 1 : 0], v3.z = r[RL > 2 ? 2 : 0];
+            *reinterpret_cast<f3 *>(o) = v3;
+        } else {
+#pragma unroll
+            for (int j = 0; j < RL; j++)
+                if (j < cnt) o[j] = r[j];
+        }
+    }
+}
 
-template <int MAXT, int ITEMS, int MODE, bool FAST>
-__global__ void __launch_bounds__(1024) fp_kernel(const DevGeom g, const PairBatch b,
-                                                   const float4 *__restrict__ image, float *__restrict__ out,
-                                                   FpIO io, int nsplit) {
-    extern __shared__ float4 lds[];
-    const int PL = FAST ? FP_PL_FAST : g.Z4 + 8;   // staged planes per column (zero beyond z_pixels)
+// FAST: no row is skipped and no axial position is negative (checked on the host), so the axial
+// fraction is one v_fract and the planes need no row test.
+template <int RL, int R, int MODE, bool FAST>
+__global__ void __launch_bounds__(1024) fp_kernel(const DevGeom g, const PairBatch b, const float4 *__restrict__ image,
+                                                  float *__restrict__ out, FpIO io, int nsplit) {
+    __shared__ float4 lds[(1 + 4 * R) * FP_PL];
     float4 *rimc = lds;
-    float4 *stage = lds + PL;  // [2][2][PL]
-    // longest rays first (x = N/2 has the most y steps), then plane share, then view pair
-    const int per_pair = g.c * nsplit;
-    // each XCD: consecutive rays of one pair of one frame
-    const int L0 = xcd_contiguous(blockIdx.x, per_pair * b.npairs * b.nframes);
-    const int frame = L0 / (per_pair * b.npairs), L = L0 - frame * per_pair * b.npairs;
+    float4 *stage = lds + FP_PL;  // [2][R][2][FP_PL]
+    int frame, lp, ray, split;
+    if (!fp_block(g, b, nsplit, blockIdx.x, frame, lp, ray, split)) return;
+    const int L0 = ((frame * b.npairs + lp) * g.c + ray) * nsplit + split;
     image += frame * b.img_stride / 4;
     out += frame * b.ratio_stride;
     if (MODE == FP_RATIO || MODE == FP_RATIO16) io.prompt += frame * b.sino_stride;
     if (MODE == FP_RATIO || MODE == FP_RATIO_W012) io.add = static_cast<const float *>(io.add) + frame * b.sino_stride;
     else if (MODE == FP_RATIO16) io.add = static_cast<const uint16_t *>(io.add) + frame * b.sino_stride;
     double ll = 0.0;
-    const int lp = L / per_pair, rem = L - lp * per_pair;
-    const int x = g.c - rem / nsplit, split = rem % nsplit;
-    const int p_lo = (int)(((long long)g.fp_np * split) / nsplit);
-    const int p_hi = (int)(((long long)g.fp_np * (split + 1)) / nsplit);
+    const int x = g.c - ray;
     const int view = b.view0 + b.view_stride * lp;
     const int N = g.N, c = g.c;
     if (g.cyl_lo[x] == g.cyl_hi[x] || g.nzmask[view * (c + 1) + x] == 0) {
@@ -346,105 +350,136 @@ __global__ void __launch_bounds__(1024) fp_kernel(const DevGeom g, const PairBat
         return;
     }
     const float cosv = g.cos_psi[view], sinv = g.sin_psi[view];
-
-    for (int i = threadIdx.x; i < 5 * PL; i += blockDim.x) lds[i] = f4(0.f);
-    __syncthreads();
-    // centre row samples (x,c),(N-x,c),(c,x),(c,N-x) PJ:1815-1829
-    for (int it = threadIdx.x; it < 4 * g.NQ; it += blockDim.x) {
-        int i = it / g.NQ, q = it - i * g.NQ;
-        int xx = i == 0 ? x : (i == 1 ? N - x : c);
-        int yy = i < 2 ? c : (i == 2 ? x : N - x);
-        float4 v;
-        if (!sample_chunk(g, image, cosv, sinv, xx, yy, q, v)) v = f4(0.f);
-        put_lanes(rimc, q, i, v, g.Z);
-    }
     const int ystart = g.cyl_lo[x];
-    if (ystart < c) sample8(g, image, cosv, sinv, x, ystart, stage, stage + PL);
-    __syncthreads();
 
-    float4 acc1[MAXT], acc2[MAXT];
-    int code[MAXT], ymin[MAXT], dbyte[MAXT];
-    float pbase[MAXT], ptan[MAXT];
-#pragma unroll
-    for (int t = 0; t < MAXT; t++) {
-        const int p = p_lo + threadIdx.x + t * blockDim.x;
-        code[t] = -1; ymin[t] = c; pbase[t] = 0.f; ptan[t] = 0.f; dbyte[t] = 0;
-        int yr = 0;
-        if (p < p_hi) {
-            const int4 e = g.fp_planes[p];
-            code[t] = e.x; pbase[t] = __int_as_float(e.y); ptan[t] = __int_as_float(e.z); ymin[t] = e.w;
-            yr = (e.x >> 8) & 0xff;
-            dbyte[t] = (e.x >> 16) * (int)sizeof(float4);   // the plane shift delta, in LDS bytes
-        }
-        const float4 v = rimc[yr];   // centre row sample at plane yr (PJ:1830-1838)
-        acc1[t] = v;
-        acc2[t] = v;
+    // This thread's run {k | first plane << 8 | planes << 16, bits(base), bits(tan), delta | ymin << 16}
+    // and single (the same with one plane; k = 0: axial).  Singles go to the waves behind the runs, then
+    // over again from the first wave.
+    int4 er = make_int4(0, 0, 0, 0), es = er;
+    {
+        const int r_lo = (int)((long long)g.fp_nr[RL == 3] * split / nsplit), r_hi = (int)((long long)g.fp_nr[RL == 3] * (split + 1) / nsplit);
+        const int s_lo = (int)((long long)g.fp_ns * split / nsplit), s_hi = (int)((long long)g.fp_ns * (split + 1) / nsplit);
+        const int nr = r_hi - r_lo, ns = s_hi - s_lo, tid = threadIdx.x;
+        int ts = tid - ((nr + 63) & ~63);
+        if (ts < 0) ts += blockDim.x;
+        if (tid < nr) er = g.fp_runs[RL == 3][r_lo + tid];
+        if (ts < ns) es = g.fp_single[s_lo + ts];
     }
 
-    // project the staged row y (halves pa, pb) into every plane this thread owns
-    auto project = [&](const float4 *pa, const float4 *pb, int y) {
-        const float fy2 = (float)(c - y);   // (y - c) * tan = -((c - y) * tan) exactly
+    // The centre row's samples (x,c),(N-x,c),(c,x),(c,N-x) (PJ:1815-1829) and the first rows.  A wave
+    // samples one item of a step: wave w the (w mod n)-th of the n of row w / n.
+    Sample s0, nxt;
+    const int per_row = 128 * ((g.NQ + 15) >> 4);
+    const int srow = __builtin_amdgcn_readfirstlane((int)threadIdx.x / per_row);
+    SampleLane sl = sample_lane(g, (int)threadIdx.x - srow * per_row, x);
+    if (srow >= R) sl.q = g.NQ, sl.slot = -1;
+    const bool wave_samples = __any(sl.slot >= 0);
+    const int cq = 16 * (threadIdx.x >> 6) + (threadIdx.x & 15), ci = (threadIdx.x & 63) >> 4;
+    {
+        const int xx = ci == 0 ? x : (ci == 1 ? N - x : c), yy = ci < 2 ? c : (ci == 2 ? x : N - x);
+        sample_load(g, image, cosv, sinv, (float)(xx - c), (float)(yy - c), cq, s0);
+    }
+    // loads of rows y .. y + R - 1 (rows from c on are not staged), and their combination into LDS
+    auto load_rows = [&](int y) __attribute__((always_inline)) {
+        nxt.ok = false;
+        if (y + srow >= c) return;
+        const float fy = (float)(y + srow - c);
+        sample_load(g, image, cosv, sinv, __builtin_fmaf(sl.sx, fy, sl.kx), __builtin_fmaf(sl.sy, fy, sl.ky), sl.q, nxt);
+    };
+    auto store_rows = [&](float4 *buf) __attribute__((always_inline)) {
+        if (!wave_samples) return;
+        const float4 v = sample_combine(nxt);
+        if (sl.slot >= 0) buf[srow * 2 * FP_PL + sl.slot] = v;
+    };
+    load_rows(ystart);
+    for (int i = threadIdx.x; i < 4 * R * FP_PL; i += blockDim.x) stage[i] = f4(0.f);   // the planes behind the image stay zero
+    __syncthreads();
+    {
+        const float4 v = sample_combine(s0);
+        if (cq < g.NQ) rimc[4 * cq + ci] = v;
+    }
+    store_rows(stage);
+    load_rows(ystart + R);
+    __syncthreads();
+
+    const bool run = er.x != 0, single = (es.x & 0xff) != 0, axial = !single && (es.x >> 16) != 0;
+    const int ryr = (er.x >> 8) & 0xff, syr = (es.x >> 8) & 0xff;
+    const float rbase = __int_as_float(er.y), rtan = __int_as_float(er.z);
+    const float sbase = __int_as_float(es.y), stan = __int_as_float(es.z);
+    const int rbyte = (er.w & 0xffff) * (int)sizeof(float4);                      // plane shift, in LDS bytes
+    const int sbyte = (axial ? syr : es.w & 0xffff) * (int)sizeof(float4);        // (an axial plane: its row)
+    const int rmin = FAST ? 0 : er.w >> 16, smin = FAST ? 0 : es.w >> 16;
+    // centre row samples (PJ:1830-1838)
+    float4 r1[RL], r2[RL], s1[1], s2[1];
 #pragma unroll
-        for (int t = 0; t < MAXT; t++) {
-            if (code[t] < 0) continue;
-            const int k = code[t] & 0xff;
-            if (k == 0) {   // theta = 0 PJ:1907-1910
-                const int yr = (code[t] >> 8) & 0xff;
-                acc1[t] = add4(acc1[t], add4(pa[yr], pb[yr]));
-                continue;
-            }
-            if (y < ymin[t]) continue;   // PJ:1920-1921
-            const float pt = fy2 * ptan[t];
-            const float zz1 = pbase[t] - pt, zz2 = pbase[t] + pt;
-            const int i1 = (int)zz1, i2 = (int)zz2;
-            float f1, f2;
-            if (FAST) {        // zz >= 0: zz - trunc(zz) = zz - floor(zz)
-                f1 = __builtin_amdgcn_fractf(zz1);
-                f2 = __builtin_amdgcn_fractf(zz2);
-            } else {
-                f1 = zz1 - i1;
-                f2 = zz2 - i2;
-            }
-            // planes z = i1 + delta and z2 = i2 + delta: the shift folded into the base address
-            const float4 *qa = reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(pa) + dbyte[t]);
-            const float4 *qb = reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(pb) + dbyte[t]);
-            const float4 a0 = qa[i1], a1 = qa[i1 + 1], b0 = qb[i1], b1 = qb[i1 + 1];
-            const float4 d0 = qb[i2], d1 = qb[i2 + 1], e0 = qa[i2], e1 = qa[i2 + 1];
-            // PJ:1934-1944: (pam2[z2+1] + pam[z])*f2 + (pam[z+1] + pam2[z2])*f1 and its mirror
-            acc1[t] = add4(acc1[t], add4(mul4(add4(d1, a0), f2), mul4(add4(a1, d0), f1)));
-            acc2[t] = add4(acc2[t], add4(mul4(add4(e1, b0), f2), mul4(add4(b1, e0), f1)));
+    for (int j = 0; j < RL; j++) r1[j] = r2[j] = rimc[ryr + j];
+    s1[0] = s2[0] = rimc[syr];
+
+    // project the staged row y (halves pa, pb) into this thread's planes
+    auto project = [&](const float4 *pa, const float4 *pb, int y) __attribute__((always_inline)) {
+        const float fy2 = (float)(c - y);   // (y - c) * tan = -((c - y) * tan) exactly
+        if (run && (FAST || y >= rmin)) {   // PJ:1920-1921
+            const FpPos q = fp_pos<FAST>(rbase, rtan, fy2, rbyte);
+            fp_add<RL>(r1, pa, pb, q);
+            fp_add<RL>(r2, pb, pa, q);
+        }
+        if (single && (FAST || y >= smin)) {
+            const FpPos q = fp_pos<FAST>(sbase, stan, fy2, sbyte);
+            fp_add<1>(s1, pa, pb, q);
+            fp_add<1>(s2, pb, pa, q);
+        }
+        if (axial) {   // theta = 0 PJ:1907-1910
+            const float4 *qa = reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(pa) + sbyte);
+            const float4 *qb = reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(pb) + sbyte);
+            s1[0] = add4(s1[0], add4(qa[0], qb[0]));
         }
     };
-    // one row per barrier: project row y (buffer ST) while the next row's samples load
-    auto row = [&](auto stc, int y) {
+    // R rows per barrier: the samples of the next R rows, loaded during the step before, go into the
+    // other buffer, the loads of the R rows behind them are issued, then this step's rows are projected
+    auto step = [&](auto stc, int y) __attribute__((always_inline)) {
         constexpr int st = decltype(stc)::value;
-        SampleRegs<ITEMS> nxt;
-        if (y + 1 < c) {
-            if (FAST) sample8x_load<ITEMS>(g, image, cosv, sinv, x, y + 1, nxt);
-            else sample8_load<ITEMS>(g, image, cosv, sinv, x, y + 1, nxt);
+        if (y + R < c) {
+            store_rows(stage + (st ^ 1) * 2 * R * FP_PL);
+            load_rows(y + 2 * R);
         }
-        const float4 *pa = stage + st * 2 * PL;
-        project(pa, pa + PL, y);
-        if (y + 1 < c) {
-            float4 *na = stage + (st ^ 1) * 2 * PL;
-            if (FAST) sample8x_store<ITEMS>(g, nxt, na, na + PL);
-            else sample8_store<ITEMS>(g, nxt, na, na + PL);
-        }
+        unroll<R>([&](auto rc) __attribute__((always_inline)) {
+            constexpr int r = decltype(rc)::value;
+            const float4 *pa = stage + (st * R + r) * 2 * FP_PL;
+            if (r == 0 || y + r < c) project(pa, pa + FP_PL, y + r);
+        });
         __syncthreads();
     };
-    for (int y = ystart; y < c; y += 2) {   // row ystart + 2j reads buffer 0, the next one buffer 1
-        row(std::integral_constant<int, 0>{}, y);
-        if (y + 1 < c) row(std::integral_constant<int, 1>{}, y + 1);
+    for (int y = ystart; y < c; y += 2 * R) {   // steps alternate between the two buffers
+        step(std::integral_constant<int, 0>{}, y);
+        if (y + R < c) step(std::integral_constant<int, 1>{}, y + R);
     }
 
-    // scaling PJ:1953-1975 and write-out
-#pragma unroll
-    for (int t = 0; t < MAXT; t++) {
-        if (code[t] < 0) continue;
-        const int k = code[t] & 0xff, yr = (code[t] >> 8) & 0xff;
-        const float sc = k == 0 ? g.y_size : g.rescalearray[(k - 1) * g.Z + yr];
-        fp_write1<MODE>(g, mul4(acc1[t], sc), k == 0 ? 0 : 2 * k, yr, x, view, lp, out, io, ll);
-        if (k != 0) fp_write1<MODE>(g, mul4(acc2[t], sc), 2 * k - 1, yr, x, view, lp, out, io, ll);
+    // scaling PJ:1953-1975 and write-out; every plane of a run has the run's scale, and the planes of a
+    // segment are consecutive
+    if (run) {
+        const int k = er.x & 0xff, cnt = er.x >> 16;
+        const float sc = g.rescalearray[(k - 1) * g.Z + ryr];
+        const int p1 = g.seg_data[2 * k] + (ryr - g.yb[2 * k]), p2 = g.seg_data[2 * k - 1] + (ryr - g.yb[2 * k - 1]);
+        const float c1 = g.bp_rescale[2 * k], c2 = g.bp_rescale[2 * k - 1];
+        FpBins<MODE, RL> b1, b2;
+        fp_bins_load(g, p1, cnt, x, view, io, b1);
+        if (MODE != FP_RATIO16) fp_bins_load(g, p2, cnt, x, view, io, b2);
+        fp_bins_write(g, r1, sc, c1, p1, cnt, x, lp, out, io, b1, ll);
+        if (MODE == FP_RATIO16) fp_bins_load(g, p2, cnt, x, view, io, b2);   // the registers of its sums hold one set
+        fp_bins_write(g, r2, sc, c2, p2, cnt, x, lp, out, io, b2, ll);
+    }
+    if (single || axial) {
+        const int k = es.x & 0xff, seg = 2 * k;
+        const float sc = k == 0 ? g.y_size : g.rescalearray[(k - 1) * g.Z + syr];
+        const int p1 = g.seg_data[seg] + (syr - g.yb[seg]);
+        FpBins<MODE, 1> b1;
+        fp_bins_load(g, p1, 1, x, view, io, b1);
+        fp_bins_write(g, s1, sc, g.bp_rescale[seg], p1, 1, x, lp, out, io, b1, ll);
+        if (single) {
+            const int p2 = g.seg_data[seg - 1] + (syr - g.yb[seg - 1]);
+            fp_bins_load(g, p2, 1, x, view, io, b1);
+            fp_bins_write(g, s2, sc, g.bp_rescale[seg - 1], p2, 1, x, lp, out, io, b1, ll);
+        }
     }
     if (MODE == FP_RATIO16 && io.ll_part) {
         // workgroup sum of the log-likelihood in a fixed order (waves, then lanes)
@@ -1511,62 +1546,62 @@ __global__ void __launch_bounds__(256) moments_reduce_kernel(const double *__res
 // ---------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------
-template <int MAXT, int ITEMS, bool FAST>
-static hipError_t fp_launch_t(const DevGeom &g, const PairBatch &b, const float *image, float *out, const FpIO &io,
-                              int mode, int nsplit, int threads, hipStream_t s) {
-    dim3 grid(g.c * nsplit * b.npairs * b.nframes), block(threads);
-    size_t shm = sizeof(float4) * 5 * (FAST ? FP_PL_FAST : g.Z4 + 8);
-    const float4 *im = reinterpret_cast<const float4 *>(image);
-    if (mode == FP_RATIO)
-        hipLaunchKernelGGL((fp_kernel<MAXT, ITEMS, FP_RATIO, FAST>), grid, block, shm, s, g, b, im, out, io, nsplit);
-    else if (mode == FP_RATIO_W012)
-        hipLaunchKernelGGL((fp_kernel<MAXT, ITEMS, FP_RATIO_W012, FAST>), grid, block, shm, s, g, b, im, out, io, nsplit);
-    else if (mode == FP_RATIO16)
-        hipLaunchKernelGGL((fp_kernel<MAXT, ITEMS, FP_RATIO16, FAST>), grid, block, shm, s, g, b, im, out, io, nsplit);
-    else
-        hipLaunchKernelGGL((fp_kernel<MAXT, ITEMS, FP_PLAIN, FAST>), grid, block, shm, s, g, b, im, out, io, nsplit);
-    return hipGetLastError();
+// Launch shape: runs of `run` middle planes per thread (1 or 3); the planes of one ray column are
+// split over nsplit workgroups of 4 to 16 waves (a multiple of 4, one per SIMD each, and enough for
+// a row's sampling).  The caller's shape (fp_maxt, fp_nsplit) is kept where it is given; otherwise:
+// * Two rays or more per CU: runs of 3, and no more waves than the runs or the singles need, so that
+//   two workgroups share a CU where the planes allow it (span 9, 8 frames of 128 x 128: 0.277 ms with
+//   8 waves, 0.40 with 12; runs of 1 0.32), unless 4 waves hold the planes one by one (3 frames of a
+//   30-ring scanner at 132 x 132: 0.424 ms a subset against 0.466).
+// * Fewer rays: a CU holds one workgroup, and what counts is the time of a row: 16 waves, and one plane
+//   per thread if that holds them (one span-9 subset at 128 x 128: 51 us, 66 with runs of 3 in 12 waves; a
+//   16-ring subset: 30 against 44); below one ray per two CUs the planes are split once
+//   (one view pair at span 3: 0.344 ms against 0.390).
+void forward_shape(const DevGeom &g, int npf, int &run, int &nsplit, int &threads) {
+    constexpr int CUS = 256;
+    const long long rays = (long long)g.c * npf;
+    const bool few = rays < 2 * CUS;
+    nsplit = g.fp_nsplit;
+    if (nsplit < 1) nsplit = 2 * rays <= CUS ? 2 : 1;
+    auto waves_of = [&](int n) { return ((n + nsplit - 1) / nsplit + 63) / 64; };
+    const int least = g.NQ > 32 ? 8 : 4;   // waves that sample a row
+    if (g.fp_maxt > 0) run = g.fp_maxt < 3 ? 1 : 3;
+    else run = waves_of(g.fp_nr[0]) <= (few ? 16 : 4) ? 1 : 3;
+    const int nr = g.fp_nr[run == 3], need = (std::max(nr, g.fp_ns) + 1023) / 1024;
+    if (nsplit < need) nsplit = need;
+    const int waves = std::max(waves_of(nr), waves_of(g.fp_ns));
+    threads = few ? 1024 : 64 * std::min(std::max((waves + 3) / 4 * 4, least), 16);
 }
 
-// Launch shape: MAXT planes per thread; the planes of one ray column are split over
-// nsplit workgroups; each workgroup has enough 64-lane waves (a multiple of 4, at most
-// 16) for its share of the planes and for the sampling of a row.
-void forward_shape(const DevGeom &g, int &maxt, int &nsplit, int &threads, int &items) {
-    maxt = g.fp_maxt;
-    nsplit = g.fp_nsplit;
-    if (maxt < 1 || maxt > 4) maxt = 1;
-    const int need = (g.fp_np + 1024 * maxt - 1) / (1024 * maxt);
-    if (nsplit < need) nsplit = need;
-    const int per = (g.fp_np + nsplit - 1) / nsplit;
-    // waves in multiples of 4, one per SIMD each: with one workgroup per CU and a barrier per
-    // row, a SIMD holding one wave more than the others would set the pace of every row
-    int waves = ((per + maxt - 1) / maxt + 63) / 64;
-    waves = (waves + 3) / 4 * 4;
-    if (waves > 16) waves = 16;
-    threads = 64 * waves;
-    if ((8 * g.NQ + threads - 1) / threads > 2) threads = ((8 * g.NQ + 1) / 2 + 63) / 64 * 64;
-    items = (8 * g.NQ + threads - 1) / threads;
+template <int MODE>
+static hipError_t fp_launch(const DevGeom &g, const PairBatch &b, const float *image, float *out, const FpIO &io,
+                            hipStream_t s) {
+    int run, nsplit, threads;
+    const int npf = b.npairs * b.nframes;
+    forward_shape(g, npf, run, nsplit, threads);
+    const long long blocks = fp_blocks(g.c, npf, nsplit);
+    if (blocks > 0x7fffffffLL) return hipErrorInvalidConfiguration;
+    const float4 *im = reinterpret_cast<const float4 *>(image);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(threads), 0, s, g, b, im, out, io, nsplit);
+        return hipGetLastError();
+    };
+    auto pick = [&](auto fast) {
+        constexpr bool F = decltype(fast)::value;
+        if (run == 3) return threads == 1024 ? go(fp_kernel<3, 2, MODE, F>) : go(fp_kernel<3, 1, MODE, F>);
+        return threads == 1024 ? go(fp_kernel<1, 2, MODE, F>) : go(fp_kernel<1, 1, MODE, F>);
+    };
+    return g.fp_fast ? pick(std::true_type{}) : pick(std::false_type{});
 }
 
 hipError_t launch_forward(const DevGeom &g, const PairBatch &b, const float *image, float *out, const FpIO &io,
                           int mode, hipStream_t s) {
-    int maxt, nsplit, threads, it2;
-    forward_shape(g, maxt, nsplit, threads, it2);
-#define FP_CASE(M)                                                                                    \
-    case M:                                                                                           \
-        return it2 <= 1 ? fp_launch_t<M, 1, false>(g, b, image, out, io, mode, nsplit, threads, s)    \
-                        : fp_launch_t<M, 2, false>(g, b, image, out, io, mode, nsplit, threads, s);
-    // the FAST path stages a row as 2 x ceil(NQ/16) whole waves of samples, one item each
-    if (maxt == 4 && g.fp_fast && g.Z4 + 8 == FP_PL_FAST && 128 * ((g.NQ + 15) / 16) <= threads)
-        return fp_launch_t<4, 1, true>(g, b, image, out, io, mode, nsplit, threads, s);
-    switch (maxt) {
-        FP_CASE(1)
-        FP_CASE(2)
-        FP_CASE(3)
-        default:
-            FP_CASE(4)
+    switch (mode) {
+        case FP_RATIO: return fp_launch<FP_RATIO>(g, b, image, out, io, s);
+        case FP_RATIO16: return fp_launch<FP_RATIO16>(g, b, image, out, io, s);
+        case FP_RATIO_W012: return fp_launch<FP_RATIO_W012>(g, b, image, out, io, s);
+        default: return fp_launch<FP_PLAIN>(g, b, image, out, io, s);
     }
-#undef FP_CASE
 }
 
 hipError_t launch_backproject(const DevGeom &g, const PairBatch &b, const void *src, int src_half, int src_global,
