@@ -504,75 +504,78 @@ extern "C" int hrrt_create(const hrrt_params *params, hrrt_ctx **out) {
             }
         }
 
-    // incremental back projector (back_proj3d_view_n1thread PJ:4162-4668).  LDS holds one lane's
-    // column: segment 0 (Z floats, padded to an even count), then per group k a window of
-    // float2 {segment 2k, segment 2k-1} for rows yr = yb-3 .. yt+1, where yb-1 and yt+1 are the
-    // reference's zero guard planes (PJ:1689-1692) and yb-3, yb-2 two more zero cells.  The
-    // window is turned in place into the reference's differences P'(yr) = (p(yr+1)-p(yr))*tan
-    // (PJ:4313-4324), then into the values the breakpoint terms read: M(yr) = P'(yr)-P'(yr+1)
+    // incremental back projector (back_proj3d_view_n1thread PJ:4162-4668).  LDS holds the columns of
+    // the bins x and N-x of one view: segment 0 (Z float2, padded to whole cells), then per group k a window
+    // of 16-byte cells {segment 2k, 2k-1 of bin x, 2k, 2k-1 of bin N-x} for rows yr = yb-3 .. yt+1, where yb-1
+    // and yt+1 are the reference's zero guard planes (PJ:1689-1692) and yb-3, yb-2 two more zero cells.  The
+    // window is turned in place into the values the breakpoint terms read, from the reference's differences
+    // P'(yr) = (p(yr+1)-p(yr))*tan (PJ:4313-4324): M(yr) = P'(yr)-P'(yr+1)
     // for yr in [yb-1, yt-1] (the middle terms PJ:4381-4394), M(yb-2) = -P'(yb-1) (the two
     // terms before the loop, PJ:4369-4380) and M(yt) = P'(yt) (the two after it, PJ:4395-4406),
     // with zeros at yb-3 and yt+1: a breakpoint then adds, to plane z, the terms read at rows
     // z + const clamped into the window, a clamped read giving exactly +0.
     int inc_ok = Z <= 256 && N <= 256 && G.K <= 32;
-    std::vector<int> isrc;
-    std::vector<int2> iconv;
+    std::vector<int4> ichunk;
+    std::vector<int2> icell;
+    std::vector<int> izero;
     std::vector<int> gbase(G.K + 1, 0);
-    for (int z = 0; z < Z; z++) {
-        isrc.push_back(G.seg_data[0] + z);
-        iconv.push_back(make_int2(0, 0));
-    }
-    if (Z & 1) {
-        isrc.push_back(-1);
-        iconv.push_back(make_int2(0, 0));
-    }
+    std::vector<float> gtan(G.K + 1, 0.f);
+    int ncells = (Z + 1) / 2;                                       // cells so far: segment 0
     for (int k = 1; k <= G.K; k++) {
         const int th = 2 * k, yb = G.yr_bottom[th], yt = G.yr_top[th];
         if (yb != G.yr_bottom[th - 1] || yt != G.yr_top[th - 1] || yt < yb) inc_ok = 0;
-        const float tn = -G.sin_theta[th] / G.cos_theta[th];
-        gbase[k] = (int)isrc.size() / 2 - (yb - 3);                  // float2 index of row 0
-        for (int yr = yb - 3; yr <= yt + 1; yr++)
-            for (int e = 0; e < 2; e++) {
-                const int sg = e == 0 ? th : th - 1;
-                isrc.push_back(yr >= yb && yr <= yt ? G.seg_data[sg] + (yr - yb) : -1);
-                const int second = yr == yb - 2 ? 2 : (yr >= yb - 1 && yr <= yt - 1 ? 1 : 0);
-                iconv.push_back(make_int2(yr >= yb - 1 && yr <= yt ? bits(tn) : 0, second));
-            }
+        gtan[k] = -G.sin_theta[th] / G.cos_theta[th];
+        gbase[k] = ncells - (yb - 3);                                // cell of row 0
+        ncells += yt - yb + 5;
+        for (int i = 0; i <= yt - yb; i += 4)
+            ichunk.push_back(make_int4(G.seg_data[th] + i, G.seg_data[th - 1] + i, gbase[k] + yb + i,
+                                       std::min(4, yt - yb + 1 - i) | (k << 8)));
+        for (int yr : {yb - 3, yb - 2, yb - 1, yt + 1}) izero.push_back(gbase[k] + yr);
+        for (int yr = yb - 2; yr <= yt; yr++)
+            icell.push_back(make_int2((gbase[k] + yr) | ((yr == yb - 2 ? 1 : (yr == yt ? 2 : 0)) << 16), bits(gtan[k])));
     }
-    const int inc_lds = (int)isrc.size();
+    izero.push_back(ncells);                                         // read above the last window, never used
+    if (ncells + 1 > 0xffff) inc_ok = 0;
     auto in_window = [&](int k, int first, int count) {      // rows first .. first+count of group k
         if (count < 0) return true;
         return first >= G.yr_bottom[2 * k] - 1 && first + count <= G.yr_top[2 * k] + 1;
     };
-    // per group k (entry k-1): {float2 index of row 0 of the window, yb, yt, 0}, row c-1 lookup
-    // {zsa, count, yra, bits(frac)}, row c+1 lookup {zsa, yra, bits(frac), 0}, row c+1 breakpoint
-    // {z_start, z_end, yr_start, 0}; a range with no planes points at yb so that its (unused)
-    // reads stay in the window
-    std::vector<int4> igroup((size_t)std::max(G.K, 1) * 4, make_int4(0, 0, 0, 0));
+    // per group k (entry k-1): {cell of row 0 of the window, yb, yt, bits(tan)}, the lookups of rows c-1 and
+    // c+1 {yra - zsa, bits(frac), the same of row c+1}, row c+1 breakpoint {z_start, z_end, yr_start, row c-1
+    // first}; a breakpoint with no planes points at yb so that its (unused) reads stay in the window.  The
+    // planes of a lookup are those whose rows lie in [yb-1, yt] (its ranges are built so, PJ:670-700; checked), so
+    // reads clamped to [yb-2, yt+1] interpolate zeros outside
+    std::vector<int4> igroup((size_t)std::max(G.K, 1) * 3, make_int4(0, 0, 0, 0));
     for (int k = 1; k <= G.K; k++) {
         const int th = 2 * k, yb = G.yr_bottom[th], yt = G.yr_top[th];
         const size_t l1 = (size_t)(c - 1) * GM + k - 1, l2 = (size_t)(c + 1) * GM + k - 1;
         const hrrt::Geometry::Blut &bc = G.blut[l2];
-        const int n = G.bl_zea[l1] - G.bl_zsa[l1] + 1;
-        int yra1 = G.bl_yra[l1], yra2 = G.bl_yra[l2], bcyr = bc.yr_start;
-        if (n <= 0) yra1 = yra2 = yb;
+        int bcyr = bc.yr_start;
         if (bc.z_end < bc.z_start) bcyr = yb;
-        if (n > 0 && (!in_window(k, yra1, n) || !in_window(k, yra2, n))) inc_ok = 0;
         if (!in_window(k, bcyr, std::max(bc.z_end - bc.z_start, 0))) inc_ok = 0;
-        int4 *e = &igroup[(size_t)(k - 1) * 4];
-        e[0] = make_int4(gbase[k], yb, yt, 0);
-        e[1] = make_int4(G.bl_zsa[l1], n, yra1, bits(G.bl_frac[l1]));
-        e[2] = make_int4(G.bl_zsa[l2], yra2, bits(G.bl_frac[l2]), 0);
-        e[3] = make_int4(bc.z_start, bc.z_end, bcyr, 0);
+        int off[2], j = 0;
+        for (size_t l : {l1, l2}) {
+            off[j] = G.bl_yra[l] - G.bl_zsa[l];
+            for (int z = 0; z < Z; z++) {
+                const int row = z + off[j];
+                if ((z >= G.bl_zsa[l] && z <= G.bl_zea[l]) != (row >= yb - 1 && row <= yt)) inc_ok = 0;
+            }
+            j++;
+        }
+        int4 *e = &igroup[(size_t)(k - 1) * 3];
+        e[0] = make_int4(gbase[k], yb, yt, bits(gtan[k]));
+        e[1] = make_int4(off[0], bits(G.bl_frac[l1]), off[1], bits(G.bl_frac[l2]));
+        e[2] = make_int4(bc.z_start, bc.z_end, bcyr, G.bl_zsa[l2] <= G.bl_zsa[l1]);
     }
-    // breakpoints of rows c-2 down to 1, groups ascending: {bits(coef1), byte offsets (from 8z) of
+    // breakpoints of rows c-2 down to 1, groups ascending: {bits(coef1), cell offsets (from z) of
     // the a-term row yr_start_pre + (z - z_start_pre) and of the b-term row yr_start_pre +
-    // (z - z_start_pre(N-y) - 1), window bounds lo | hi << 16 in bytes}.  Handled: the range moved
+    // (z - z_start_pre(N-y) - 1), window bounds lo | hi << 16 in cells}; the offsets are times 16,
+    // their low four bits hold the row y (a: its low half).  Handled: the range moved
     // down by one plane, it spans the segment's rows [yb-1, yt], and the b-term's iteration of a
     // plane is never after its a-term's (z_start_pre(N-y) + 1 > z_start_pre), so every plane takes
     // its b-term first (PJ:4381-4394)
     std::vector<int4> isched;
-    std::vector<int> inrow(c + 1, 0);
+    std::vector<int> icount(c + 1, 0);
     for (int y = c - 2; y >= 1; y--) {
         for (int k = 1; k <= G.K; k++) {
             const size_t li = (size_t)y * GM + k - 1;
@@ -586,17 +589,18 @@ extern "C" int hrrt_create(const hrrt_params *params, hrrt_ctx **out) {
             float tn = -G.sin_theta[th] / G.cos_theta[th];
             tn = 1 - tn * (float)ba.num - ba.coef_pre;                    // PJ:4371-4373
             const float coef1 = -tn * G.cos_theta[th] / G.sin_theta[th];
-            const int offa = 8 * (gbase[k] + ba.yr_start_pre - zp), offb = 8 * (gbase[k] + ba.yr_start_pre - z2p - 1);
-            const int lo8 = 8 * (gbase[k] + yb - 3), hi8 = 8 * (gbase[k] + yt + 1);
-            isched.push_back(make_int4(bits(coef1), offa, offb, lo8 | (hi8 << 16)));
-            inrow[y]++;
+            const int offa = 16 * (gbase[k] + ba.yr_start_pre - zp) + (y & 15);       // 16 x cells, then 4 bits of y
+            const int offb = 16 * (gbase[k] + ba.yr_start_pre - z2p - 1) + (y >> 4);
+            isched.push_back(make_int4(bits(coef1), offa, offb, (gbase[k] + yb - 3) | ((gbase[k] + yt + 1) << 16)));
         }
+        icount[y] = (int)isched.size();
     }
-    isched.push_back(make_int4(0, 0, 0, 0));                           // read ahead of the last one
+    for (int i = 0; i < 128; i++) isched.push_back(make_int4(0, 0, 0, 0));   // read ahead of the last one
     d.inc_ok = inc_ok;
-    d.inc_lds = inc_lds;
-    d.inc_shm = (int)(sizeof(float) * (inc_lds + 2));                // + the two floats the last conversion reads
-    if (d.inc_shm > 64 * 1024) d.inc_ok = 0;
+    d.inc_nchunk = (int)ichunk.size();
+    d.inc_ncell = (int)icell.size();
+    d.inc_shm = (int)sizeof(float4) * (ncells + 1);                      // + the cell read above the last window
+    if (d.inc_shm > 128 * 1024) d.inc_ok = 0;
 
     int r = 0;
     if ((r = ctx->upload(G.cyl_lo, d.cyl_lo)) || (r = ctx->upload(G.cyl_hi, d.cyl_hi)) ||
@@ -608,9 +612,9 @@ extern "C" int hrrt_create(const hrrt_params *params, hrrt_ctx **out) {
         (r = ctx->upload(rot, d.rot)) || (r = ctx->upload(fruns[0], d.fp_runs[0])) ||
         (r = ctx->upload(fruns[1], d.fp_runs[1])) || (r = ctx->upload(fsingle, d.fp_single)) || (r = ctx->upload(pseg, d.pseg)) ||
         (r = ctx->upload(plane_seg, d.plane_seg)) || (r = ctx->upload(bp_src, d.bp_src)) ||
-        (r = ctx->upload(blut2, d.bp_lut2)) || (r = ctx->upload(isrc, d.inc_src)) ||
-        (r = ctx->upload(iconv, d.inc_conv)) || (r = ctx->upload(igroup, d.inc_group)) ||
-        (r = ctx->upload(isched, d.inc_sched)) || (r = ctx->upload(inrow, d.inc_nrow))) {
+        (r = ctx->upload(blut2, d.bp_lut2)) || (r = ctx->upload(ichunk, d.inc_chunk)) ||
+        (r = ctx->upload(izero, d.inc_zero)) || (r = ctx->upload(icell, d.inc_cell)) || (r = ctx->upload(igroup, d.inc_group)) ||
+        (r = ctx->upload(isched, d.inc_sched)) || (r = ctx->upload(icount, d.inc_count))) {
         delete ctx;
         return r;
     }

@@ -38,13 +38,15 @@ struct DevGeom {
     int8_t *nzmask;                      // [views/2][N/2+1], 0 = masked column
     // incremental back projector (back_proj3d_view_n1thread PJ:4162-4668)
     int inc_ok;                          // 1 when every breakpoint of the geometry is of the kind handled
-    int inc_lds;                         // LDS floats of one lane's column (segment 0, then one window per group)
-    int inc_shm;                         // LDS bytes of the incremental back projector's workgroup
-    const int *inc_src;                  // [inc_lds] LDS float -> pair-column plane (-1 = zero)
-    const int2 *inc_conv;                // [inc_lds] {bits(-tan) of the difference step (0 = none), second step}
-    const int4 *inc_group;               // [K][4] per group: window, first-row lookups, row c+1 breakpoint
-    const int4 *inc_sched;               // [n+1] breakpoints of rows c-2 down to 1, groups ascending
-    const int *inc_nrow;                 // [c+1] breakpoints of row y
+    int inc_shm;                         // LDS bytes of the incremental back projector's two-bin workgroup
+    // one pair of bins' column in LDS: segment 0, then one window of cells per group
+    const int4 *inc_chunk;               // [inc_nchunk] {planes of segments 2k, 2k-1 (first of up to four), cell, planes | k << 8}
+    const int *inc_zero;                 // [4K+1] cells that stay zero
+    const int2 *inc_cell;                // [inc_ncell] {cell | kind << 16, bits(tan)}, ascending
+    int inc_nchunk, inc_ncell;
+    const int4 *inc_group;               // [K][3] per group: window, first-row lookups, row c+1 breakpoint
+    const int4 *inc_sched;               // breakpoints of rows c-2 down to 1, groups ascending, and 128 unused ones
+    const int *inc_count;                // [c+1] breakpoints of rows c-2 .. y
     int fp_maxt, fp_nsplit;              // forward-projector launch shape asked for (tasks/thread, workgroups/(pair,x)), 0: by rule
     int bp_waves;                        // back-projector waves per workgroup
 };

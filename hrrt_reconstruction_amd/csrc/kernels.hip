@@ -635,198 +635,295 @@ __global__ void __launch_bounds__(1024) bp_kernel(const DevGeom g, const PairBat
 // column's rows away from the centre, each plane keeps running sums s1 (row y)
 // and s2 (row N-y) and their per-row increments d1, d2; at the rows where a
 // group's integer shift changes (the breakpoints of blutacc, PJ:718-784) the
-// increments are corrected.  One workgroup per (column x <= N/2, lane, view
-// pair); lane l is bin x or N-x (l & 1) of view v or v+90 (l >> 1); a thread
-// owns one plane and applies, to its own accumulators, exactly the terms the
-// reference's loops apply to that plane, in the reference's order.  Lanes 0/1
-// write the rotated-frame half A, lanes 2/3 the half B, so each voxel of A and
+// increments are corrected.  One workgroup per (column x <= N/2, view v or
+// v+90, view pair), for NB = 2 bins x and N-x, or for one of them (NB = 1); a thread
+// owns one plane of its bins and applies, to its own accumulators, exactly the terms the
+// reference's loops apply to that plane, in the reference's order.  View v
+// writes the rotated-frame half A, view v+90 the half B, so each voxel of A and
 // of B has one writer and R = A + B as for the direct variant.
 //
-// LDS: segment 0, then per group a window of float2 {segment 2k, 2k-1} by row
-// (layout and the two in-place conversions are described with the host
-// tables).  A breakpoint is then, for every plane, two clamped float2 reads
-// and eight fixed operations (b-term first, then a-term, each one s += m*coef,
-// d -= m for both sums); the reads that fall outside the breakpoint's rows hit
-// the window's zero cells and add +0.  Breakpoint records come through the
-// scalar cache one ahead of use; per-group constants sit in VGPRs (lane k-1).
+// LDS: segment 0, then per group a window of cells by row (layout described with the host tables).  The
+// centre and the first row read the raw column and form the reference's differences from it; the window
+// is then converted once, in place, to the values the breakpoint terms read.  A breakpoint
+// is then, for every plane, two clamped reads and eight fixed operations per bin (b-term first, then
+// a-term, each one s += m*coef, d -= m for both sums); the reads that fall outside the breakpoint's rows
+// hit the window's zero cells and add +0.
+//
+// What bounds it (9 pairs at 256 x 256, span 3, 0.346 ms; 0.435 with one bin per workgroup, scalar loads of the
+// records and table-driven staging): VALU issue (149 M wave instructions, 78 % of the SIMDs' time at
+// four cycles each), then the 0.7 GB of halves written, which alone take 0.11 ms. Two bins per thread share a
+// breakpoint's record, addresses and reads; its cells are read while the one before is applied, across the
+// rows; the longest columns start first.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ int rl(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
-__device__ __forceinline__ float rlf(int v, int lane) { return __int_as_float(__builtin_amdgcn_readlane(v, lane)); }
 __device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
-__global__ void __launch_bounds__(256) bp_inc_kernel(const DevGeom g, const PairBatch b, const float *__restrict__ src,
-                                                     int src_global, int apply_rescale,
-                                                     const int16_t *__restrict__ pseg, float *__restrict__ bufA,
-                                                     float *__restrict__ bufB) {
-    extern __shared__ float P[];
-    const float2 *W = reinterpret_cast<const float2 *>(P);
-    const int x = blockIdx.x + 1, l = blockIdx.y, lp = blockIdx.z % b.npairs, frame = blockIdx.z / b.npairs;
-    const int N = g.N, c = g.c, Z = g.Z, K = g.K;
-    if (x == c && (l & 1)) return;          // at x == N/2 lanes 1/3 duplicate lanes 0/2
+// A cell of the window: {segment 2k, segment 2k-1} of each of the NB bins.
+template <int NB>
+struct __attribute__((aligned(8 * NB))) IncCell {
+    float2 b[NB];
+};
+__device__ __forceinline__ float2 sub2(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
+__device__ __forceinline__ float2 mul2(float2 a, float s) { return make_float2(a.x * s, a.y * s); }
+
+template <int NB>
+__global__ void __launch_bounds__(256, NB == 2 ? 3 : 6) bp_inc_kernel(const DevGeom g, const PairBatch b,
+                                                                    const float *__restrict__ src, int src_global,
+                                                                    int apply_rescale, float *__restrict__ bufA,
+                                                                    float *__restrict__ bufB) {
+    constexpr int ITEMS = 4;    // chunks a thread has in flight while the column loads
+    constexpr int CELLS = 13;        // cells a thread converts between two barriers
+    extern __shared__ float4 inc_lds[];
+    typedef IncCell<NB> Cell;
+    Cell *W = reinterpret_cast<Cell *>(inc_lds);
+    float *S0 = reinterpret_cast<float *>(inc_lds);   // [Z][NB]
+    const int N = g.N, c = g.c, Z = g.Z, K = g.K, NT = blockDim.x;
+    const int x = c - blockIdx.x, h = NB == 2 ? blockIdx.y : blockIdx.y >> 1, second = NB == 2 ? 0 : blockIdx.y & 1;
+    const int lp = blockIdx.z % b.npairs, frame = blockIdx.z / b.npairs;
     const int lo = g.cyl_lo[x], hi = g.cyl_hi[x];
-    if (lo == hi) return;
+    if (lo == hi || (second && x == c)) return;    // at x == N/2 the second bin duplicates the first
     const int view = b.view0 + b.view_stride * lp;
-    const int h = l >> 1, col = (l & 1) ? N - x : x;
-    const int z = threadIdx.x, lane = threadIdx.x & 63;
-    const bool act = z < Z;
-    float *dst = (l < 2 ? bufA : bufB) + frame * b.buf_stride + (size_t)lp * N * N * g.Z4;
+    const int tid = threadIdx.x;
+    const int z = tid < Z ? tid : Z - 1;    // the threads behind the last plane repeat it: no store is masked
+    const int col = second ? N - x : x;     // the first bin
+    const bool two = NB == 2 && x != c;
     // s1 of row y goes to A(col, y) / B(N-y, col), s2 to A(col, N-y) / B(y, col)
-    auto vox = [&](int y, bool second) -> float * {
-        const int X = l < 2 ? col : (second ? y : N - y);
-        const int Y = l < 2 ? (second ? N - y : y) : col;
-        return dst + ((size_t)X * N + Y) * g.Z4;
+    float *dst = (h == 0 ? bufA : bufB) + frame * b.buf_stride + (size_t)lp * N * N * g.Z4;
+    const long long step = h == 0 ? -g.Z4 : (long long)N * g.Z4;             // of s1 per row towards the edge
+    const long long other = (h == 0 ? (long long)(N - 2 * x) * N : N - 2 * x) * g.Z4;   // from bin x to bin N-x
+    float *o1 = dst + (h == 0 ? (size_t)col * N + c : (size_t)c * N + col) * g.Z4, *o2 = o1;   // row c
+    auto put = [&](float *o, const float (&v)[NB]) __attribute__((always_inline)) {
+        o[z] = v[0];
+        if (two) o[other + z] = v[NB - 1];
     };
     const int ylast = lo < c - 1 ? lo : c - 1;                       // rows c-1 .. ylast are written
     if (g.nzmask[view * (c + 1) + x] == 0) {                          // masked column PJ:4236-4262
-        if (act) {
-            vox(c, false)[z] = 0.0f;
-            for (int y = c - 1; y >= ylast; y--) {
-                vox(y, false)[z] = 0.0f;
-                vox(y, true)[z] = 0.0f;
-            }
+        const float zero[NB] = {};
+        put(o1, zero);
+        for (int y = c - 1; y >= ylast; y--) {
+            o1 += step;
+            o2 -= step;
+            put(o1, zero);
+            put(o2, zero);
         }
         return;
     }
     src += frame * b.ratio_stride;
     const int gp = src_global ? view : lp;
-    const float *cp = src + ((size_t)(gp * 2 + h) * N + col) * g.spp;
-    for (int base = 0; base < g.inc_lds; base += 4 * (int)blockDim.x) {   // transpose PJ:1654-1693
-        int si[4];
+    const float *cp[NB];
+    cp[0] = src + ((size_t)(gp * 2 + h) * N + col) * g.spp;
+    if (NB == 2) cp[NB - 1] = cp[0] + (long long)(N - 2 * x) * g.spp;
+    // column -> LDS (transpose PJ:1654-1693): chunks of four planes of the segments 2k and 2k-1
+    const bool wide = (reinterpret_cast<uintptr_t>(src) & 15) == 0;   // columns are whole 16-byte words apart
+    auto load4 = [&](const float *p) __attribute__((always_inline)) {
+        if (wide) return *reinterpret_cast<const float4 *>(p);
+        return make_float4(p[0], p[1], p[2], p[3]);
+    };
+    for (int base = tid; base < g.inc_nchunk; base += ITEMS * NT) {
+        int4 it[ITEMS];
+        float4 va[ITEMS][NB], vb[ITEMS][NB];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int i = base + threadIdx.x + j * blockDim.x;
-            si[j] = i < g.inc_lds ? g.inc_src[i] : -1;
-        }
-        float v[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            v[j] = 0.0f;
-            if (si[j] >= 0) v[j] = apply_rescale ? cp[si[j]] * g.bp_rescale[pseg[si[j]]] : cp[si[j]];
+        for (int j = 0; j < ITEMS; j++) {
+            it[j] = make_int4(0, 0, 0, 0);
+            if (base + j * NT < g.inc_nchunk) it[j] = g.inc_chunk[base + j * NT];
         }
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int i = base + threadIdx.x + j * blockDim.x;
-            if (i < g.inc_lds) P[i] = v[j];
-        }
-    }
-    // per-group constants of group lane+1
-    int4 e0 = make_int4(0, 0, 0, 0), e1 = e0, e2 = e0, e3 = e0;
-    if (lane < K) {
-        const int4 *q = g.inc_group + 4 * lane;
-        e0 = q[0]; e1 = q[1]; e2 = q[2]; e3 = q[3];
-    }
-    __syncthreads();
-    const int zc = act ? z : 0;
-    // centre voxels PJ:4265-4285
-    {
-        float sv = P[zc];
-        for (int k = 0; k < K; k++) {
-            const int gb = rl(e0.x, k), yb = rl(e0.y, k), yt = rl(e0.z, k);
-            const float2 w = W[gb + clampi(z, yb, yt)];
-            const float t = sv + (w.x + w.y);
-            sv = (z >= yb && z <= yt) ? t : sv;
-        }
-        if (act) vox(c, false)[z] = sv;
-    }
-    // first row y = c-1 by direct interpolation PJ:4287-4312
-    float s1 = P[zc], s2 = s1, d1 = 0.0f, d2 = 0.0f;
-    for (int k = 0; k < K; k++) {
-        const int gb = rl(e0.x, k);
-        const int za = rl(e1.x, k), n = rl(e1.y, k), ya = rl(e1.z, k), zb = rl(e2.x, k), yb2 = rl(e2.y, k);
-        const float c1 = rlf(e1.w, k), c2 = rlf(e2.z, k);
-        const int ia = z - za, ib = z - zb, nm = n > 1 ? n - 1 : 0;
-        const bool va = ia >= 0 && ia < n, vb = ib >= 0 && ib < n;
-        const int ra = gb + ya + clampi(ia, 0, nm), rb = gb + yb2 + clampi(ib, 0, nm);
-        const float2 pa = W[ra], qa = W[ra + 1], pb = W[rb], qb = W[rb + 1];
-        const float a1 = pa.x + c1 * (qa.x - pa.x), a2 = pa.y + c1 * (qa.y - pa.y);
-        const float b1 = pb.y + c2 * (qb.y - pb.y), b2 = pb.x + c2 * (qb.x - pb.x);
-        if (zb <= za) {              // iteration ia <= ib: the row-y term first
-            s1 = va ? s1 + a1 : s1; s2 = va ? s2 + a2 : s2;
-            s1 = vb ? s1 + b1 : s1; s2 = vb ? s2 + b2 : s2;
-        } else {
-            s1 = vb ? s1 + b1 : s1; s2 = vb ? s2 + b2 : s2;
-            s1 = va ? s1 + a1 : s1; s2 = va ? s2 + a2 : s2;
-        }
-    }
-    __syncthreads();
-    // in place, twice: the reference's scaled differences P' (PJ:4313-4324), then the values the
-    // breakpoint terms read
-    for (int pass = 0; pass < 2; pass++) {
-        for (int base = 0; base < g.inc_lds; base += 4 * (int)blockDim.x) {
-            float nv[4];
+        for (int j = 0; j < ITEMS; j++) {
+            if (it[j].w == 0) continue;
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int i = base + threadIdx.x + j * blockDim.x;
-                nv[j] = 0.0f;
-                if (i < g.inc_lds) {
-                    const int2 cv = g.inc_conv[i];
-                    const float p = P[i];
-                    if (pass == 0) nv[j] = cv.x ? (P[i + 2] - p) * __int_as_float(cv.x) : p;
-                    else nv[j] = cv.y == 1 ? p - P[i + 2] : (cv.y == 2 ? -P[i + 2] : p);
+            for (int n = 0; n < NB; n++) {
+                va[j][n] = load4(cp[n] + it[j].x);
+                vb[j][n] = load4(cp[n] + it[j].y);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < ITEMS; j++) {
+            const int cnt = it[j].w & 0xff, k = it[j].w >> 8;
+            if (cnt == 0) continue;
+            if (apply_rescale) {
+                const float ra = g.bp_rescale[2 * k], rb = g.bp_rescale[2 * k - 1];
+#pragma unroll
+                for (int n = 0; n < NB; n++) {
+                    va[j][n] = mul4(va[j][n], ra);
+                    vb[j][n] = mul4(vb[j][n], rb);
                 }
             }
-            __syncthreads();
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int i = base + threadIdx.x + j * blockDim.x;
-                if (i < g.inc_lds) P[i] = nv[j];
+            for (int i = 0; i < 4; i++) {
+                Cell w;
+#pragma unroll
+                for (int n = 0; n < NB; n++) w.b[n] = make_float2(lane(va[j][n], i), lane(vb[j][n], i));
+                if (i < cnt) W[it[j].z + i] = w;
             }
-            __syncthreads();
         }
-        if (pass == 1) break;
-        for (int k = 0; k < K; k++) {                                // PJ:4325-4335
-            const int gb = rl(e0.x, k), yb = rl(e0.y, k), yt = rl(e0.z, k);
-            const int zs = rl(e3.x, k), ze = rl(e3.y, k), yr0 = rl(e3.z, k);
-            const bool vd = z >= yb - 1 && z <= yt;
-            const float2 w = W[gb + clampi(z, yb - 1, yt)];
-            const float t1 = d1 + w.x, t2 = d2 + w.y;
-            d1 = vd ? t1 : d1; d2 = vd ? t2 : d2;
-            const int j = z - zs;
-            const bool vj = j >= 0 && j <= ze - zs;
-            const float2 u = W[gb + yr0 + clampi(j, 0, ze > zs ? ze - zs : 0)];
-            const float u1 = d1 - u.y, u2 = d2 - u.x;
-            d1 = vj ? u1 : d1; d2 = vj ? u2 : d2;
+    }
+#pragma unroll
+    for (int n = 0; n < NB; n++) {
+        const float v = cp[n][g.seg_data[0] + z];
+        S0[NB * z + n] = apply_rescale ? v * g.bp_rescale[0] : v;
+    }
+    for (int i = tid; i < 4 * K + 1; i += NT) W[g.inc_zero[i]] = Cell{};
+    __syncthreads();
+    // Every group's terms on the raw column: the centre voxel (PJ:4265-4285), the first row y = c-1 by direct
+    // interpolation (PJ:4287-4312), and the increments from the scaled differences
+    // P'(yr) = (p(yr+1) - p(yr)) * tan (PJ:4313-4335).  Reads clamped to the zero cells around the segment
+    // give exactly +0 where the reference's plane ranges end.
+    float sv[NB], s1[NB], s2[NB], d1[NB], d2[NB];
+#pragma unroll
+    for (int n = 0; n < NB; n++) sv[n] = s1[n] = s2[n] = S0[NB * z + n], d1[n] = d2[n] = 0.0f;
+    for (int k = 0; k < K; k++) {
+        const int4 e0 = g.inc_group[3 * k], e1 = g.inc_group[3 * k + 1], e2 = g.inc_group[3 * k + 2];
+        const int gb = e0.x, yb = e0.y, yt = e0.z;
+        const float tn = __int_as_float(e0.w);
+        const Cell *G = W + gb;
+        const int ra = clampi(z + e1.x, yb - 2, yt + 1), rb = clampi(z + e1.z, yb - 2, yt + 1);
+        const int rd = clampi(z, yb - 2, yt + 1);
+        const Cell w0 = G[rd], w1 = G[rd + 1], pa = G[ra], qa = G[ra + 1], pb = G[rb], qb = G[rb + 1];
+        const float f1 = __int_as_float(e1.y), f2 = __int_as_float(e1.w);
+        const int zs = e2.x, ze = e2.y, j = z - zs;
+        const bool vj = j >= 0 && j <= ze - zs;
+        const int row = e2.z + clampi(j, 0, ze > zs ? ze - zs : 0);
+        const Cell q0 = G[row], q1 = G[row + 1];
+#pragma unroll
+        for (int n = 0; n < NB; n++) {
+            sv[n] = sv[n] + (w0.b[n].x + w0.b[n].y);
+            const float a1 = pa.b[n].x + f1 * (qa.b[n].x - pa.b[n].x), a2 = pa.b[n].y + f1 * (qa.b[n].y - pa.b[n].y);
+            const float b1 = pb.b[n].y + f2 * (qb.b[n].y - pb.b[n].y), b2 = pb.b[n].x + f2 * (qb.b[n].x - pb.b[n].x);
+            if (e2.w) {              // the row-y term first
+                s1[n] = (s1[n] + a1) + b1;
+                s2[n] = (s2[n] + a2) + b2;
+            } else {
+                s1[n] = (s1[n] + b1) + a1;
+                s2[n] = (s2[n] + b2) + a2;
+            }
+            const float2 w = mul2(sub2(w1.b[n], w0.b[n]), tn);
+            d1[n] = d1[n] + w.x;
+            d2[n] = d2[n] + w.y;
+            const float2 u = row <= yt ? mul2(sub2(q1.b[n], q0.b[n]), tn) : q0.b[n];   // row yt+1 is a zero cell
+            d1[n] = vj ? d1[n] - u.y : d1[n];
+            d2[n] = vj ? d2[n] - u.x : d2[n];
+        }
+    }
+    put(o1, sv);
+    o1 += step;
+    o2 -= step;
+    put(o1, s1);
+    put(o2, s2);
+    // The window, in place and upwards (a cell needs only itself and the two above): M(yr) = P'(yr) - P'(yr+1), M(yb-2) =
+    // -P'(yb-1), M(yt) = P'(yt)
+    for (int base = 0; base < g.inc_ncell; base += CELLS * NT) {
+        Cell m[CELLS];
+        int cell[CELLS];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < CELLS; j++) {
+            const int i = base + j * NT + tid;
+            cell[j] = -1;
+            if (i < g.inc_ncell) {
+                const int2 e = g.inc_cell[i];   // {cell | kind << 16, bits(tan)}
+                const float tn = __int_as_float(e.y);
+                const int kind = e.x >> 16;
+                cell[j] = e.x & 0xffff;
+                const Cell *r = W + cell[j];
+                const Cell p0 = r[0], p1 = r[1], p2 = r[2];
+#pragma unroll
+                for (int n = 0; n < NB; n++) {
+                    const float2 lower = mul2(sub2(p1.b[n], p0.b[n]), tn), upper = mul2(sub2(p2.b[n], p1.b[n]), tn);
+                    m[j].b[n] = kind == 1 ? make_float2(-upper.x, -upper.y) : (kind == 2 ? lower : sub2(lower, upper));
+                }
+            }
         }
         __syncthreads();
+#pragma unroll
+        for (int j = 0; j < CELLS; j++)
+            if (cell[j] >= 0) W[cell[j]] = m[j];
     }
-    if (act) {
-        vox(c - 1, false)[z] = s1;
-        vox(c - 1, true)[z] = s2;
-    }
-    // rows c-2 .. ystart PJ:4337-4562: breakpoints, then the running sums advance by their
-    // increments
-    const int z8 = 8 * z;
-    const char *Wb = reinterpret_cast<const char *>(P);
+    __syncthreads();
+    // rows c-2 .. lo PJ:4337-4562: breakpoints, then the running sums advance by their increments.  Stores
+    // take 32-bit byte offsets from two scalar bases (a pair's half holds < 2^32 bytes); LDS addresses are
+    // absolute, so the clamped offset is the address.
+    char *const h0 = reinterpret_cast<char *>(dst), *const h1 = h0 + 4 * other;
+    unsigned off1 = (unsigned)((o1 - dst + z) * 4), off2 = (unsigned)((o2 - dst + z) * 4);
+    const unsigned step4 = (unsigned)(int)(4 * step);
+    constexpr int CB = 8 * NB;   // bytes of a cell
+    const int lds0 = (int)(unsigned)(uintptr_t)(__attribute__((address_space(3))) const float4 *)inc_lds;
+    const int zoff = lds0 + CB * z, lane64 = tid & 63;
     const int4 *__restrict__ T = g.inc_sched;
-    int e = 0;
-    int4 cur = T[0];
-    for (int y = c - 2; y >= lo; y--) {
-        const int n = g.inc_nrow[y];
-        for (int j = 0; j < n; j++) {
-            const int4 nxt = T[e + 1];
-            const float cf = __int_as_float(cur.x);
-            const int lo8 = cur.w & 0xffff, hi8 = cur.w >> 16;
-            // lo8 < hi8 always, so the clamp is max(lo, min(v, hi)): two VALU instead of a compare,
-            // a select and a min
-            const int ra = max(lo8, min(z8 + cur.y, hi8)), rb = max(lo8, min(z8 + cur.z, hi8));
-            const float2 ma = *reinterpret_cast<const float2 *>(Wb + ra);
-            const float2 mb = *reinterpret_cast<const float2 *>(Wb + rb);
+    struct Record {
+        int cf, oa, ob, lo, hi, row;
+    };
+    struct Cells {
+        Cell a, b;
+    };
+    auto read = [&](const Record &r) __attribute__((always_inline)) {
+        typedef float vn __attribute__((ext_vector_type(2 * NB)));
+        typedef __attribute__((address_space(3))) const vn *LdsCell;
+        // lo < hi always, so the clamp is max(lo, min(v, hi))
+        const int ra = max(r.lo, min(zoff + r.oa, r.hi)), rb = max(r.lo, min(zoff + r.ob, r.hi));
+        const vn va = *(LdsCell)(uintptr_t)(unsigned)ra, vb = *(LdsCell)(uintptr_t)(unsigned)rb;
+        Cells m;
+#pragma unroll
+        for (int n = 0; n < NB; n++) m.a.b[n] = make_float2(va[2 * n], va[2 * n + 1]), m.b.b[n] = make_float2(vb[2 * n], vb[2 * n + 1]);
+        return m;
+    };
+    int y = c - 2;
+    auto rows_to = [&](int row) __attribute__((always_inline)) {   // rows y .. row + 1
+        for (; y > row; y--) {
+#pragma unroll
+            for (int n = 0; n < NB; n++) s1[n] = s1[n] + d1[n], s2[n] = s2[n] + d2[n];
+            off1 += step4;
+            off2 -= step4;
+            *reinterpret_cast<float *>(h0 + off1) = s1[0];
+            *reinterpret_cast<float *>(h0 + off2) = s2[0];
+            if (two) {
+                *reinterpret_cast<float *>(h1 + off1) = s1[NB - 1];
+                *reinterpret_cast<float *>(h1 + off2) = s2[NB - 1];
+            }
+        }
+    };
+    auto apply = [&](const Record &r, const Cells &m) __attribute__((always_inline)) {
+        rows_to(r.row);
+        const float cf = __int_as_float(r.cf);
+#pragma unroll
+        for (int n = 0; n < NB; n++) {
             // b-term (PJ:4386-4391 for rows N-y): s1 += m2*coef, s2 += m1*coef, d1 -= m2, d2 -= m1
-            s1 = s1 + mb.y * cf; d1 = d1 - mb.y;
-            s2 = s2 + mb.x * cf; d2 = d2 - mb.x;
+            s1[n] = s1[n] + m.b.b[n].y * cf; d1[n] = d1[n] - m.b.b[n].y;
+            s2[n] = s2[n] + m.b.b[n].x * cf; d2[n] = d2[n] - m.b.b[n].x;
             // a-term (PJ:4382-4385): s1 += m1*coef, s2 += m2*coef, d1 -= m1, d2 -= m2
-            s1 = s1 + ma.x * cf; d1 = d1 - ma.x;
-            s2 = s2 + ma.y * cf; d2 = d2 - ma.y;
-            cur = nxt;
-            e++;
+            s1[n] = s1[n] + m.a.b[n].x * cf; d1[n] = d1[n] - m.a.b[n].x;
+            s2[n] = s2[n] + m.a.b[n].y * cf; d2[n] = d2[n] - m.a.b[n].y;
         }
-        s1 = s1 + d1;
-        s2 = s2 + d2;
-        if (act) {
-            vox(y, false)[z] = s1;
-            vox(y, true)[z] = s2;
+    };
+    const int E = lo < c - 1 ? g.inc_count[lo] : 0;   // breakpoints of rows c-2 .. lo
+    // A wave holds 64 records, one per lane, unpacked once, and takes them with readlane (scalar loads
+    // would make every wait for a cell one for the records behind it too: 0.371 ms against 0.351).  The last
+    // two of a batch are the first two of the next, so that a record's successors are always at hand.
+    auto unpack = [&](const int4 &t) __attribute__((always_inline)) {
+        return Record{t.x, (t.y >> 4) * CB, (t.z >> 4) * CB, lds0 + (t.w & 0xffff) * CB, lds0 + (int)((unsigned)t.w >> 16) * CB,
+                      (t.y & 15) | ((t.z & 15) << 4)};
+    };
+    int4 ahead = T[lane64];
+    for (int e0 = 0; e0 < E; e0 += 62) {
+        const Record rec = unpack(ahead);
+        ahead = T[e0 + 62 + lane64];
+        auto get = [&](int i) __attribute__((always_inline)) {
+            auto rl = [&](int v) __attribute__((always_inline)) { return __builtin_amdgcn_readlane(v, i); };
+            return Record{rl(rec.cf), rl(rec.oa), rl(rec.ob), rl(rec.lo), rl(rec.hi), rl(rec.row)};
+        };
+        const int n = E - e0 < 62 ? E - e0 : 62;
+        Record r0 = get(0);
+        Cells m0 = read(r0);
+        int i = 0;
+        for (; i + 2 <= n; i += 2) {
+            const Record r1 = get(i + 1);
+            const Cells m1 = read(r1);
+            apply(r0, m0);
+            r0 = get(i + 2);
+            m0 = read(r0);
+            apply(r1, m1);
         }
+        if (i < n) apply(r0, m0);
     }
+    rows_to(lo - 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -1625,9 +1722,17 @@ static dim3 rot_grid(const DevGeom &g, int nframes = 1) { return dim3(g.N * ((g.
 hipError_t launch_backproject_incremental(const DevGeom &g, const PairBatch &b, const float *src, int src_global,
                                           int apply_rescale, float *bufA, float *bufB, hipStream_t s) {
     if (!g.inc_ok) return hipErrorInvalidValue;   // tables failed the host's window checks
-    dim3 grid(g.c, 4, b.npairs * b.nframes), block(256);
-    hipLaunchKernelGGL(bp_inc_kernel, grid, block, g.inc_shm, s, g, b, src, src_global, apply_rescale,
-                       g.pseg, bufA, bufB);
+    const dim3 block((g.Z + 63) / 64 * 64);
+    const int npf = b.npairs * b.nframes;
+    // Both bins of a ray in one workgroup share the breakpoints' work (9 pairs at 256 x 256, span 3: 0.346 ms
+    // against 0.408 with a bin each); below two such workgroups per CU a bin each fills the chip better (one
+    // view pair of that size, forward to image: 0.318 ms against 0.324; a 16-ring subset: 50.6 us against 51.9).
+    if ((long long)g.c * 2 * npf >= 512)
+        hipLaunchKernelGGL(bp_inc_kernel<2>, dim3(g.c, 2, npf), block, g.inc_shm, s, g, b, src, src_global, apply_rescale,
+                           bufA, bufB);
+    else
+        hipLaunchKernelGGL(bp_inc_kernel<1>, dim3(g.c, 4, npf), block, g.inc_shm / 2, s, g, b, src, src_global,
+                           apply_rescale, bufA, bufB);
     return hipGetLastError();
 }
 
