@@ -11,6 +11,7 @@
 #include <functional>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/hrrt_osem.h"
@@ -434,11 +435,10 @@ extern "C" int hrrt_create(const hrrt_params *params, hrrt_ctx **out) {
         }
     }
     for (int yr = 0; yr < Z; yr++) fsingle.push_back(make_int4((yr << 8) | (1 << 16), 0, 0, 0));   // axial planes last
-    std::vector<int16_t> pseg(G.spp, -1), plane_seg(G.segmentsize, 0);
+    std::vector<int16_t> pseg(G.spp, -1);
     for (int s = 0; s < G.th_pixels; s++)
         for (int i = 0; i < G.nplanes(s); i++) {
             pseg[G.seg_data[s] + i] = (int16_t)s;
-            plane_seg[G.segment_offset[s] + i] = (int16_t)s;
         }
     std::vector<int> file_seg(G.th_pixels);
     for (int s = 0; s < G.th_pixels; s++) {
@@ -446,6 +446,12 @@ extern "C" int hrrt_create(const hrrt_params *params, hrrt_ctx **out) {
         file_seg[s] = G.seg_offset[sw] / (N * G.views);
     }
     ctx->file_seg = file_seg;
+    std::vector<int2> stage_plane(G.spp, make_int2(-1, 0));
+    for (int s = 0; s < G.th_pixels; s++)
+        for (int i = 0; i < G.nplanes(s); i++) {
+            const bool killed = i < G.p.npskip || i + G.p.npskip >= G.nplanes(s);   // of the norm (FIO:110-180)
+            stage_plane[G.seg_data[s] + i] = make_int2(file_seg[s] + i, s | (killed << 8));
+        }
     std::vector<float> resc = G.rescalearray;
     // back-projection column in LDS: segment 0, then every oblique segment inside a window of
     // zero planes wide enough that the back projector's 64-plane slots 0-2 (z < 192) always,
@@ -611,7 +617,7 @@ extern "C" int hrrt_create(const hrrt_params *params, hrrt_ctx **out) {
         (r = ctx->upload(resc, d.rescalearray)) || (r = ctx->upload(blut, d.bp_lut)) ||
         (r = ctx->upload(rot, d.rot)) || (r = ctx->upload(fruns[0], d.fp_runs[0])) ||
         (r = ctx->upload(fruns[1], d.fp_runs[1])) || (r = ctx->upload(fsingle, d.fp_single)) || (r = ctx->upload(pseg, d.pseg)) ||
-        (r = ctx->upload(plane_seg, d.plane_seg)) || (r = ctx->upload(bp_src, d.bp_src)) ||
+        (r = ctx->upload(stage_plane, d.stage_plane)) || (r = ctx->upload(bp_src, d.bp_src)) ||
         (r = ctx->upload(blut2, d.bp_lut2)) || (r = ctx->upload(ichunk, d.inc_chunk)) ||
         (r = ctx->upload(izero, d.inc_zero)) || (r = ctx->upload(icell, d.inc_cell)) || (r = ctx->upload(igroup, d.inc_group)) ||
         (r = ctx->upload(isched, d.inc_sched)) || (r = ctx->upload(icount, d.inc_count))) {
@@ -728,8 +734,8 @@ extern "C" int hrrt_stage_sinograms(hrrt_ctx *ctx, const int16_t *d_prompt_file,
     if (d_norm_file && G.x_rebin * G.v_rebin > 1)
         if ((r = ctx->zalloc((void **)&ctx->gapmask, (size_t)G.th_pixels * G.p.def_angles * G.p.def_elements))) return r;
     HIP_TRY(hrrt::launch_stage(ctx->dg, d_prompt_file, d_delayed_file, d_norm_file, d_scatter_file, d_atten_file,
-                               d_prompt, d_add, d_invnorm, ctx->gapmask, ctx->colmask, 0, G.th_pixels, 0,
-                               G.segmentsize, true, S(stream)));
+                               d_prompt, d_add, d_invnorm, ctx->gapmask, ctx->colmask, 0, G.th_pixels, 0, G.spp, true,
+                               S(stream)));
     return HRRT_OK;
 }
 
@@ -752,7 +758,7 @@ extern "C" int hrrt_stage_sinograms_w012(hrrt_ctx *ctx, int weighting, int preco
         if ((r = ctx->zalloc((void **)&ctx->gapmask, (size_t)G.th_pixels * G.p.def_angles * G.p.def_elements))) return r;
     HIP_TRY(hrrt::launch_stage_w012(ctx->dg, weighting, precorrected != 0, d_data16_file, d_dataf_file, d_delayed_file,
                                     d_norm_file, d_scatter_file, d_atten_file, d_data, d_invnorm, ctx->gapmask,
-                                    ctx->colmask, 0, G.th_pixels, 0, G.segmentsize, true, S(stream)));
+                                    ctx->colmask, 0, G.th_pixels, 0, G.spp, true, S(stream)));
     return HRRT_OK;
 }
 
@@ -768,6 +774,12 @@ struct HostFile {
     const void *src;   // host memory of the whole flat file, or null (file absent)
     size_t elem;       // bytes per element
 };
+
+// The padded planes that segment th's launch writes: its own and the guards before them (behind the last one too).
+static std::pair<int, int> segment_columns(const hrrt::Geometry &G, int th) {
+    const int q0 = th == 0 ? 0 : G.seg_data[th - 1] + G.nplanes(th - 1);
+    return {q0, th == G.th_pixels - 1 ? G.spp : G.seg_data[th] + G.nplanes(th)};
+}
 
 static int stage_host(hrrt_ctx *ctx, HostFile files[5], void *dev[5], hipStream_t s,
                       const std::function<hipError_t(int th, bool finish)> &launch) {
@@ -835,10 +847,10 @@ extern "C" int hrrt_stage_sinograms_host(hrrt_ctx *ctx, const int16_t *prompt_fi
     HostFile files[5] = {{prompt_file, 2}, {delayed_file, 4}, {norm_file, 4}, {scatter_file, 4}, {atten_file, 4}};
     void *dev[5];
     return stage_host(ctx, files, dev, S(stream), [&](int th, bool finish) {
-        const int p0 = G.segment_offset[th], p1 = p0 + G.yr_top[th] - G.yr_bottom[th] + 1;
+        const auto [q0, q1] = segment_columns(G, th);
         return hrrt::launch_stage(ctx->dg, (const int16_t *)dev[0], (const float *)dev[1], (const float *)dev[2],
                                   (const float *)dev[3], (const float *)dev[4], d_prompt, d_add, d_invnorm,
-                                  ctx->gapmask, ctx->colmask, th, 1, p0, p1, finish, S(stream));
+                                  ctx->gapmask, ctx->colmask, th, 1, q0, q1, finish, S(stream));
     });
 }
 
@@ -864,12 +876,12 @@ extern "C" int hrrt_stage_sinograms_w012_host(hrrt_ctx *ctx, int weighting, int 
                          {delayed_file, 4}, {norm_file, 4}, {scatter_file, 4}, {atten_file, 4}};
     void *dev[5];
     return stage_host(ctx, files, dev, S(stream), [&](int th, bool finish) {
-        const int p0 = G.segment_offset[th], p1 = p0 + G.yr_top[th] - G.yr_bottom[th] + 1;
+        const auto [q0, q1] = segment_columns(G, th);
         return hrrt::launch_stage_w012(ctx->dg, weighting, precorrected != 0,
                                        data16_file ? (const int16_t *)dev[0] : nullptr,
                                        data16_file ? nullptr : (const float *)dev[0], (const float *)dev[1],
                                        (const float *)dev[2], (const float *)dev[3], (const float *)dev[4], d_data,
-                                       d_invnorm, ctx->gapmask, ctx->colmask, th, 1, p0, p1, finish, S(stream));
+                                       d_invnorm, ctx->gapmask, ctx->colmask, th, 1, q0, q1, finish, S(stream));
     });
 }
 

@@ -1321,13 +1321,13 @@ struct StageArgs {
     float *add, *invnorm;
     const uint8_t *gapmask;   // [th][def_angles][def_elements] when rebinning the norm
     int *colmask;             // [views][N]
-    const int16_t *plane_seg; // [S]
     // UW/AW/ANW staging (weighting 0, 1, 2; 3 = OP above): prompt_f holds short prompts or
     // trues, dataf_f a float sinogram (fully precorrected when precor); data is the output
     int weighting = 3, precor = 0;
     const float *dataf_f = nullptr;
     float *data = nullptr;
-    int p_lo = 0, p_hi = 0;   // internal planes [p_lo, p_hi) staged by this launch
+    int q_lo = 0, q_hi = 0;   // padded planes [q_lo, q_hi) of a column written by this launch
+    bool wide = false;        // the files are 16-byte aligned and so are the outputs
 };
 
 __device__ __forceinline__ float rebin_sum(const DevGeom &g, const float *f, size_t fplane, int v, int col) {
@@ -1390,59 +1390,57 @@ __device__ __forceinline__ int16_t rebin_short(const DevGeom &g, const int16_t *
     return out;
 }
 
-// mask of file (view, bin) with a positive norm in some non-killed plane of segment th (FIO:158-160)
-__global__ void gapmask_kernel(const DevGeom g, const float *__restrict__ norm_f, uint8_t *__restrict__ gm, int th0) {
+// mask of file (view, bin) with a positive norm in some non-killed plane of segment th (FIO:158-160).  A
+// thread takes four file bins (VEC; their count is a multiple of four) and eight planes at a time.
+template <bool VEC>
+__global__ void __launch_bounds__(256) gapmask_kernel(const DevGeom g, const float *__restrict__ norm_f,
+                                                      uint8_t *__restrict__ gm, int th0) {
+    constexpr int NB = VEC ? 4 : 1;
     const int th = th0 + blockIdx.y;
     const size_t fp = (size_t)g.def_angles * g.def_elements;
-    const int np = g.yt[th] - g.yb[th] + 1;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < fp; i += (size_t)gridDim.x * blockDim.x) {
-        uint8_t m = 0;
-        for (int pl = 0; pl < np; pl++) {
-            if (pl < g.npskip || pl + g.npskip >= np) continue;
-            if (norm_f[((size_t)g.file_seg[th] + pl) * fp + i] > 0.0f) m = 1;
+    const size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * NB;
+    if (i >= fp) return;
+    const int np = g.yt[th] - g.yb[th] + 1, p1 = np - g.npskip;
+    const float *f = norm_f + (size_t)g.file_seg[th] * fp + i;
+    bool m[NB] = {};
+    int pl = g.npskip;
+    auto take = [&](int p) __attribute__((always_inline)) {
+        if constexpr (VEC) {
+            const float4 x = *reinterpret_cast<const float4 *>(f + (size_t)p * fp);
+            m[0] |= x.x > 0.0f, m[NB > 1 ? 1 : 0] |= x.y > 0.0f, m[NB > 2 ? 2 : 0] |= x.z > 0.0f, m[NB > 3 ? 3 : 0] |= x.w > 0.0f;
+        } else {
+            m[0] |= f[(size_t)p * fp] > 0.0f;
         }
-        gm[th * fp + i] = m;
+    };
+    for (; pl + 8 <= p1; pl += 8) {
+#pragma unroll
+        for (int k = 0; k < 8; k++) take(pl + k);
     }
+    for (; pl < p1; pl++) take(pl);
+#pragma unroll
+    for (int n = 0; n < NB; n++) gm[th * fp + i + n] = m[n];
 }
 
-// One element (internal plane p, view v, bin col) of the staging: the corrected data or the
-// additive term (o1), the sensitivity weight (o_inv) and, for OP, the prompt (o_pr); flags the
-// column when its norm is non-zero.
-__device__ __forceinline__ void stage_one(const DevGeom &g, const StageArgs &a, int p, int v, int col, float &o1,
-                                          float &o_inv, int16_t &o_pr) {
-    const int th = a.plane_seg[p];
-    const int i = p - g.segment_offset[th];
-    const int np = g.yt[th] - g.yb[th] + 1;
-    const size_t fplane = (size_t)g.file_seg[th] + i;
-    const int rebin = g.x_rebin * g.v_rebin;
-    // norm (read with norm_flag = 1, FIO:110-180)
-    float nrm = 1.0f;
-    if (a.norm_f) {
-        if (i < g.npskip || i + g.npskip >= np) {
-            nrm = 0.0f;
-        } else if (rebin == 1) {
-            nrm = rebin_sum(g, a.norm_f, fplane, v, col);
-        } else {
-            nrm = rebin_norm(g, a.norm_f, fplane, v, col);
-            const size_t fp = (size_t)g.def_angles * g.def_elements;
-            int cnt = 0;
-            for (int vr = 0; vr < g.v_rebin; vr++)
-                for (int xr = 0; xr < g.x_rebin; xr++)
-                    cnt += a.gapmask[th * fp + (size_t)(v * g.v_rebin + vr) * g.def_elements + col * g.x_rebin + xr];
-            if (cnt < rebin) nrm = 0.0f;
-        }
-    }
-    const float d = a.delayed_f ? rebin_sum(g, a.delayed_f, fplane, v, col) : 0.0f;
-    const float at = a.atten_f ? rebin_sum(g, a.atten_f, fplane, v, col) : 1.0f;
-    if (nrm != 0.0f) atomicOr(&a.colmask[v * g.N + col], 1);
-    if (a.weighting < 3) {
+// What the files hold for one bin of the staging, rebinned: the norm (0 where the plane is killed or the gap mask
+// says so, 1 without a norm file), the delayed and scatter (0 without), the attenuation (1 without), and
+// the prompts (OP) or the data (UW, AW, ANW).
+struct StageBin {
+    float nrm, d, sc, at, data;
+    int16_t pr;
+};
+
+// One element of the staging: the corrected data or the additive term (o1), the sensitivity weight
+// (o_inv) and, for OP, the prompt (pr).
+template <bool OP>
+__device__ __forceinline__ void stage_one(const DevGeom &g, const StageArgs &a, StageBin &in, float &o1, float &o_inv) {
+    const float nrm = in.nrm, at = in.at;
+    const float am = at < 1.0f ? 1.0f : at;
+    if constexpr (!OP) {
         // prepare_osem3dw0 S3:1198-1256, w1 S3:1346-1407 and w2 S3:1505-1546; precorrected data
         // S3:1309-1323, 1410-1482, 1548-1636; then setnegative2zero simd_operation.cpp:78-96
-        float t;
+        float t = in.data;
         if (!a.precor) {
-            t = a.prompt_f ? rebin_short_f(g, a.prompt_f, fplane, v, col) : rebin_sum(g, a.dataf_f, fplane, v, col);
-            if (a.delayed_f) t = t - d;                               // readsinogram S3:1124-1131
-            const float sc = a.scatter_f ? rebin_sum(g, a.scatter_f, fplane, v, col) : 0.0f;
+            if (a.delayed_f) t = t - in.d;                            // readsinogram S3:1124-1131
             if (a.weighting == 0) {
                 if (a.norm_f) {
                     t = t * nrm;                                      // S3:1224, 1244
@@ -1451,87 +1449,252 @@ __device__ __forceinline__ void stage_one(const DevGeom &g, const StageArgs &a, 
                 if (a.atten_f) t = t * at;                            // S3:1253
             } else if (a.weighting == 1) {
                 if (a.scatter_f) {
-                    if (a.norm_f) t = nrm > 0.0f ? t - sc / nrm : 0.0f;   // S3:1380-1382
-                    else t = t - sc;                                      // S3:1389
+                    if (a.norm_f) t = nrm > 0.0f ? t - in.sc / nrm : 0.0f;   // S3:1380-1382
+                    else t = t - in.sc;                                      // S3:1389
                 }
                 if (a.norm_f) t = t * nrm;                                // S3:1405
             } else if (a.scatter_f) {
-                t = nrm > 0.0f ? t - sc / nrm : 0.0f;                     // S3:1535-1537
+                t = nrm > 0.0f ? t - in.sc / nrm : 0.0f;                  // S3:1535-1537
             }
         } else {
-            t = rebin_sum(g, a.dataf_f, fplane, v, col);
             if (a.weighting == 2) t = nrm > 0.0f ? t / nrm : 0.0f;        // S3:1564-1566
             if (a.weighting >= 1 && a.atten_f && at > 0.0f) t = t / at;  // divideprojection simd_operation.cpp:34
         }
         o1 = t > 0.0f ? t : 0.0f;
-        float inv;
         if (a.weighting == 0) {                                           // norm_UW S3:756-771
-            inv = nrm > 0.0f ? 1.0f : nrm;
-        } else if (a.weighting == 1) {                                    // norm_AW S3:774-791
-            inv = nrm > 0.0f ? 1.0f / (at < 1.0f ? 1.0f : at) : 0.0f;
-        } else {                                                          // norm_ANW S3:796-821
-            const float am = at < 1.0f ? 1.0f : at;
-            if (nrm > 0.0f) {
-                const float den = nrm * am;
-                inv = den > g.eps2 ? 1.0f / den : 0.0f;
-            } else {
-                inv = nrm;
-            }
+            o_inv = nrm > 0.0f ? 1.0f : nrm;
+            return;
         }
-        o_inv = inv;
-        return;
-    }
-    int16_t pr = 0;
-    if (a.prompt_f) pr = rebin_short(g, a.prompt_f, fplane, v, col);
-    float ad = d * nrm;                                     // mulprojection S3:1715
-    if (nrm == 0.0f) pr = 0;                                // S3:1720-1724
-    if (a.scatter_f) ad = ad + rebin_sum(g, a.scatter_f, fplane, v, col);  // addprojection S3:1753
-    ad = ad * at;                                           // mulprojection S3:1769
-    float inv;                                              // norm_ANW S3:809-817
-    const float am = at < 1.0f ? 1.0f : at;
-    if (nrm > 0.0f) {
-        const float den = nrm * am;
-        inv = den > g.eps2 ? 1.0f / den : 0.0f;
+        if (a.weighting == 1) {                                           // norm_AW S3:774-791
+            o_inv = nrm > 0.0f ? 1.0f / am : 0.0f;
+            return;
+        }
     } else {
-        inv = nrm;
+        float ad = in.d * nrm;                                  // mulprojection S3:1715
+        if (nrm == 0.0f) in.pr = 0;                             // S3:1720-1724
+        if (a.scatter_f) ad = ad + in.sc;                       // addprojection S3:1753
+        o1 = ad * at;                                           // mulprojection S3:1769
     }
-    o_pr = pr;
-    o1 = ad;
-    o_inv = inv;
+    if (nrm > 0.0f) {                                           // norm_ANW S3:796-821
+        const float den = nrm * am;
+        o_inv = den > g.eps2 ? 1.0f / den : 0.0f;
+    } else {
+        o_inv = nrm;
+    }
 }
 
-// Staging of internal planes [p_lo, p_hi): a workgroup computes a tile of 32 planes x 64 bins of
-// one view in the files' layout (bins contiguous, coalesced reads), turns it in LDS, and writes
-// it in the pair-column layout (planes contiguous, coalesced writes).
+// The bins of one staging item from the files: NB output bins from `col` of file plane fplane, view v, by
+// 16-byte loads (RB = 1: four bins; RB = 2: two bins of 2 x 2 file bins) or one by one (RB = 0).
+template <bool OP, int RB, int NB>
+__device__ __forceinline__ void stage_load(const DevGeom &g, const StageArgs &a, int th, size_t fplane, int v, int col,
+                                           bool killed, StageBin (&in)[NB]) {
+    const bool norm = a.norm_f && !killed;
+    const int DE = g.def_elements;
+#pragma unroll
+    for (int n = 0; n < NB; n++) {
+        in[n].nrm = a.norm_f ? 0.0f : 1.0f;
+        in[n].d = in[n].sc = in[n].data = 0.0f;
+        in[n].at = 1.0f;
+        in[n].pr = 0;
+    }
+    if constexpr (RB == 0) {
+        const size_t fp = (size_t)g.def_angles * DE;
+        if (norm) {
+            if (g.x_rebin * g.v_rebin == 1) {
+                in[0].nrm = rebin_sum(g, a.norm_f, fplane, v, col);
+            } else {
+                in[0].nrm = rebin_norm(g, a.norm_f, fplane, v, col);
+                int cnt = 0;
+                for (int vr = 0; vr < g.v_rebin; vr++)
+                    for (int xr = 0; xr < g.x_rebin; xr++)
+                        cnt += a.gapmask[th * fp + (size_t)(v * g.v_rebin + vr) * DE + col * g.x_rebin + xr];
+                if (cnt < g.x_rebin * g.v_rebin) in[0].nrm = 0.0f;
+            }
+        }
+        if (a.delayed_f) in[0].d = rebin_sum(g, a.delayed_f, fplane, v, col);
+        if (a.scatter_f) in[0].sc = rebin_sum(g, a.scatter_f, fplane, v, col);
+        if (a.atten_f) in[0].at = rebin_sum(g, a.atten_f, fplane, v, col);
+        if (OP) {
+            if (a.prompt_f) in[0].pr = rebin_short(g, a.prompt_f, fplane, v, col);
+        } else {
+            in[0].data = a.prompt_f && !a.precor ? rebin_short_f(g, a.prompt_f, fplane, v, col) : rebin_sum(g, a.dataf_f, fplane, v, col);
+        }
+    } else {
+        // rows of the item: RB file rows of four file bins each
+        const size_t row = fplane * (size_t)g.def_angles * DE + (size_t)(v * RB) * DE + col * RB;
+        struct F {
+            float4 r[RB];
+        };
+        struct S {
+            short4 r[RB];
+        };
+        auto rows = [&](const float *f) __attribute__((always_inline)) {
+            F x;
+#pragma unroll
+            for (int k = 0; k < RB; k++) x.r[k] = *reinterpret_cast<const float4 *>(f + row + (size_t)k * DE);
+            return x;
+        };
+        auto srows = [&](const int16_t *f) __attribute__((always_inline)) {
+            S x;
+#pragma unroll
+            for (int k = 0; k < RB; k++) x.r[k] = *reinterpret_cast<const short4 *>(f + row + (size_t)k * DE);
+            return x;
+        };
+        F fn{}, fd{}, fs{}, fa{}, ff{};
+        S sp{};
+        uchar4 gm[RB];
+        if (norm) {
+            fn = rows(a.norm_f);
+            if (RB > 1) {
+                const size_t fp = (size_t)g.def_angles * DE;
+#pragma unroll
+                for (int k = 0; k < RB; k++)
+                    gm[k] = *reinterpret_cast<const uchar4 *>(a.gapmask + th * fp + (size_t)(v * RB + k) * DE + col * RB);
+            }
+        }
+        if (a.delayed_f) fd = rows(a.delayed_f);
+        if (a.scatter_f) fs = rows(a.scatter_f);
+        if (a.atten_f) fa = rows(a.atten_f);
+        const bool shorts = a.prompt_f && (OP || !a.precor);
+        if (shorts) sp = srows(a.prompt_f);
+        else if (!OP) ff = rows(a.dataf_f);
+        // sino_rebin FIO:38-66: views summed first, then radial bins
+        auto sum = [&](const F &x, int n) __attribute__((always_inline)) {
+            if constexpr (RB == 1) return lane(x.r[0], n);
+            else return (lane(x.r[0], 2 * n) + lane(x.r[1], 2 * n)) + (lane(x.r[0], 2 * n + 1) + lane(x.r[1], 2 * n + 1));
+        };
+        auto slane = [](const short4 &x, int l) { return l == 0 ? x.x : (l == 1 ? x.y : (l == 2 ? x.z : x.w)); };
+        auto glane = [](const uchar4 &x, int l) { return l == 0 ? x.x : (l == 1 ? x.y : (l == 2 ? x.z : x.w)); };
+#pragma unroll
+        for (int n = 0; n < NB; n++) {
+            if (norm) {
+                if constexpr (RB == 1) {
+                    in[n].nrm = lane(fn.r[0], n);
+                } else {   // rebin_norm
+                    float c[2];
+                    int cnt = 0;
+#pragma unroll
+                    for (int xr = 0; xr < 2; xr++) {
+                        float t = lane(fn.r[0], 2 * n + xr);
+                        const float u = lane(fn.r[1], 2 * n + xr);
+                        if (t > 0.0f) t = 1.0f / t;
+                        if (u > 0.0f) t += 1.0f / u;
+                        c[xr] = t;
+                        cnt += glane(gm[0], 2 * n + xr) + glane(gm[1], 2 * n + xr);
+                    }
+                    float t = c[0] + c[1];
+                    if (t > 0.0f) t = 1.0f / t;
+                    in[n].nrm = cnt < 4 ? 0.0f : t;
+                }
+            }
+            if (a.delayed_f) in[n].d = sum(fd, n);
+            if (a.scatter_f) in[n].sc = sum(fs, n);
+            if (a.atten_f) in[n].at = sum(fa, n);
+            if constexpr (OP) {
+                if (shorts) {
+                    if constexpr (RB == 1) in[n].pr = slane(sp.r[0], n);
+                    else in[n].pr = (int16_t)((int16_t)(slane(sp.r[0], 2 * n) + slane(sp.r[1], 2 * n)) +
+                                              (int16_t)(slane(sp.r[0], 2 * n + 1) + slane(sp.r[1], 2 * n + 1)));
+                }
+            } else if (shorts) {   // rebin_short_f
+                if constexpr (RB == 1) in[n].data = (float)slane(sp.r[0], n);
+                else in[n].data = (0.0f + (float)(int16_t)(slane(sp.r[0], 2 * n) + slane(sp.r[1], 2 * n))) +
+                                  (float)(int16_t)(slane(sp.r[0], 2 * n + 1) + slane(sp.r[1], 2 * n + 1));
+            } else {
+                in[n].data = sum(ff, n);
+            }
+        }
+    }
+}
+
+// Staging of the padded planes [q_lo, q_hi) of every column (the zero guard planes among them): a workgroup
+// computes a tile of 64 planes x 64 bins of one view in the files' layout (bins contiguous, 16-byte loads),
+// turns it in LDS, and writes it in the pair-column layout (planes contiguous, 16-byte stores of whole 256-byte lines).
+// A column's flag is set once per tile, by a look before the atomic.
+//
+// What bounds it: HBM (a span-3 study: 8.5 GB read, 4.8 GB written).  With 32 x 64 tiles, one element per lane, a
+// flag atomic per element and the guards cleared beforehand it took 7.8 ms + 0.75 ms of clearing; now 3.7 ms, 3.6
+// TB/s, where a copy of that size reaches 4.35.  Tiles of 32 bins or planes take 3.95-4.04 ms.
+constexpr int STAGE_TILE = 64;
+
+template <bool OP, int RB>
 __global__ void __launch_bounds__(256) stage_kernel(const DevGeom g, StageArgs a) {
-    __shared__ float t_o1[64][33], t_inv[64][33];
-    __shared__ int16_t t_pr[64][34];
+    constexpr int NB = RB == 1 ? 4 : (RB == 2 ? 2 : 1);   // bins of an item
+    constexpr int LANES = STAGE_TILE / NB, ROWS = 256 / LANES;    // items across the tile's bins, planes per pass
+    __shared__ float t_o1[STAGE_TILE][STAGE_TILE + 1], t_inv[STAGE_TILE][STAGE_TILE + 1];
+    __shared__ int16_t t_pr[OP ? STAGE_TILE : 1][STAGE_TILE + 2];
+    __shared__ int t_live[STAGE_TILE];
     const int N = g.N, V = g.views;
-    const int p0 = a.p_lo + 32 * (int)blockIdx.x, v = blockIdx.y, c0 = 64 * (int)blockIdx.z;
-    for (int e = threadIdx.x; e < 32 * 64; e += blockDim.x) {
-        const int pl = e >> 6, cl = e & 63, p = p0 + pl, col = c0 + cl;
-        if (p >= a.p_hi || col >= N) continue;
-        float o1 = 0.0f, inv = 0.0f;
-        int16_t pr = 0;
-        stage_one(g, a, p, v, col, o1, inv, pr);
-        t_o1[cl][pl] = o1;
-        t_inv[cl][pl] = inv;
-        t_pr[cl][pl] = pr;
+    const int q0 = (a.q_lo & ~63) + STAGE_TILE * (int)blockIdx.z, v = blockIdx.y, c0 = STAGE_TILE * (int)blockIdx.x;
+    const int cl = NB * (threadIdx.x % LANES), r = threadIdx.x / LANES, col = c0 + cl;
+    if (threadIdx.x < STAGE_TILE) t_live[threadIdx.x] = 0;
+    bool live[NB] = {};
+    if (col < N) {
+#pragma unroll 4
+        for (int pl = r; pl < STAGE_TILE; pl += ROWS) {
+            const int q = q0 + pl;
+            int2 e = make_int2(-1, 0);   // {file plane, segment | killed << 8}; -1: a guard plane
+            if (q >= a.q_lo && q < a.q_hi) e = g.stage_plane[q];
+            float o1[NB] = {}, inv[NB] = {};
+            StageBin in[NB];
+            if (e.x >= 0) {
+                stage_load<OP, RB>(g, a, e.y & 0xff, (size_t)e.x, v, col, (e.y >> 8) != 0, in);
+#pragma unroll
+                for (int n = 0; n < NB; n++) {
+                    live[n] |= in[n].nrm != 0.0f;
+                    stage_one<OP>(g, a, in[n], o1[n], inv[n]);
+                }
+            } else {
+#pragma unroll
+                for (int n = 0; n < NB; n++) in[n].pr = 0;
+            }
+#pragma unroll
+            for (int n = 0; n < NB; n++) {
+                t_o1[cl + n][pl] = o1[n];
+                t_inv[cl + n][pl] = inv[n];
+                if (OP) t_pr[cl + n][pl] = in[n].pr;
+            }
+        }
     }
     __syncthreads();
+#pragma unroll
+    for (int n = 0; n < NB; n++)
+        if (live[n]) atomicOr(&t_live[cl + n], 1);
     const int pair = v % (V / 2), h = v / (V / 2);
-    for (int e = threadIdx.x; e < 32 * 64; e += blockDim.x) {
-        const int cl = e >> 5, pl = e & 31, p = p0 + pl, col = c0 + cl;
-        if (p >= a.p_hi || col >= N) continue;
-        const int th = a.plane_seg[p];
-        const size_t o = ((size_t)(pair * 2 + h) * N + col) * g.spp + g.seg_data[th] + (p - g.segment_offset[th]);
-        if (a.weighting < 3) {
-            a.data[o] = t_o1[cl][pl];
-        } else {
-            a.prompt[o] = t_pr[cl][pl];
-            a.add[o] = t_o1[cl][pl];
+    constexpr int QL = STAGE_TILE / 4, BR = 256 / QL;     // the write-out's groups of four planes, bins per pass
+    const int pq = 4 * (threadIdx.x % QL), q = q0 + pq;
+#pragma unroll
+    for (int j = 0; j < STAGE_TILE / BR; j++) {
+        const int b = threadIdx.x / QL + BR * j;
+        if (c0 + b >= N) continue;
+        const size_t o = ((size_t)(pair * 2 + h) * N + c0 + b) * g.spp + q;
+        float x[4], w[4];
+        int16_t p[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            x[k] = t_o1[b][pq + k];
+            w[k] = t_inv[b][pq + k];
+            p[k] = OP ? t_pr[b][pq + k] : (int16_t)0;
         }
-        a.invnorm[o] = t_inv[cl][pl];
+        float *const o1 = OP ? a.add : a.data;
+        if (a.wide && q >= a.q_lo && q + 4 <= a.q_hi) {
+            *reinterpret_cast<float4 *>(o1 + o) = make_float4(x[0], x[1], x[2], x[3]);
+            *reinterpret_cast<float4 *>(a.invnorm + o) = make_float4(w[0], w[1], w[2], w[3]);
+            if (OP) *reinterpret_cast<short4 *>(a.prompt + o) = make_short4(p[0], p[1], p[2], p[3]);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                if (q + k < a.q_lo || q + k >= a.q_hi) continue;
+                o1[o + k] = x[k];
+                a.invnorm[o + k] = w[k];
+                if (OP) a.prompt[o + k] = p[k];
+            }
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < STAGE_TILE && t_live[threadIdx.x]) {
+        int *m = &a.colmask[v * N + c0 + threadIdx.x];
+        if (*m == 0) atomicOr(m, 1);
     }
 }
 
@@ -1865,40 +2028,58 @@ hipError_t launch_end_iteration(const DevGeom &g, float *image, int z_min, int z
     return hipGetLastError();
 }
 
-// Segments [th0, th0 + nth) with internal planes [p_lo, p_hi): their gap masks first when the
+// Segments [th0, th0 + nth), which write the padded planes [q_lo, q_hi): their gap masks first when the
 // norm is rebinned, then their planes; finish derives the zero-column mask from the column
 // flags of every segment staged so far.
-static void stage_launch(const DevGeom &g, StageArgs a, int th0, int nth, int p_lo, int p_hi, bool finish,
+template <bool OP>
+static void stage_launch(const DevGeom &g, StageArgs a, int th0, int nth, int q_lo, int q_hi, bool finish,
                          hipStream_t s) {
-    a.p_lo = p_lo;
-    a.p_hi = p_hi;
-    if (a.norm_f && g.x_rebin * g.v_rebin > 1 && nth > 0)
-        hipLaunchKernelGGL(gapmask_kernel, dim3(256, nth), dim3(256), 0, s, g, a.norm_f, const_cast<uint8_t *>(a.gapmask), th0);
-    if (p_hi > p_lo)
-        hipLaunchKernelGGL(stage_kernel, dim3((p_hi - p_lo + 31) / 32, g.views, (g.N + 63) / 64), dim3(256), 0, s, g, a);
+    a.q_lo = q_lo;
+    a.q_hi = q_hi;
+    auto off = [](const void *p, uintptr_t n) { return reinterpret_cast<uintptr_t>(p) % n; };
+    // 16-byte loads and stores: file rows, columns and tiles are whole groups of four values (radial
+    // bins a multiple of four), so what remains is where the buffers begin
+    const bool files = !off(a.prompt_f, 8) && !off(a.delayed_f, 16) && !off(a.norm_f, 16) && !off(a.scatter_f, 16) &&
+                       !off(a.atten_f, 16) && !off(a.dataf_f, 16) && g.def_elements % 4 == 0;
+    a.wide = !off(a.prompt, 8) && !off(a.add, 16) && !off(a.invnorm, 16) && !off(a.data, 16);
+    const bool one = g.x_rebin == 1 && g.v_rebin == 1, two = g.x_rebin == 2 && g.v_rebin == 2;
+    if (a.norm_f && !one && nth > 0) {
+        const size_t fp = (size_t)g.def_angles * g.def_elements;
+        const size_t n = files ? fp / 4 : fp;
+        const dim3 grid((unsigned)((n + 255) / 256), nth);
+        uint8_t *gm = const_cast<uint8_t *>(a.gapmask);
+        if (files) hipLaunchKernelGGL(gapmask_kernel<true>, grid, dim3(256), 0, s, g, a.norm_f, gm, th0);
+        else hipLaunchKernelGGL(gapmask_kernel<false>, grid, dim3(256), 0, s, g, a.norm_f, gm, th0);
+    }
+    if (q_hi > q_lo) {
+        // the tiles of a view's rows next to each other: 3.7 ms against 4.0 with its planes next to each other
+        const dim3 grid((g.N + STAGE_TILE - 1) / STAGE_TILE, g.views, (q_hi - (q_lo & ~63) + STAGE_TILE - 1) / STAGE_TILE);
+        if (files && one) hipLaunchKernelGGL((stage_kernel<OP, 1>), grid, dim3(256), 0, s, g, a);
+        else if (files && two) hipLaunchKernelGGL((stage_kernel<OP, 2>), grid, dim3(256), 0, s, g, a);
+        else hipLaunchKernelGGL((stage_kernel<OP, 0>), grid, dim3(256), 0, s, g, a);
+    }
     if (finish) hipLaunchKernelGGL(nzmask_kernel, dim3(g.views / 2), dim3(256), 0, s, g, a.colmask, g.nzmask);
 }
 
 hipError_t launch_stage(const DevGeom &g, const int16_t *prompt_f, const float *delayed_f, const float *norm_f,
                         const float *scatter_f, const float *atten_f, int16_t *prompt, float *add, float *invnorm,
-                        uint8_t *gapmask, int *colmask, int th0, int nth, int p_lo, int p_hi, bool finish,
+                        uint8_t *gapmask, int *colmask, int th0, int nth, int q_lo, int q_hi, bool finish,
                         hipStream_t s) {
-    StageArgs a{prompt_f, delayed_f, norm_f, scatter_f, atten_f, prompt, add, invnorm, gapmask, colmask, g.plane_seg};
-    stage_launch(g, a, th0, nth, p_lo, p_hi, finish, s);
+    StageArgs a{prompt_f, delayed_f, norm_f, scatter_f, atten_f, prompt, add, invnorm, gapmask, colmask};
+    stage_launch<true>(g, a, th0, nth, q_lo, q_hi, finish, s);
     return hipGetLastError();
 }
 
 hipError_t launch_stage_w012(const DevGeom &g, int weighting, int precor, const int16_t *data_f16,
                              const float *data_ff, const float *delayed_f, const float *norm_f, const float *scatter_f,
                              const float *atten_f, float *data, float *invnorm, uint8_t *gapmask, int *colmask,
-                             int th0, int nth, int p_lo, int p_hi, bool finish, hipStream_t s) {
-    StageArgs a{data_f16, delayed_f, norm_f, scatter_f, atten_f, nullptr, nullptr, invnorm, gapmask, colmask,
-                g.plane_seg};
+                             int th0, int nth, int q_lo, int q_hi, bool finish, hipStream_t s) {
+    StageArgs a{data_f16, delayed_f, norm_f, scatter_f, atten_f, nullptr, nullptr, invnorm, gapmask, colmask};
     a.weighting = weighting;
     a.precor = precor;
     a.dataf_f = data_ff;
     a.data = data;
-    stage_launch(g, a, th0, nth, p_lo, p_hi, finish, s);
+    stage_launch<false>(g, a, th0, nth, q_lo, q_hi, finish, s);
     return hipGetLastError();
 }
 

@@ -197,6 +197,10 @@ class Osem3D(Layout):
     def paircol_zeros(self, dtype=torch.float32):
         return torch.zeros((self.views // 2, 2, self.N, self.spp), dtype=dtype, device=self.device)
 
+    def _paircol(self, dtype=torch.float32):
+        """A pair-column buffer that the staging writes whole, guard planes included."""
+        return torch.empty((self.views // 2, 2, self.N, self.spp), dtype=dtype, device=self.device)
+
     # ---- staging (PrepareOsem3dFiles S3:3876 + PrepareNormfac S3:3726) ----
     def stage(self, prompt_file, delayed_file, norm_file, scatter_file, atten_file):
         fb = self.file_bins
@@ -205,9 +209,9 @@ class Osem3D(Layout):
                 self._t(norm_file, torch.float32, fb, "norm_file", optional=True),
                 self._t(scatter_file, torch.float32, fb, "scatter_file", optional=True),
                 self._t(atten_file, torch.float32, fb, "atten_file", optional=True)]
-        prompt = self.paircol_zeros(torch.int16)
-        add = self.paircol_zeros()
-        invnorm = self.paircol_zeros()
+        prompt = self._paircol(torch.int16)
+        add = self._paircol()
+        invnorm = self._paircol()
         _lib.call("hrrt_stage_sinograms", self.ctx, *args, _p(prompt), _p(add), _p(invnorm), _stream())
         return prompt, add, invnorm
 
@@ -226,8 +230,8 @@ class Osem3D(Layout):
                 self._t(norm_file, torch.float32, fb, "norm_file", optional=True),
                 self._t(scatter_file, torch.float32, fb, "scatter_file", optional=True),
                 self._t(atten_file, torch.float32, fb, "atten_file", optional=True)]
-        data = self.paircol_zeros()
-        invnorm = self.paircol_zeros()
+        data = self._paircol()
+        invnorm = self._paircol()
         _lib.call("hrrt_stage_sinograms_w012", self.ctx, int(weighting), int(bool(precorrected)), *args, _p(data),
                   _p(invnorm), _stream())
         return data, invnorm
@@ -243,9 +247,9 @@ class Osem3D(Layout):
                 self._h(norm_file, torch.float32, fb, "norm_file", optional=True),
                 self._h(scatter_file, torch.float32, fb, "scatter_file", optional=True),
                 self._h(atten_file, torch.float32, fb, "atten_file", optional=True)]
-        prompt = self.paircol_zeros(torch.int16)
-        add = self.paircol_zeros()
-        invnorm = self.paircol_zeros()
+        prompt = self._paircol(torch.int16)
+        add = self._paircol()
+        invnorm = self._paircol()
         _lib.call("hrrt_stage_sinograms_host", self.ctx, *args, _p(prompt), _p(add), _p(invnorm), _stream())
         return prompt, add, invnorm
 
@@ -261,8 +265,8 @@ class Osem3D(Layout):
                 self._h(norm_file, torch.float32, fb, "norm_file", optional=True),
                 self._h(scatter_file, torch.float32, fb, "scatter_file", optional=True),
                 self._h(atten_file, torch.float32, fb, "atten_file", optional=True)]
-        data = self.paircol_zeros()
-        invnorm = self.paircol_zeros()
+        data = self._paircol()
+        invnorm = self._paircol()
         _lib.call("hrrt_stage_sinograms_w012_host", self.ctx, int(weighting), int(bool(precorrected)), *args,
                   _p(data), _p(invnorm), _stream())
         return data, invnorm

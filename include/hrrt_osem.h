@@ -120,7 +120,8 @@ const char *hrrt_last_error(void);
  *   d_invnorm float  N>0 ? (N*max(A,1) > eps2 ? 1/(N*max(A,1)) : 0) : N
  * Rebinning (-X 128: x_rebin = v_rebin = 2), norm harmonic rebin with gap
  * mask and npskip end-plane killing follow FIO:29-180.  Also computes the
- * norm zero-column mask (S3:864-909) kept in the context. */
+ * norm zero-column mask (S3:864-909) kept in the context.  Every element of the outputs is written,
+ * the guard planes as zeros. */
 int hrrt_stage_sinograms(hrrt_ctx *ctx, const int16_t *d_prompt_file, const float *d_delayed_file,
                          const float *d_norm_file, const float *d_scatter_file, const float *d_atten_file,
                          int16_t *d_prompt, float *d_add, float *d_invnorm, void *stream);
