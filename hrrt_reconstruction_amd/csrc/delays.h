@@ -65,6 +65,8 @@ struct hrrt_delays {
     int4 *d_lor = nullptr;
     int *d_lor_off = nullptr;
     int2 *d_seg = nullptr;
+    int2 *d_seg_col = nullptr;               // [128] by segment code {planes from 103 to its end, 8 * file offset}
+    int *d_scale = nullptr;                  // [nsino] fixed-point exponent of each bin
     float2 *d_z = nullptr;
     float *d_sings = nullptr;                // transposed singles [layer][head][x][ring], then column maxima
     float *d_cols = nullptr;                 // [nsino][nplanes rounded up to 64] columns
@@ -146,7 +148,7 @@ struct hrrt_delays {
 
 
 namespace hrrt_dl {
-// Device copies of the tables (d_lor, d_lor_off, d_seg, d_z, d_sings) on the current device,
+// Device copies of the tables (d_lor, d_lor_off, d_seg, d_seg_col, d_z, d_sings) on the current device,
 // made once; later calls must run with the same device current.
 int upload(hrrt_delays &c);
 }  // namespace hrrt_dl

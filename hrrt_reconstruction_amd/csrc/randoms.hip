@@ -7,11 +7,12 @@
 // Device side (per smoothing):
 //   sings_prepare_kernel    singles [layer][ring][head][x] -> [layer][head][x][ring], so that a
 //                           crystal's 104 rings are contiguous, and each column's largest magnitude
-//   delays_column_kernel    one workgroup per sinogram bin: every crystal pair of every LOR that
+//   bin_scale_kernel        per sinogram bin, its fixed-point unit from the largest possible term
+//   delays_column_kernel    per sinogram bin: every crystal pair of every LOR that
 //                           lands in the bin, accumulated into the bin's column of planes in
-//                           LDS (64-bit fixed point, ds_add_u64), then stored into the
-//                           plane-major output (span 9) or as a contiguous column (span 3)
-//   column_transpose_kernel span 3: [bin][plane] columns -> [plane][view][bin], 64 x 64 tiles
+//                           LDS (64-bit fixed point, ds_add_u64), then stored as a
+//                           contiguous column
+//   column_transpose_kernel [bin][plane] columns -> [plane][view][bin], 64 x 64 tiles
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -19,6 +20,7 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/hrrt_randoms.h"
@@ -32,187 +34,233 @@ namespace {
 struct Tables {    // device tables of one context
     const int4 *lor;      // [nlor] {A ring-column offset, B ring-column offset, bits(d), bits(z)}
     const int *lor_off;   // [nsino + 1] LORs of bin b: lor[lor_off[b] .. lor_off[b+1])
-    const int2 *seg;      // [128] {first | last << 16, file offset} by 2*(int)seg + (seg < 0) + 64
+    const int2 *seg;      // [128] {planes from 103 to the segment's end, 8 * file offset} by segment code
     const float2 *z;      // [104] {ring z (cm), ring z in planes + 0.5}
     int nsino, nplanes, window;
 };
 
 // ---------------------------------------------------------------- kernels
 
-// One workgroup: singles [layer][ring][head][x] -> [layer][head][x][ring] (a crystal's 104 rings
-// contiguous), then the largest |singles| of each such crystal column into out[NCRYS + column],
-// which sets the fixed-point scale of every sinogram bin.
-constexpr int PREP_THREADS = 1024;
+// Singles [layer][ring][head][x] -> [layer][head][x][ring] (a crystal's 104 rings contiguous),
+// then the largest |singles| of each such crystal column into out[NCRYS + column], which sets the
+// fixed-point scale of every sinogram bin.  A workgroup turns 8 columns in LDS (one workgroup for
+// all of them took 67 us, 144 take 3).  A NaN contributes nothing, as a term of value zero.
+constexpr int PREP_COLS = 8;
 constexpr int NCOLS = NCRYS / NY;   // 1152 crystal columns
+static_assert(NX % PREP_COLS == 0, "whole column groups per head");
 
-__global__ __launch_bounds__(PREP_THREADS) void sings_prepare_kernel(const float *__restrict__ in,
-                                                                     float *__restrict__ out) {
-    for (int i = threadIdx.x; i < NCRYS; i += PREP_THREADS) {
-        const int ring = i % NY, x = (i / NY) % NX, head = (i / (NY * NX)) % NHEADS, layer = i / (NY * NX * NHEADS);
-        out[i] = in[layer * XYH + ring * HX + head * NX + x];
+__global__ __launch_bounds__(256) void sings_prepare_kernel(const float *__restrict__ in, float *__restrict__ out) {
+    __shared__ float v[PREP_COLS][NY];
+    const int j0 = blockIdx.x * PREP_COLS;      // first column
+    const int x = j0 % NX, head = (j0 / NX) % NHEADS, layer = j0 / (NX * NHEADS);
+    const float *src = in + layer * XYH + head * NX + x;
+    for (int i = threadIdx.x; i < PREP_COLS * NY; i += 256) {
+        const float f = src[(i / PREP_COLS) * HX + i % PREP_COLS];
+        v[i % PREP_COLS][i / PREP_COLS] = f == f ? f : 0.0f;
     }
-    for (int j = threadIdx.x; j < NCOLS; j += PREP_THREADS) {
-        const int x = j % NX, head = (j / NX) % NHEADS, layer = j / (NX * NHEADS);
-        const float *src = in + layer * XYH + head * NX + x;
-        float m = 0.0f;
-        for (int ring = 0; ring < NY; ring++) m = fmaxf(m, fabsf(src[ring * HX]));
-        out[NCRYS + j] = m;
-    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < PREP_COLS * NY; i += 256) out[j0 * NY + i] = (&v[0][0])[i];
+    const int c = threadIdx.x >> 5, l = threadIdx.x & 31;
+    float m = 0.0f;
+    for (int ring = l; ring < NY; ring += 32) m = fmaxf(m, fabsf(v[c][ring]));
+    for (int o = 16; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 32));
+    if (l == 0) out[NCRYS + j0 + c] = m;
 }
 
 // Exponent k of a bin's fixed-point unit 2^-k.  A term s_A*tau*T*s_B of the bin is at most
 // about m = max over its LORs of colmax(A)*colmax(B)*tau*T < 2^E, and an element of the bin
 // sums at most nlor*1664 terms (104 A rings, each with at most 16 B rings on one segment and
 // plane), so terms below 2^(62-bits) with 2^bits >= nlor*1664 keep every sum inside int64.
+// bits is at least 11; where it is 11 and m lies just below 2^E, a term that rounds up to 2^E
+// would reach 2^51, which to_fixed does not take: the unit doubles there.
 __device__ inline int fixed_point_exponent(float m, int nlor) {
     int e = 0;
-    if (m > 0.0f && m <= 3.0e38f) frexpf(m, &e);
+    float f = 0.5f;
+    if (m > 0.0f && m <= 3.0e38f) f = frexpf(m, &e);
     const int bits = 32 - __clz(nlor * 1664);
-    return max(min(62 - bits - e, 127), -126);
+    return max(min(62 - bits - e - (bits < 12 && f > 0.9999f ? 1 : 0), 127), -126);
 }
 
-// Term -> int64 in units of 2^-k, rounded to nearest: x = v*2^k is exact (a power of two), and
-// so are its split into x = hi*2^32 + lo (hi integral) and lo's rounding below 2^32.
-// (x - hi*2^32 is exact: below 2^32 hi is 0, above it x is a multiple of 2^9 and the difference
-// below 2^32 has at most 23 bits, so one fused multiply-add gives it.)
+// Per bin its fixed-point exponent, and 256 more where a factor or a term may not be finite.
+__global__ __launch_bounds__(256) void bin_scale_kernel(Tables t, const float *__restrict__ sings, float tauftime,
+                                                        int *__restrict__ scale) {
+    const int bin = blockIdx.x * 256 + threadIdx.x;
+    if (bin >= t.nsino) return;
+    const int k0 = t.lor_off[bin], k1 = t.lor_off[bin + 1];
+    float m = 0.0f, mb = 0.0f;
+    bool finite = true;
+    for (int k = k0; k < k1; k++) {
+        const int2 L = *reinterpret_cast<const int2 *>(t.lor + k);
+        const float a = sings[NCRYS + L.x / NY], b = sings[NCRYS + L.y / NY];
+        m = fmaxf(m, a * b);
+        mb = fmaxf(mb, b);
+        finite &= a <= 3.0e38f;
+    }
+    m *= tauftime;
+    const int k = fixed_point_exponent(m, max(k1 - k0, 1));
+    finite &= m <= 3.0e38f && mb * ldexpf(1.0f, k) <= 3.0e38f;
+    scale[bin] = k + (finite ? 0 : 256);
+}
+
+// Term -> int64 in units of 2^-k, rounded to nearest.  FINITE (|x| < 2^51): x + 1.5*2^52 in
+// double rounds at the last bit of its mantissa, whose low bits are then the integer (3
+// instructions; splitting x into two 32-bit halves takes 6 and gives the same integer).  Otherwise
+// the halves, which saturate: x = hi*2^32 + lo (hi integral), x - hi*2^32 exact by one fused
+// multiply-add.
+template <bool FINITE>
 __device__ inline unsigned long long to_fixed(float x) {
+    if (FINITE) return (unsigned long long)__double_as_longlong((double)x + 0x1.8p52) - 0x4338000000000000ull;
     const float hi = floorf(x * 0x1p-32f);
     const float lo = __builtin_fmaf(hi, -0x1p32f, x);
     return ((unsigned long long)(long long)(int)hi << 32) + (unsigned long long)(unsigned)rintf(lo);
 }
 
-// One sinogram bin per workgroup of 512 threads (8 waves).  A wave covers 64 B rings (wave
-// parity: rings 0..63 or 64..103) for every fourth A ring (row = wave / 2).  The A singles
-// and ring z of the LOR sit one per lane in registers and are read with v_readlane for the
-// wave-uniform A ring, so the ring loop issues no memory instruction but the segment-table
-// read and the LDS add.  Each crystal pair adds s_A*tau*T*s_B to plane segplane(code, plane)
-// of the bin's column, with the reference's float operations (compute_delays
-// gen_delays_fromarchive.cpp:205-222):
+// |a - b| of unsigned numbers, in one instruction
+__device__ inline unsigned abs_diff(unsigned a, unsigned b) {
+    unsigned d;
+    asm("v_sad_u32 %0, %1, %2, 0" : "=v"(d) : "v"(a), "s"(b));
+    return d;
+}
+
+// COL_BINS consecutive sinogram bins per workgroup of 832 threads (13 full waves), one after the
+// other.  Each crystal pair (A ring ay, B ring by) of each LOR of the bin adds s_A*tau*T*s_B to
+// plane segplane(code, plane) of the bin's column, with the reference's float operations
+// (compute_delays gen_delays_fromarchive.cpp:205-222):
 //   plane = (int)(cay + z*dz),  seg = 0.5 + dz*d,  code = seg < 0 ? 1 - 2(int)seg : 2(int)seg
+// The kernel is bound by vector instructions, then by LDS, so the pairs are laid out for few of
+// both: a thread keeps A ring ay = tid mod 104 and takes the 13 B rings by = (ay + tid / 104 +
+// 8 i) mod 104.  Every lane has a pair (64 + 40 B rings over two waves left 19 % idle), dz of its
+// pairs stays in registers for all LORs and bins, s_A and cay too, and pairs outside the ring
+// window carry a dz whose segment does not exist instead of a test.  s_B comes from LDS at a
+// constant offset (each LOR's B column twice in a row, so the index needs no wrap).  Lanes of a
+// wave share by - ay, so their segment entries are broadcast and their adds go to every second
+// plane of a segment or two.
+// An entry is {103 - first plane + 1, 8 * file offset}: a segment's planes lie symmetrically
+// about 103, so |plane - 103| < that count says whether the pair has a plane.
 // The column accumulates in 64-bit fixed point (ds_add_u64; LDS float atomics run about
 // four times slower on gfx950), in units of 2^-k with k from the largest possible term:
 // the sum is order-independent, hence reproducible, and each element differs from the
 // exact sum of its float terms by at most n*2^-(k+1) for n terms before the final rounding
 // to float.
-constexpr int COL_THREADS = 512;
-// Columns up to this many planes (span 9: 2209) are stored straight into the plane-major
-// output; longer ones (span 3: 6367) go through bin-major columns and a tiled transpose,
-// since 96 workgroups' worth of them per XCD no longer gather in its L2.
-constexpr int DIRECT_PLANES = 4096;
-// The bin-major column path's LDS column (6400 planes: span 3 at maxrd up to 68 has 6367).
+// The next bin's LORs and singles are loaded while a bin is summed, and a cell is cleared by the
+// thread that stores it.  Columns go bin-major into scratch and through column_transpose_kernel:
+// stores straight into the plane-major output, one 4-byte request each, took 0.35 ms longer at
+// span 9 (2209 planes) and 1 ms at span 3 with maxrd 25.
+// 73728 bins of 6367 planes, 0.41 M LORs: 2.42 ms, the layout by B ring and two-halves conversion
+// 2.78 ms; a pair takes 17 vector instructions (31 before).
+constexpr int COL_ROWS = 8, COL_STEPS = NY / COL_ROWS, COL_THREADS = NY * COL_ROWS;
+static_assert(COL_STEPS * COL_ROWS == NY && COL_THREADS % 64 == 0, "rings split evenly");
+constexpr int COL_BINS = 8;     // bins per workgroup (the bin count is a multiple of 8)
+// steps 4..8 (B - A ring differences of 32 to 72, modulo 104) lie outside ring windows below 32
+constexpr int MID_LO = 4, MID_HI = 9, MID_WINDOW = 32;
+constexpr float NO_PAIR = 1e38f;
+constexpr int MID_PLANE = NY - 1;   // 103
+// Planes of the LDS column (span 3 at maxrd up to 68 has 6367).
 constexpr int COLUMN_PLANES = 6400;
 
-__device__ inline float lane_value(float v, int lane) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
-}
-
-template <bool DIRECT>
 __global__ __launch_bounds__(COL_THREADS) void delays_column_kernel(Tables t, const float *__restrict__ sings,
-                                                                    float tauftime, float *__restrict__ cols,
-                                                                    int cstride) {
-    // segment entry by e = 2*(int)seg + (seg < 0) + 64: {first plane | last plane << 16, 8 * file offset}
+                                                                    const int *__restrict__ scale, float tauftime,
+                                                                    float *__restrict__ cols, int cstride) {
     __shared__ int2 seg[128];
     // the bin's column of planes (a static array: its adds take their LDS base as an immediate)
-    __shared__ unsigned long long col[DIRECT ? DIRECT_PLANES : COLUMN_PLANES];
-    // XCD-aware: workgroups are dealt to the 8 XCDs in turn, so XCD x gets bins
-    // [x*nsino/8, (x+1)*nsino/8) in order and its L2 gathers whole lines of the plane-major output
-    const int per = gridDim.x >> 3;
-    const int bin = (blockIdx.x & 7) * per + (blockIdx.x >> 3), tid = threadIdx.x;
+    __shared__ unsigned long long col[COLUMN_PLANES];
+    __shared__ float sB[COL_ROWS][2 * NY], sA[COL_ROWS][NY];
+    __shared__ float2 sL[COL_ROWS];
+    // workgroups are dealt to the 8 XCDs in turn: XCD x gets bins [x*nsino/8, (x+1)*nsino/8)
+    const int per = t.nsino >> 3, wg = blockIdx.x >> 3, tid = threadIdx.x;
+    const int end = (blockIdx.x & 7) * per + min(per, (wg + 1) * COL_BINS);
+    const int first = (blockIdx.x & 7) * per + wg * COL_BINS;
     for (int i = tid; i < t.nplanes; i += COL_THREADS) col[i] = 0ull;
-    if (tid < 128) {
-        const int2 e = t.seg[tid];
-        seg[tid] = make_int2(e.x, 8 * e.y);
+    if (tid < 128) seg[tid] = t.seg[tid];
+    const int row = tid / NY, ay = tid % NY;
+    const float2 za = t.z[ay];
+    float dz[COL_STEPS];
+#pragma unroll
+    for (int i = 0; i < COL_STEPS; i++) {
+        int by = ay + row + COL_ROWS * i;
+        by -= by >= NY ? NY : 0;
+        dz[i] = abs(by - ay) <= t.window ? t.z[by].x - za.x : NO_PAIR;
     }
-    const int k0 = t.lor_off[bin], k1 = t.lor_off[bin + 1];
-    float mlor = 0.0f;
-    for (int k = k0; k < k1; k++) {
-        const int4 L = t.lor[k];
-        mlor = fmaxf(mlor, sings[NCRYS + L.x / NY] * sings[NCRYS + L.y / NY]);
-    }
-    const int kexp = fixed_point_exponent(mlor * tauftime, max(k1 - k0, 1));
-    const float up = ldexpf(1.0f, kexp);
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int row = wave >> 1;
-    const int by = (wave & 1) * 64 + lane;
-    const bool live = by < NY;
-    const int w = t.window;
-    const int ay_lo = by - w, ay_hi = by + w;   // A rings inside the ring window of B ring by
-    const float2 z0 = t.z[lane];                                          // A rings 0..63
-    const float2 z1 = lane < NY - 64 ? t.z[64 + lane] : make_float2(0.0f, 0.0f);   // A rings 64..103
-    const float zb = live ? t.z[by].x : 0.0f;
-    __syncthreads();
-    if (k0 == k1) goto store;
-    {
-        int4 L = t.lor[k0];
-        float sb = live ? sings[L.y + by] : 0.0f;
-        float sa0 = sings[L.x + lane];
-        float sa1 = lane < NY - 64 ? sings[L.x + 64 + lane] : 0.0f;
-        for (int k = k0; k < k1; k++) {
-            const float sd = __int_as_float(L.z), sz = __int_as_float(L.w);
-            // the term s_B*(s_A*tau*T) scaled by 2^k: scaling s_B first is exact and rounds the
-            // same product (a power of two commutes with rounding)
-            const float bu = sb * up, a0 = sa0 * tauftime, a1 = sa1 * tauftime;
-            if (k + 1 < k1) {     // next LOR's loads overlap this LOR's rings
-                L = t.lor[k + 1];
-                sb = live ? sings[L.y + by] : 0.0f;
-                sa0 = sings[L.x + lane];
-                sa1 = lane < NY - 64 ? sings[L.x + 64 + lane] : 0.0f;
+    const bool mid = t.window >= MID_WINDOW;
+    // this thread's LOR of the first eight of a bin, and its singles
+    int k0 = t.lor_off[first], k1 = t.lor_off[first + 1];
+    int4 L = make_int4(0, 0, 0, 0);
+    float a = 0.0f, b = 0.0f;
+    auto load_lor = [&](int k, int kend) { if (k < kend) L = t.lor[k]; };
+    auto load_sings = [&](int k, int kend) { if (k < kend) a = sings[L.x + ay], b = sings[L.y + ay]; };
+    load_lor(k0 + row, k1);
+    load_sings(k0 + row, k1);
+    for (int bin = first; bin < end; bin++) {
+        const int sc = scale[bin], kexp = sc >= 128 ? sc - 256 : sc;
+        const float up = ldexpf(1.0f, kexp);
+        const int n0 = k1, n1 = bin + 1 < end ? t.lor_off[bin + 2] : k1;    // the next bin's LORs
+        auto sum = [&](auto finite) __attribute__((always_inline)) {
+            for (int kb = k0; kb < k1; kb += COL_ROWS) {
+                if (kb > k0) {
+                    load_lor(kb + row, k1);
+                    load_sings(kb + row, k1);
+                    __syncthreads();
+                }
+                // the term s_B*(s_A*tau*T) scaled by 2^k: scaling s_B first is exact and rounds the
+                // same product (a power of two commutes with rounding)
+                sB[row][ay] = sB[row][NY + ay] = b * up;
+                sA[row][ay] = a * tauftime;
+                if (ay == 0) sL[row] = make_float2(__int_as_float(L.z), __int_as_float(L.w));
+                __syncthreads();
+                if (kb + COL_ROWS >= k1) {
+                    load_lor(n0 + row, n1);
+                    load_sings(n0 + row, n1);
+                }
+                const int n = min(COL_ROWS, k1 - kb);
+                for (int k = 0; k < n; k++) {
+                    const float sd = sL[k].x, sz = sL[k].y, awt = sA[k][ay];
+                    const float *bk = &sB[k][ay + row];
+                    auto steps = [&](auto lo, auto hi) __attribute__((always_inline)) {
+                        constexpr int I0 = decltype(lo)::value, NI = decltype(hi)::value - I0;
+                        bool ok[NI];
+                        int idx8[NI];
+                        unsigned long long q[NI];
+#pragma unroll
+                        for (int i = 0; i < NI; i++) {
+                            const float dzi = dz[I0 + i];
+                            const unsigned plane = (unsigned)(int)(za.y + sz * dzi);
+                            const float s = 0.5f + dzi * sd;
+                            const unsigned j = (unsigned)fminf(fabsf(s), 63.5f);
+                            // byte offset of entry 2 |(int)s| + (s < 0)
+                            const unsigned e8 = __builtin_amdgcn_alignbit(j, __float_as_uint(s), 28) & ~7u;
+                            const int2 ent = *reinterpret_cast<const int2 *>(reinterpret_cast<const char *>(seg) + e8);
+                            ok[i] = abs_diff(plane, MID_PLANE) < (unsigned)ent.x;
+                            idx8[i] = (int)(plane << 3) + ent.y;
+                            q[i] = to_fixed<decltype(finite)::value>(bk[COL_ROWS * (I0 + i)] * awt);
+                        }
+                        // whole groups before their adds, or each add would wait for its own chain
+#pragma unroll
+                        for (int i = 0; i < NI; i++) asm volatile("" : "+v"(idx8[i]), "+v"(q[i]));
+#pragma unroll
+                        for (int i = 0; i < NI; i++)
+                            if (ok[i]) atomicAdd(reinterpret_cast<unsigned long long *>(reinterpret_cast<char *>(col) + idx8[i]), q[i]);
+                    };
+                    steps(std::integral_constant<int, 0>(), std::integral_constant<int, MID_LO>());
+                    if (mid) steps(std::integral_constant<int, MID_LO>(), std::integral_constant<int, MID_HI>());
+                    steps(std::integral_constant<int, MID_HI>(), std::integral_constant<int, COL_STEPS>());
+                }
             }
-            // one crystal pair per lane for A ring ay (A singles*tau*T awt, ring z za, plane
-            // cay): the predicate, column index and fixed-point value of its add.  The
-            // reference skips silent A crystals; their terms are exact zeros here.
-            auto prepare = [&](int ay, float awt, float za, float cay, bool &ok, int &idx8, unsigned long long &q) {
-                const float dz = zb - za;
-                const int plane = (int)(cay + sz * dz);
-                const float s = 0.5f + dz * sd;
-                const int si = (int)s;
-                // e - 64 = 2*(int)seg + (seg < 0) names the code (2*si for seg >= 0, 1 - 2*si
-                // for seg < 0); e outside [0, 128) and impossible pairs map to no plane.  The
-                // byte offset 8 (e - 64), clamped to [-512, 504], reads seg[e].
-                const int e8 = min(max((si * 16) | (s < 0.0f ? 8 : 0), -512), 504);
-                const long long ent = *reinterpret_cast<const long long *>(reinterpret_cast<const char *>(seg) + 512 + e8);
-                const int first = (int)(ent & 0xffff), last = (int)((ent >> 16) & 0xffff);
-                ok = live & (ay >= ay_lo) & (ay <= ay_hi) & (plane >= first) & (plane <= last);
-                idx8 = (plane << 3) + (int)(ent >> 32);
-                q = to_fixed(bu * awt);
-            };
-            auto add = [&](int idx8, unsigned long long q) {
-                atomicAdd(reinterpret_cast<unsigned long long *>(reinterpret_cast<char *>(col) + idx8), q);
-            };
-            // A rings row, row+4, ..., two per step: 16 below ring 64 and 10 from it (row < 4)
-#pragma unroll 2
-            for (int i = 0; i < 16; i += 2) {
-                const int ay = row + 4 * i;
-                bool okA, okB;
-                int iA, iB;
-                unsigned long long qA, qB;
-                prepare(ay, lane_value(a0, ay), lane_value(z0.x, ay), lane_value(z0.y, ay), okA, iA, qA);
-                prepare(ay + 4, lane_value(a0, ay + 4), lane_value(z0.x, ay + 4), lane_value(z0.y, ay + 4), okB, iB, qB);
-                if (okA) add(iA, qA);
-                if (okB) add(iB, qB);
-            }
-#pragma unroll 1
-            for (int i = 0; i < 10; i += 2) {
-                const int ay = 64 + row + 4 * i, r = row + 4 * i;
-                bool okA, okB;
-                int iA, iB;
-                unsigned long long qA, qB;
-                prepare(ay, lane_value(a1, r), lane_value(z1.x, r), lane_value(z1.y, r), okA, iA, qA);
-                prepare(ay + 4, lane_value(a1, r + 4), lane_value(z1.x, r + 4), lane_value(z1.y, r + 4), okB, iB, qB);
-                if (okA) add(iA, qA);
-                if (okB) add(iB, qB);
-            }
+        };
+        if (k0 == k1) {
+            load_lor(n0 + row, n1);
+            load_sings(n0 + row, n1);
+        } else if (sc < 128) {
+            sum(std::true_type());
+        } else {
+            sum(std::false_type());
         }
-    }
-store:
-    __syncthreads();
-    const double down = ldexp(1.0, -kexp);
-    if (DIRECT) {   // plane-major output [nplanes][nsino]
-        for (int i = tid; i < t.nplanes; i += COL_THREADS) cols[(size_t)i * t.nsino + bin] = (float)((double)(long long)col[i] * down);
-    } else {        // bin-major columns [nsino][cstride], cstride a multiple of 64 planes
-        float *dst = cols + (size_t)bin * cstride;
-        for (int i = tid; i < t.nplanes; i += COL_THREADS) dst[i] = (float)((double)(long long)col[i] * down);
+        __syncthreads();
+        const double down = ldexp(1.0, -kexp);
+        for (int i = tid; i < t.nplanes; i += COL_THREADS) {
+            cols[(size_t)bin * cstride + i] = (float)((double)(long long)col[i] * down);
+            col[i] = 0ull;
+        }
+        k0 = n0, k1 = n1;
     }
 }
 
@@ -370,7 +418,10 @@ int group_lors(hrrt_delays &c) {
                 int4 e;
                 e.x = ((al * NHEADS + ahead) * NX + ax) * NY;
                 e.y = ((bl * NHEADS + bhead) * NX + bx) * NY;
-                memcpy(&e.z, &s.d, 4);
+                // a slope of zero (a record of zeros in a LUT file) becomes one that leaves 0.5 + dz*d at
+                // 0.5 for every ring difference but not for a pair outside the window
+                const float d = std::fabs(s.d) < 1e-30f ? std::copysign(1e-30f, s.d) : s.d;
+                memcpy(&e.z, &d, 4);
                 memcpy(&e.w, &s.z, 4);
                 lor[fill[s.nsino]++] = e;
                 c.pairs_full += ring_pairs;
@@ -416,17 +467,22 @@ int hrrt_dl::upload(hrrt_delays &c) {
         const int code = (ee >= 0 && ee % 2 == 0) ? ee : ((ee <= 1 && (ee & 1)) ? 2 - ee : -1);
         if (code >= 0 && code < c.nsegs) seg[e] = make_int2(c.segz0[code] | (c.segzmax[code] << 16), c.segoff[code]);
     }
+    std::vector<int2> seg_col(128, make_int2(0, 0));   // no plane
+    for (int code = 0; code < c.nsegs; code++) seg_col[code] = make_int2(MID_PLANE + 1 - c.segz0[code], 8 * c.segoff[code]);
     std::vector<float2> z(NY);
     for (int i = 0; i < NY; i++) z[i] = make_float2(c.zpos[i], c.zpos2[i]);
     DTRY(hipGetDevice(&c.device));
     DTRY(hipMalloc(&c.d_lor, sizeof(int4) * lor.size()));
     DTRY(hipMalloc(&c.d_lor_off, sizeof(int) * count.size()));
     DTRY(hipMalloc(&c.d_seg, sizeof(int2) * 128));
+    DTRY(hipMalloc(&c.d_seg_col, sizeof(int2) * 128));
+    DTRY(hipMalloc(&c.d_scale, sizeof(int) * c.nsino));
     DTRY(hipMalloc(&c.d_z, sizeof(float2) * NY));
     DTRY(hipMalloc(&c.d_sings, sizeof(float) * (NCRYS + NCOLS)));
     DTRY(hipMemcpy(c.d_lor, lor.data(), sizeof(int4) * lor.size(), hipMemcpyHostToDevice));
     DTRY(hipMemcpy(c.d_lor_off, count.data(), sizeof(int) * count.size(), hipMemcpyHostToDevice));
     DTRY(hipMemcpy(c.d_seg, seg.data(), sizeof(int2) * 128, hipMemcpyHostToDevice));
+    DTRY(hipMemcpy(c.d_seg_col, seg_col.data(), sizeof(int2) * 128, hipMemcpyHostToDevice));
     DTRY(hipMemcpy(c.d_z, z.data(), sizeof(float2) * NY, hipMemcpyHostToDevice));
     return HRRT_OK;
 }
@@ -458,7 +514,7 @@ extern "C" int hrrt_delays_create(const hrrt_delays_params *params, hrrt_delays 
 
 extern "C" void hrrt_delays_destroy(hrrt_delays *c) {
     if (!c) return;
-    for (void *p : {(void *)c->d_lor, (void *)c->d_lor_off, (void *)c->d_seg, (void *)c->d_z, (void *)c->d_sings,
+    for (void *p : {(void *)c->d_lor, (void *)c->d_lor_off, (void *)c->d_seg, (void *)c->d_seg_col, (void *)c->d_scale, (void *)c->d_z, (void *)c->d_sings,
                     (void *)c->d_cols, (void *)c->d_sol, (void *)c->d_lm_keys, (void *)c->d_lm_sort_tmp, (void *)c->d_lm_tiles,
                     (void *)c->d_lm_coin_seg, (void *)c->d_lm_coin_cnt, (void *)c->d_lm_coin_part, (void *)c->d_lm_chunks,
                     (void *)c->d_lm_stats})
@@ -559,17 +615,14 @@ extern "C" int hrrt_delays_smooth(hrrt_delays *c, const float *d_singles, float 
     if (dev != c->device) return hrrt_dl::fail(HRRT_ERR_ARG, "context tables live on another device");
     const float ftime = scan_duration > 0.0f ? scan_duration : 1.0f;
     const float tauftime = c->tau * ftime;
-    Tables t{c->d_lor, c->d_lor_off, c->d_seg, c->d_z, c->nsino, c->nplanes, c->maxrd + 5};
-    sings_prepare_kernel<<<1, PREP_THREADS, 0, s>>>(d_singles, c->d_sings);
+    Tables t{c->d_lor, c->d_lor_off, c->d_seg_col, c->d_z, c->nsino, c->nplanes, c->maxrd + 5};
+    sings_prepare_kernel<<<NCOLS / PREP_COLS, 256, 0, s>>>(d_singles, c->d_sings);
+    bin_scale_kernel<<<(c->nsino + 255) / 256, 256, 0, s>>>(t, c->d_sings, tauftime, c->d_scale);
     DTRY(hipGetLastError());
-    if (c->nplanes <= DIRECT_PLANES) {
-        delays_column_kernel<true><<<c->nsino, COL_THREADS, 0, s>>>(t, c->d_sings, tauftime, d_delays, 0);
-        DTRY(hipGetLastError());
-        return HRRT_OK;
-    }
+    const unsigned grid = 8 * ((c->nsino / 8 + COL_BINS - 1) / COL_BINS);
     const int cstride = (c->nplanes + 63) & ~63;
     if (!c->d_cols) DTRY(hipMalloc(&c->d_cols, sizeof(float) * (size_t)c->nsino * cstride));
-    delays_column_kernel<false><<<c->nsino, COL_THREADS, 0, s>>>(t, c->d_sings, tauftime, c->d_cols, cstride);
+    delays_column_kernel<<<grid, COL_THREADS, 0, s>>>(t, c->d_sings, c->d_scale, tauftime, c->d_cols, cstride);
     DTRY(hipGetLastError());
     column_transpose_kernel<<<dim3((c->nplanes + 64 * TT - 1) / (64 * TT), (c->nsino + 63) / 64), 256, 0, s>>>(c->d_cols, d_delays,
                                                                                                c->nsino, c->nplanes, cstride);
