@@ -72,7 +72,7 @@ struct hrrt_delays {
     float *d_cols = nullptr;                 // [nsino][nplanes rounded up to 64] columns
     // list-mode histogramming: the LUT by (module pair, A crystal, B crystal) on the device,
     // and its scratch (uploaded / allocated on first use)
-    int4 *d_sol = nullptr;                   // [21][144][144] {nsino, bits(d), bits(z), 0}
+    int3 *d_sol = nullptr;                   // [21][144][144] {nsino, bits(d), bits(z)}
     unsigned *d_lm_keys = nullptr;           // [2][lm_key_cap] key slots of the events (2*bin + delayed), then sorted
     long long lm_key_cap = 0;
     void *d_lm_sort_tmp = nullptr;           // radix sort scratch

@@ -91,7 +91,7 @@ struct LmArgs {
     const unsigned *w;
     long long nwords;
     int mode, start_ms, end_ms, ignore_border, doi;
-    const int4 *sol;        // [21][144][144] {nsino, bits(d), bits(z), 0}
+    const int3 *sol;        // [21][144][144] {nsino, bits(d), bits(z)}
     const float2 *z;        // [104] {ring z, ring z in planes + 0.5}
     const int2 *seg;        // [128] by 2*(int)seg + (seg < 0) + 64: {first | last << 16, offset}
     int nsino;
@@ -153,25 +153,27 @@ __device__ unsigned chunk_mask_word(const unsigned *__restrict__ w, long long cs
     return mine;
 }
 
-// The walk through one chunk from relative position `entry` (0 or 1): the relative positions
-// of the out-of-sync words it steps on (sw, may be null) and the parity it leaves with.
-__device__ int chunk_walk(const unsigned *mask, int entry, unsigned short *sw, int &nsw) {
+// The walk through one chunk from relative position `entry` (0 or 1), by one wave: lane l holds mask
+// word l (chunk_mask_word).  The relative positions of the out-of-sync words it steps on go to sw
+// (may be null), their number to nsw; returns the parity it leaves with.  All of it is scalar: a
+// ballot says which mask words hold any, so a chunk without them costs a few instructions (one
+// lane searching the 32 words of its parity in LDS took 40 us of a 40 M word stream's 80).
+__device__ int chunk_walk(unsigned mask, int entry, unsigned short *sw, int &nsw, int lane) {
+    const unsigned long long some = __ballot(mask != 0);
     int p = entry;
     nsw = 0;
     while (p < CHUNK) {
         const int par = p & 1, k = p >> 1;
-        int f = -1;
-        for (int wi = k >> 5; wi < 32; wi++) {
-            unsigned m = mask[par * 32 + wi];
-            if (wi == (k >> 5)) m &= ~0u << (k & 31);
-            if (m) {
-                f = (wi << 5) + __ffs(m) - 1;
-                break;
-            }
+        int wi = k >> 5;
+        unsigned m = (unsigned)__builtin_amdgcn_readlane((int)mask, par * 32 + wi) & (~0u << (k & 31));
+        if (!m) {
+            const unsigned later = (unsigned)(some >> (32 * par)) & (unsigned)(~1ull << wi);
+            if (!later) break;
+            wi = __builtin_ctz(later);
+            m = (unsigned)__builtin_amdgcn_readlane((int)mask, par * 32 + wi);
         }
-        if (f < 0) break;
-        const int pos = 2 * f + par;
-        if (sw) sw[nsw] = (unsigned short)pos;
+        const int pos = 2 * ((wi << 5) + __builtin_ctz(m)) + par;
+        if (sw && lane == 0) sw[nsw] = (unsigned short)pos;
         nsw++;
         p = pos + 1;
     }
@@ -179,57 +181,46 @@ __device__ int chunk_walk(const unsigned *mask, int entry, unsigned short *sw, i
 }
 
 __global__ __launch_bounds__(WAVES * 64) void lm_summary_kernel(LmArgs a, long long nchunks) {
-    __shared__ unsigned masks[WAVES][64];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const long long c = (long long)blockIdx.x * WAVES + wv;
     if (c >= nchunks) return;
     const unsigned m = chunk_mask_word(a.w, c * CHUNK, a.nwords, a.w16, lane);
-    masks[wv][lane] = m;
     a.cmask[c * 64 + lane] = m;
-    __builtin_amdgcn_wave_barrier();
-    // the walks from entry 0 (lane 0) and entry 1 (lane 32) side by side
-    int e = 0;
-    if ((lane & 31) == 0) {
-        int n;
-        e = chunk_walk(masks[wv], lane >> 5, nullptr, n);
-    }
-    const int e1 = __shfl(e, 32);
-    if (lane == 0) a.chunks[c] = (unsigned)(e | (e1 << 1));
+    int n;
+    const int e0 = chunk_walk(m, 0, nullptr, n, lane), e1 = chunk_walk(m, 1, nullptr, n, lane);
+    if (lane == 0) a.chunks[c] = (unsigned)(e0 | (e1 << 1));
 }
 
-// one workgroup per packet: the chunk summaries staged in LDS, walked in order by one thread
-// (the walk enters the packet's first chunk at word 0)
-__global__ __launch_bounds__(256) void lm_resolve_kernel(unsigned *chunks, long long nchunks) {
-    __shared__ unsigned sum[CHUNKS_PER_PACKET];
-    const long long c0 = (long long)blockIdx.x * CHUNKS_PER_PACKET;
-    const int n = (int)(c0 + CHUNKS_PER_PACKET < nchunks ? CHUNKS_PER_PACKET : nchunks - c0);
-    for (int i = threadIdx.x; i < n; i += 256) sum[i] = chunks[c0 + i] & 3u;
+// One workgroup per packet (the walk enters the packet's first chunk at word 0).  A chunk maps its
+// entry parity to its exit parity: to a constant, to itself or to the other.  The entry of a chunk
+// follows from the last constant before it and the number of exchanges since, so ballots give it
+// for a wave of chunks at once, and the waves' own maps chain the 16 of them (a single thread
+// walking the 1024 summaries took 27 us).
+__global__ __launch_bounds__(CHUNKS_PER_PACKET) void lm_resolve_kernel(unsigned *chunks, long long nchunks) {
+    __shared__ unsigned wave_map[CHUNKS_PER_PACKET / 64];   // exit parity for entry 0 (bit 0) and 1 (bit 1)
+    const long long c = (long long)blockIdx.x * CHUNKS_PER_PACKET + threadIdx.x;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const unsigned v = c < nchunks ? chunks[c] & 3u : 2u;   // past the end: the identity
+    const unsigned long long constant = __ballot(v == 0u || v == 3u), value = __ballot(v & 1u), flip = __ballot(v == 1u);
+    // the parity entering position n of the wave for an entry parity of `in`
+    auto entering = [&](int n, unsigned in) {
+        const unsigned long long below = n < 64 ? (1ull << n) - 1 : ~0ull, cb = constant & below;
+        if (!cb) return (in ^ (unsigned)__popcll(flip & below)) & 1u;
+        const int j = 63 - __clzll((long long)cb);
+        return ((unsigned)(value >> j) ^ (unsigned)__popcll(flip & below & (~1ull << j))) & 1u;
+    };
+    if (lane == 0) wave_map[wv] = entering(64, 0) | (entering(64, 1) << 1);
     __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned e = 0;
-        for (int i = 0; i < n; i++) {
-            const unsigned v = sum[i];
-            sum[i] = v | (e << 2);
-            e = (v >> e) & 1u;
-        }
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < n; i += 256) chunks[c0 + i] = sum[i];
+    unsigned in = 0;
+    for (int w = 0; w < wv; w++) in = (wave_map[w] >> in) & 1u;
+    if (c < nchunks) chunks[c] = v | (entering(lane, in) << 2);
 }
 
-// Per wave: masks and the switch list of the walk through chunk c; returns the entry parity.
-__device__ int chunk_visit_setup(const LmArgs &a, long long c, unsigned *mask, unsigned short *sw, int &nsw,
-                                 int lane) {
-    mask[lane] = a.cmask[c * 64 + lane];
+// Per wave: the switch list of the walk through chunk c; returns the entry parity.
+__device__ int chunk_visit_setup(const LmArgs &a, long long c, unsigned short *sw, int &nsw, int lane) {
+    const int entry = __builtin_amdgcn_readfirstlane((int)((a.chunks[c] >> 2) & 1u));
+    chunk_walk(a.cmask[c * 64 + lane], entry, sw, nsw, lane);
     __builtin_amdgcn_wave_barrier();
-    const int entry = (int)((a.chunks[c] >> 2) & 1u);
-    if (lane == 0) {
-        int n;
-        chunk_walk(mask, entry, sw, n);
-        mask[64] = (unsigned)n;
-    }
-    __builtin_amdgcn_wave_barrier();
-    nsw = (int)mask[64];
     return entry;
 }
 
@@ -248,9 +239,8 @@ __device__ inline bool visited(int r, int entry, const unsigned short *sw, int n
 
 template <int PASS>
 __global__ __launch_bounds__(WAVES * 64) void lm_window_kernel(LmArgs a, long long nchunks) {
-    __shared__ unsigned masks[WAVES][65];
     __shared__ unsigned short sws[WAVES][CHUNK];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const long long c = (long long)blockIdx.x * WAVES + wv;
     if (c >= nchunks) return;
     // pass 1 looks for the end tag from the start tag on (the start tag itself may end the frame)
@@ -260,7 +250,7 @@ __global__ __launch_bounds__(WAVES * 64) void lm_window_kernel(LmArgs a, long lo
         from = (long long)a.st[ST_START];
     }
     int nsw;
-    const int entry = chunk_visit_setup(a, c, masks[wv], sws[wv], nsw, lane);
+    const int entry = chunk_visit_setup(a, c, sws[wv], nsw, lane);
     const long long cs = c * CHUNK, pend = packet_end(cs, a.nwords);
     const int bound = PASS == 0 ? a.start_ms : a.end_ms;
     for (int i = 0; i < CHUNK / 64; i++) {
@@ -278,7 +268,7 @@ __global__ __launch_bounds__(WAVES * 64) void lm_window_kernel(LmArgs a, long lo
 
 // rebin_event LM_Rebinner_mp.cpp:188-219 from the event's LUT entry e (gathered from a.sol) and
 // the ring and segment tables in LDS: sinogram address or -1
-__device__ inline long long rebin(int4 e, int ay, int by, const float2 *zs, const int2 *segs, int nsino) {
+__device__ inline long long rebin(int3 e, int ay, int by, const float2 *zs, const int2 *segs, int nsino) {
     if (e.x < 0) return -1;
     const float sd = __int_as_float(e.y), sz = __int_as_float(e.z);
     const float2 za = zs[ay];
@@ -298,14 +288,13 @@ __device__ inline void wave_flush(unsigned long long *dst, unsigned v, int lane)
 }
 
 __global__ __launch_bounds__(WAVES * 64) void lm_hist_kernel(LmArgs a, long long nchunks) {
-    __shared__ unsigned masks[WAVES][65];
     __shared__ unsigned short sws[WAVES][CHUNK];
     __shared__ float2 zs[NY];
     __shared__ int2 segs[128];
     for (int j = threadIdx.x; j < NY; j += blockDim.x) zs[j] = a.z[j];
     for (int j = threadIdx.x; j < 128; j += blockDim.x) segs[j] = a.seg[j];
     __syncthreads();
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const long long c = (long long)blockIdx.x * WAVES + wv;
     if (c >= nchunks) return;
     // a chunk holds at most CHUNK/2 events (the walk steps two words past an event)
@@ -328,7 +317,7 @@ __global__ __launch_bounds__(WAVES * 64) void lm_hist_kernel(LmArgs a, long long
 #pragma unroll
     for (int h = 0; h < NHEADS; h++) cc[h] = 0;
     int nsw;
-    const int entry = chunk_visit_setup(a, c, masks[wv], sws[wv], nsw, lane);
+    const int entry = chunk_visit_setup(a, c, sws[wv], nsw, lane);
     const int xhigh = a.ignore_border ? NX - 1 : NX;
     unsigned n_tags = 0, n_time = 0, n_events = 0, n_rej = 0, n_tx = 0, n_prompts = 0, n_randoms = 0;
     unsigned nk = 0;   // keys of the chunk so far (wave-uniform)
@@ -356,7 +345,7 @@ __global__ __launch_bounds__(WAVES * 64) void lm_hist_kernel(LmArgs a, long long
                      !(a.mode == 2 && v.type != 0);
         return v;
     };
-    auto step = [&](long long q, unsigned ew1, unsigned ew2, const Ev &v, int4 e) __attribute__((always_inline)) {
+    auto step = [&](long long q, unsigned ew1, unsigned ew2, const Ev &v, int3 e) __attribute__((always_inline)) {
         // tags (process_tagword histogram_mp.cpp:225-295)
         const bool is_tag = v.type == 2;
         const unsigned tag = (ew1 & 0xffffu) | ((ew2 & 0xffffu) << 16);
@@ -450,11 +439,11 @@ __global__ __launch_bounds__(WAVES * 64) void lm_hist_kernel(LmArgs a, long long
         for (int g = 0; g < G; g++) n1[g] = n2[g] = 0u, np[g] = -1, nl[g] = false;
         if (i0 + G < NIT) load_words(i0 + G, n1, n2, np, nl);
         Ev v[G];
-        int4 e[G];
+        int3 e[G];
 #pragma unroll
         for (int g = 0; g < G; g++) {
             v[g] = decode(w1[g], w2[g], lv[g]);
-            e[g] = make_int4(-1, 0, 0, 0);
+            e[g] = make_int3(-1, 0, 0);
             if (v[g].binnable)
                 e[g] = a.sol[((v[g].mpe * NXD) + v[g].ax + NX * v[g].doia) * NXD + v[g].bx + NX * v[g].doib];
         }
@@ -577,8 +566,7 @@ __global__ __launch_bounds__(TILE_THREADS) void lm_tile_kernel(const unsigned *_
 }
 
 // Coincidence maps, pass 1: per (chunk range, head) the head's entries of the range's chunks
-// counted in LDS, written as the range's partial counts.  Each wave takes one chunk at a time and
-// loads its first 256 entries together with the chunk's count.
+// counted in LDS, written as the range's partial counts.  Each wave takes one chunk at a time.
 __global__ __launch_bounds__(1024) void lm_coin_kernel(const unsigned short *__restrict__ cseg,
                                                        const unsigned *__restrict__ ccnt, long long nchunks,
                                                        unsigned *__restrict__ part) {
@@ -589,16 +577,28 @@ __global__ __launch_bounds__(1024) void lm_coin_kernel(const unsigned short *__r
     __syncthreads();
     const long long per = (nchunks + COIN_RANGES - 1) / COIN_RANGES;
     const long long c0 = r * per, c1 = min(nchunks, c0 + per);
-    for (long long c = c0 + wv; c < c1; c += nw) {
+    // a chunk's first COIN_FIRST * 64 entries (a head has 256 of a full chunk on average) are loaded
+    // with its count, one chunk ahead: the loads of one chunk at a time left the wave waiting
+    constexpr int COIN_FIRST = 6;
+    unsigned n = 0, nn = 0;
+    unsigned short v[COIN_FIRST], vn[COIN_FIRST];
+    auto load = [&](long long c) __attribute__((always_inline)) {
         const unsigned short *e = cseg + (c * NHEADS + h) * (CHUNK / 2);
-        const unsigned n = ccnt[c * NHEADS + h];
-        unsigned short v[4];
+        nn = ccnt[c * NHEADS + h];
 #pragma unroll
-        for (int k = 0; k < 4; k++) v[k] = e[k * 64 + lane];   // inside the chunk's 1024 slots
+        for (int k = 0; k < COIN_FIRST; k++) vn[k] = e[k * 64 + lane];   // inside the chunk's 1024 slots
+    };
+    if (c0 + wv < c1) load(c0 + wv);
+    for (long long c = c0 + wv; c < c1; c += nw) {
+        n = nn;
 #pragma unroll
-        for (int k = 0; k < 4; k++)
+        for (int k = 0; k < COIN_FIRST; k++) v[k] = vn[k];
+        if (c + nw < c1) load(c + nw);
+#pragma unroll
+        for (int k = 0; k < COIN_FIRST; k++)
             if ((unsigned)(k * 64 + lane) < n) atomicAdd(&cnt[v[k]], 1u);
-        for (unsigned j = 256 + lane; j < n; j += 64) atomicAdd(&cnt[e[j]], 1u);
+        const unsigned short *e = cseg + (c * NHEADS + h) * (CHUNK / 2);
+        for (unsigned j = COIN_FIRST * 64 + lane; j < n; j += 64) atomicAdd(&cnt[e[j]], 1u);
     }
     __syncthreads();
     unsigned *o = part + ((long long)r * NHEADS + h) * COIN_HEAD;
@@ -634,17 +634,10 @@ int ensure_lm(hrrt_delays &c, long long nchunks, bool coin) {
     DTRY(hipGetDevice(&dev));
     if (dev != c.device) return hrrt_dl::fail(HRRT_ERR_ARG, "context tables live on another device");
     if (!c.d_sol) {
-        std::vector<int4> sol(c.lut.size());
-        for (size_t i = 0; i < c.lut.size(); i++) {
-            int4 e;
-            e.x = c.lut[i].nsino;
-            memcpy(&e.y, &c.lut[i].d, 4);
-            memcpy(&e.z, &c.lut[i].z, 4);
-            e.w = 0;
-            sol[i] = e;
-        }
-        DTRY(hipMalloc(&c.d_sol, sizeof(int4) * sol.size()));
-        DTRY(hipMemcpy(c.d_sol, sol.data(), sizeof(int4) * sol.size(), hipMemcpyHostToDevice));
+        // 12-byte records as the host holds them: 5.2 MB gather better from a 4 MB L2 than padded ones
+        static_assert(sizeof(int3) == sizeof(Sol), "LUT record is three words");
+        DTRY(hipMalloc(&c.d_sol, sizeof(int3) * c.lut.size()));
+        DTRY(hipMemcpy(c.d_sol, c.lut.data(), sizeof(int3) * c.lut.size(), hipMemcpyHostToDevice));
     }
     if (!c.d_lm_stats) DTRY(hipMalloc(&c.d_lm_stats, sizeof(unsigned long long) * ST_WORDS));
     if (!c.d_lm_tiles) {
@@ -732,7 +725,7 @@ extern "C" int hrrt_lm_histogram(hrrt_delays *c, const uint32_t *d_words, long l
         const unsigned grid = (unsigned)((nchunks + WAVES - 1) / WAVES);
         const long long npackets = (nchunks + CHUNKS_PER_PACKET - 1) / CHUNKS_PER_PACKET;
         lm_summary_kernel<<<grid, WAVES * 64, 0, s>>>(a, nchunks);
-        lm_resolve_kernel<<<(unsigned)npackets, 256, 0, s>>>(a.chunks, nchunks);
+        lm_resolve_kernel<<<(unsigned)npackets, CHUNKS_PER_PACKET, 0, s>>>(a.chunks, nchunks);
         if (opt->start_ms > 0) lm_window_kernel<0><<<grid, WAVES * 64, 0, s>>>(a, nchunks);
         if (opt->end_ms > 0) lm_window_kernel<1><<<grid, WAVES * 64, 0, s>>>(a, nchunks);
         lm_hist_kernel<<<grid, WAVES * 64, 0, s>>>(a, nchunks);
