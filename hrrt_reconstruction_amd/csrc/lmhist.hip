@@ -128,28 +128,37 @@ __device__ inline unsigned spread16(unsigned x) {
 __device__ unsigned chunk_mask_word(const unsigned *__restrict__ w, long long cs, long long nwords, bool w16, int lane) {
     const long long pend = packet_end(cs, nwords);
     const int par = lane >> 5, mi = lane & 3, kk = (lane & 31) >> 2;
-    unsigned mine = 0;
+    constexpr int BLOCKS = CHUNK / 256;
+    uint4 v[BLOCKS];
+    if (w16 && cs + CHUNK <= nwords) {     // every load in flight before the first is used
 #pragma unroll
-    for (int k = 0; k < CHUNK / 256; k++) {
-        const long long q0 = cs + 256 * k + 4 * lane;
-        unsigned v[5];
-        if (w16 && q0 + 3 < nwords) {
-            const uint4 x = *reinterpret_cast<const uint4 *>(w + q0);
-            v[0] = x.x, v[1] = x.y, v[2] = x.z, v[3] = x.w;
-        } else {
+        for (int k = 0; k < BLOCKS; k++) v[k] = *reinterpret_cast<const uint4 *>(w + cs + 256 * k + 4 * lane);
+    } else {
 #pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = q0 + j < nwords ? w[q0 + j] : 0u;
+        for (int k = 0; k < BLOCKS; k++) {
+            const long long q = cs + 256 * k + 4 * lane;
+            v[k].x = q < nwords ? w[q] : 0u;
+            v[k].y = q + 1 < nwords ? w[q + 1] : 0u;
+            v[k].z = q + 2 < nwords ? w[q + 2] : 0u;
+            v[k].w = q + 3 < nwords ? w[q + 3] : 0u;
         }
-        v[4] = __shfl_down(v[0], 1);
-        if (lane == 63) v[4] = q0 + 4 < pend ? w[q0 + 4] : 0u;
+    }
+    const unsigned tail = cs + CHUNK < pend ? w[cs + CHUNK] : 0u;
+    const int last = (int)min(pend - cs, (long long)CHUNK + 1) - 1;    // positions below it have a successor
+    unsigned long long lo = 0, hi = 0;
+#pragma unroll
+    for (int k = 0; k < BLOCKS; k++) {
+        const unsigned block_next = k + 1 < BLOCKS ? (unsigned)__builtin_amdgcn_readfirstlane((int)v[(k + 1) % BLOCKS].x) : tail;
+        unsigned next = __shfl_down(v[k].x, 1);
+        if (lane == 63) next = block_next;
+        const unsigned u[5] = {v[k].x, v[k].y, v[k].z, v[k].w, next};
         unsigned long long b[4];
 #pragma unroll
-        for (int j = 0; j < 4; j++) b[j] = __ballot(q0 + j + 1 < pend && word_type(v[j], v[j + 1]) == 3);
+        for (int j = 0; j < 4; j++) b[j] = __ballot(256 * k + 4 * lane + j < last && word_type(u[j], u[j + 1]) == 3);
         // relative position 256 k + 4 l + j: parity j & 1, bit 2 (l mod 16) + (j >> 1) of mask word 4 k + l / 16
-        const unsigned long long lo = par ? b[1] : b[0], hi = par ? b[3] : b[2];
-        const unsigned word = spread16((unsigned)(lo >> (16 * mi))) | (spread16((unsigned)(hi >> (16 * mi))) << 1);
-        if (kk == k) mine = word;
+        if (kk == k) lo = par ? b[1] : b[0], hi = par ? b[3] : b[2];
     }
+    const unsigned mine = spread16((unsigned)(lo >> (16 * mi))) | (spread16((unsigned)(hi >> (16 * mi))) << 1);
     return mine;
 }
 
@@ -266,212 +275,236 @@ __global__ __launch_bounds__(WAVES * 64) void lm_window_kernel(LmArgs a, long lo
     }
 }
 
-// rebin_event LM_Rebinner_mp.cpp:188-219 from the event's LUT entry e (gathered from a.sol) and
-// the ring and segment tables in LDS: sinogram address or -1
-__device__ inline long long rebin(int3 e, int ay, int by, const float2 *zs, const int2 *segs, int nsino) {
-    if (e.x < 0) return -1;
-    const float sd = __int_as_float(e.y), sz = __int_as_float(e.z);
-    const float2 za = zs[ay];
-    const float dz = zs[by].x - za.x;
-    const int plane = (int)(za.y + sz * dz);
-    const float s = 0.5f + dz * sd;
-    const int si = (int)s;
-    const int2 ent = segs[64 + min(max(2 * si + (s < 0.0f ? 1 : 0), -64), 63)];
-    if (plane < (ent.x & 0xffff) || plane > (ent.x >> 16)) return -1;
-    return (long long)(plane + ent.y) * nsino + e.x;
+// Event fields (rebin_packet histogram_mp.cpp:1111-1227) of a word pair; a pair of zeros is out of
+// sync, neither event nor tag.
+struct Event {
+    int type, mpe, ax, ay, bx, by, doia, doib;
+    bool is_event, bad, tx, em, binnable;
+};
+__device__ inline Event decode(const LmArgs &a, unsigned ew1, unsigned ew2) {
+    Event v;
+    v.type = word_type(ew1, ew2);
+    v.is_event = v.type < 2;
+    v.mpe = (int)(((ew1 & 0x00070000u) >> 16) | ((ew2 & 0x00070000u) >> 13));
+    v.ax = (int)(ew1 & 0xff), v.ay = (int)((ew1 & 0xff00) >> 8);
+    v.bx = (int)(ew2 & 0xff), v.by = (int)((ew2 & 0xff00) >> 8);
+    v.doia = a.doi ? (int)((ew1 & 0x01C00000u) >> 22) : 1;
+    v.doib = a.doi ? (int)((ew2 & 0x01C00000u) >> 22) : 1;
+    v.bad = v.is_event & ((v.mpe < 1) | (v.mpe > NMP) | (max(v.ax, v.bx) >= NX) | (max(v.ay, v.by) >= NY));
+    const bool ok = v.is_event & !v.bad;
+    v.tx = ok & ((v.doia == 7) | (v.doib == 7));
+    v.em = ok & !v.tx & (max(v.doia, v.doib) <= 1);
+    const int xhigh = NX - 1;
+    v.binnable = v.em & !(a.ignore_border & ((v.ax * v.bx == 0) | (v.ax == xhigh) | (v.bx == xhigh))) &
+                 !((a.mode == 2) & (v.type != 0));
+    return v;
 }
 
-// sum of a lane counter over the wave, added once by lane 0
-__device__ inline void wave_flush(unsigned long long *dst, unsigned v, int lane) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    if (lane == 0 && v) atomicAdd(dst, (unsigned long long)v);
+__device__ inline unsigned lanes_below(unsigned long long mask, unsigned base) {
+    return __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, base));
 }
 
-__global__ __launch_bounds__(WAVES * 64) void lm_hist_kernel(LmArgs a, long long nchunks) {
+// p by a 32-bit byte offset: a uniform base and an offset register, no 64-bit address per lane
+template <typename T>
+__device__ inline T *at_byte(T *p, unsigned off) {
+    return (T *)((char *)p + off);
+}
+
+// two words at any word address
+struct __attribute__((packed, aligned(4))) WordPair {
+    unsigned x, y;
+};
+
+// One wave per chunk.  The walk visits one position of each aligned word pair (2k, 2k + 1): the
+// one of its parity, entry parity flipped by every out-of-sync word before 2k; an out-of-sync word
+// is visited but not decoded, and when it is the pair's even word the walk goes on to the odd one.
+// Each lane takes a pair per row of 64; rows go in groups of G.  What bounds the kernel is vector
+// instructions and the latency of its gathers, so every load is unconditional: the words of the next
+// group and the LUT records of this one are in flight together (a record of an undecoded pair is
+// record 0, module pair 0, which has no bin), a chunk that the walk passes in step inside the frame
+// needs no position tests, and what is counted is counted in scalar registers from ballots.
+template <bool COIN>
+__global__ __launch_bounds__(WAVES * 64, 6) void lm_hist_kernel(LmArgs a, long long nchunks) {
     __shared__ unsigned short sws[WAVES][CHUNK];
-    __shared__ float2 zs[NY];
+    __shared__ float2 zs[256];                  // by the ring byte
     __shared__ int2 segs[128];
-    for (int j = threadIdx.x; j < NY; j += blockDim.x) zs[j] = a.z[j];
-    for (int j = threadIdx.x; j < 128; j += blockDim.x) segs[j] = a.seg[j];
+    __shared__ unsigned heads[64];              // by module pair: A head's bit, B head's bit << 8
+    __shared__ unsigned counts[7];
+    const int tid = threadIdx.x;
+    for (int j = tid; j < 256; j += WAVES * 64) zs[j] = j < NY ? a.z[j] : make_float2(0.0f, 0.0f);
+    for (int j = tid; j < 128; j += WAVES * 64) segs[j] = a.seg[j];
+    if (tid < 64) heads[tid] = tid >= 1 && tid <= NMP ? (1u << ((MP_A >> (3 * tid)) & 7)) | (256u << ((MP_B >> (3 * tid)) & 7)) : 0u;
+    if (tid < 7) counts[tid] = 0;
     __syncthreads();
-    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const long long c = (long long)blockIdx.x * WAVES + wv;
-    if (c >= nchunks) return;
-    // a chunk holds at most CHUNK/2 events (the walk steps two words past an event)
-    unsigned *keys = a.keys + c * (CHUNK / 2);
-    auto no_keys_from = [&](unsigned j0) {
-        for (unsigned j = j0 + lane; j < CHUNK / 2; j += 64) keys[j] = NOKEY;
-    };
     // the frame: from its start tag (or word 0) through its end tag (or the last word)
     const unsigned long long s0 = a.st[ST_START], s1 = a.st[ST_END];
     const long long lo = a.start_ms > 0 ? (long long)s0 : 0;
     const long long hi = (a.end_ms > 0 && s1 != NONE) ? (long long)s1 + 1 : a.nwords;
     const long long cs = c * CHUNK, pend = packet_end(cs, a.nwords);
-    if ((a.start_ms > 0 && s0 == NONE) || cs + CHUNK <= lo || cs >= hi) {
-        no_keys_from(0);
-        if (a.cseg && lane < NHEADS) a.ccnt[c * NHEADS + lane] = 0;
-        return;
-    }
-    unsigned short *cseg = a.cseg + c * (NHEADS * (CHUNK / 2));
-    unsigned cc[NHEADS];   // entries per head so far (wave-uniform)
+    // a chunk holds at most CHUNK/2 events (the walk steps two words past an event)
+    unsigned *keys = a.keys + c * (CHUNK / 2);
+    unsigned n_tags = 0, n_time = 0, n_events = 0, n_rej = 0, n_tx = 0, n_prompts = 0, n_randoms = 0;
+    unsigned nk = 0;   // keys of the chunk so far
+    unsigned cc[NHEADS];   // crystal entries per head so far
 #pragma unroll
     for (int h = 0; h < NHEADS; h++) cc[h] = 0;
-    int nsw;
-    const int entry = chunk_visit_setup(a, c, sws[wv], nsw, lane);
-    const int xhigh = a.ignore_border ? NX - 1 : NX;
-    unsigned n_tags = 0, n_time = 0, n_events = 0, n_rej = 0, n_tx = 0, n_prompts = 0, n_randoms = 0;
-    unsigned nk = 0;   // keys of the chunk so far (wave-uniform)
     unsigned long long last_time = 0;
-
-    // event fields (rebin_packet histogram_mp.cpp:1111-1227)
-    struct Ev {
-        int type, mpe, ax, ay, bx, by, doia, doib;
-        bool is_event, bad, tx, em, binnable;
-    };
-    auto decode = [&](unsigned ew1, unsigned ew2, bool live) __attribute__((always_inline)) {
-        Ev v;
-        v.type = live ? word_type(ew1, ew2) : 3;
-        v.is_event = v.type < 2;
-        v.mpe = (int)(((ew1 & 0x00070000u) >> 16) | ((ew2 & 0x00070000u) >> 13));
-        v.ax = (int)(ew1 & 0xff), v.ay = (int)((ew1 & 0xff00) >> 8);
-        v.bx = (int)(ew2 & 0xff), v.by = (int)((ew2 & 0xff00) >> 8);
-        v.doia = a.doi ? (int)((ew1 & 0x01C00000u) >> 22) : 1;
-        v.doib = a.doi ? (int)((ew2 & 0x01C00000u) >> 22) : 1;
-        v.bad = v.is_event && (v.mpe < 1 || v.mpe > NMP || v.ax >= NX || v.ay >= NY || v.bx >= NX || v.by >= NY);
-        const bool ok = v.is_event && !v.bad;
-        v.tx = ok && (v.doia == 7 || v.doib == 7);
-        v.em = ok && !v.tx && v.doia <= 1 && v.doib <= 1;
-        v.binnable = v.em && !(a.ignore_border && (v.ax * v.bx == 0 || v.ax == xhigh || v.bx == xhigh)) &&
-                     !(a.mode == 2 && v.type != 0);
-        return v;
-    };
-    auto step = [&](long long q, unsigned ew1, unsigned ew2, const Ev &v, int3 e) __attribute__((always_inline)) {
-        // tags (process_tagword histogram_mp.cpp:225-295)
-        const bool is_tag = v.type == 2;
-        const unsigned tag = (ew1 & 0xffffu) | ((ew2 & 0xffffu) << 16);
-        const bool time_tag = is_tag && (tag & 0xE0000000u) == 0x80000000u;
-        n_tags += is_tag;
-        n_time += time_tag;
-        if (time_tag) last_time = ((unsigned long long)q << 30) | (tag & 0x3fffffffu);   // q grows along the lane
-        if (is_tag && (tag & 0xE0000000u) == 0xA0000000u) {
-            const int block = (int)((tag & 0x1ff80000u) >> 19);
-            const unsigned val = tag & 0x0007ffffu;
-            if (block < NBLOCKS) {
-                atomicAdd(&a.st[ST_BLOCKS + block], (unsigned long long)val);
-                atomicAdd(&a.st[ST_BLOCKS + NBLOCKS + block], 1ull);
-                atomicMax(&a.st[ST_BLOCKS + 2 * NBLOCKS + block], ((unsigned long long)q << 19) | val);
+    if (c < nchunks && cs + 1 < a.nwords && !(a.start_ms > 0 && s0 == NONE) && cs + CHUNK > lo && cs < hi) {
+        unsigned short *cseg = COIN ? a.cseg + c * (NHEADS * (CHUNK / 2)) : nullptr;
+        const unsigned short *sw = sws[wv];
+        int nsw;
+        const int entry = chunk_visit_setup(a, c, sws[wv], nsw, lane);
+        const bool in_step = entry == 0 && nsw == 0 && cs + CHUNK <= a.nwords && cs >= lo && cs + CHUNK <= hi;
+        constexpr int G = 4, ROWS = CHUNK / 128;
+        static_assert(ROWS % G == 0, "whole groups");
+        unsigned x[G], y[G], xn[G], yn[G];
+        const int last = (int)min(a.nwords - 2 - cs, (long long)CHUNK - 2);   // the chunk's last word pair in the stream
+        auto load_words = [&](int r0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                const WordPair v = *reinterpret_cast<const WordPair *>(a.w + cs + min(128 * (r0 + g) + 2 * lane, last));
+                xn[g] = v.x, yn[g] = v.y;
+            }
+        };
+        load_words(0);
+        for (int r0 = 0; r0 < ROWS; r0 += G) {
+            int odd[G];      // the position taken is 2k + odd
+            int3 e[G];
+#pragma unroll
+            for (int g = 0; g < G; g++) x[g] = xn[g], y[g] = yn[g], odd[g] = 0;
+            // x, y become the pair of words at the position visited, zeros where there is none
+            if (!in_step) {
+                const long long qa = cs + 128 * (r0 + G);
+                const unsigned after = qa < a.nwords ? a.w[qa] : 0u;    // the word after the group
+#pragma unroll
+                for (int g = 0; g < G; g++) {       // words past the stream's end are zeros
+                    const int r = 128 * (r0 + g) + 2 * lane;
+                    x[g] = r <= last ? x[g] : (r == last + 1 ? y[g] : 0u);
+                    y[g] = r <= last ? y[g] : 0u;
+                }
+#pragma unroll
+                for (int g = 0; g < G; g++) {
+                    const int p0 = 2 * ((r0 + g) * 64 + lane);
+                    int n = 0, m = nsw;   // out-of-sync words visited before p0
+                    while (n < m) {
+                        const int mid = (n + m) >> 1;
+                        if (sw[mid] < p0) n = mid + 1;
+                        else m = mid;
+                    }
+                    const int par = (entry + n) & 1;
+                    int p = p0 + par;
+                    if (n < nsw && sw[n] == p) p = (par == 0 && !(n + 1 < nsw && sw[n + 1] == p0 + 1)) ? p0 + 1 : -1;
+                    const long long q = cs + p;
+                    const bool live = p >= 0 && q + 1 < pend && q >= lo && q < hi;
+                    unsigned next = __shfl_down(x[g], 1);
+                    const unsigned row_next = g + 1 < G ? (unsigned)__builtin_amdgcn_readfirstlane((int)x[(g + 1) % G]) : after;
+                    if (lane == 63) next = row_next;
+                    odd[g] = p & 1;
+                    const unsigned w1 = odd[g] ? y[g] : x[g], w2 = odd[g] ? next : y[g];
+                    x[g] = live ? w1 : 0u, y[g] = live ? w2 : 0u;
+                }
+            }
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                const Event v = decode(a, x[g], y[g]);
+                const unsigned i = (unsigned)(((v.mpe * NXD) + v.ax + NX * v.doia) * NXD + v.bx + NX * v.doib);
+                e[g] = *at_byte(a.sol, v.binnable ? i * 12u : 0u);
+            }
+            // the fields are decoded again below: held across the gathers they would cost the occupancy
+#pragma unroll
+            for (int g = 0; g < G; g++) asm volatile("" : "+v"(x[g]), "+v"(y[g]));
+            load_words(min(r0 + G, ROWS - G));      // always a group, or the gathers would wait for it
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                const Event v = decode(a, x[g], y[g]);
+                // tags (process_tagword histogram_mp.cpp:225-295)
+                const bool is_tag = v.type == 2;
+                const unsigned long long tags = __ballot(is_tag);
+                if (tags) {
+                    const long long q = cs + 2 * ((r0 + g) * 64 + lane) + odd[g];
+                    const unsigned tag = (x[g] & 0xffffu) | ((y[g] & 0xffffu) << 16);
+                    const bool time_tag = is_tag && (tag & 0xE0000000u) == 0x80000000u;
+                    n_tags += (unsigned)__popcll(tags);
+                    n_time += (unsigned)__popcll(__ballot(time_tag));
+                    if (time_tag) last_time = ((unsigned long long)q << 30) | (tag & 0x3fffffffu);   // q grows along the lane
+                    if (is_tag && (tag & 0xE0000000u) == 0xA0000000u) {
+                        const int block = (int)((tag & 0x1ff80000u) >> 19);
+                        const unsigned val = tag & 0x0007ffffu;
+                        if (block < NBLOCKS) {
+                            atomicAdd(&a.st[ST_BLOCKS + block], (unsigned long long)val);
+                            atomicAdd(&a.st[ST_BLOCKS + NBLOCKS + block], 1ull);
+                            atomicMax(&a.st[ST_BLOCKS + 2 * NBLOCKS + block], ((unsigned long long)q << 19) | val);
+                        }
+                    }
+                }
+                n_events += (unsigned)__popcll(__ballot(v.is_event));
+                n_rej += (unsigned)__popcll(__ballot(v.bad));
+                n_tx += (unsigned)__popcll(__ballot(v.tx));
+                // rebin_event LM_Rebinner_mp.cpp:188-219
+                const float sd = __int_as_float(e[g].y), sz = __int_as_float(e[g].z);
+                const float2 za = zs[v.ay];
+                const float dz = zs[v.by].x - za.x;
+                const int plane = (int)(za.y + sz * dz);
+                const float sg = 0.5f + dz * sd;
+                const int si = (int)sg;
+                const int2 ent = segs[64 + min(max(2 * si + (sg < 0.0f ? 1 : 0), -64), 63)];
+                const bool has = v.binnable & (e[g].x >= 0) & (plane >= (ent.x & 0xffff)) & (plane <= (ent.x >> 16));
+                // trues mode counts prompt - delayed, mode 1 the two apart, mode 2 prompts only (the
+                // delayed events have no bin there): every mode keeps the delayed flag in bit 0
+                const unsigned key = 2u * ((unsigned)(plane + ent.y) * (unsigned)a.nsino + (unsigned)e[g].x) + (unsigned)v.type;
+                const unsigned long long bal = __ballot(has), del = __ballot(has & (v.type != 0));
+                n_randoms += (unsigned)__popcll(del);
+                n_prompts += (unsigned)__popcll(bal & ~del);
+                if (has) *at_byte(keys, 4u * lanes_below(bal, nk)) = key;
+                nk += (unsigned)__popcll(bal);
+                // coincidence maps (histogram_mp.cpp:1218-1222, ring stride of histogram_mp_fromarchive.cpp:1092):
+                // the event's two crystals, each an entry [map][layer][ring][x] in its head's segment of the
+                // chunk (the two heads of a module pair differ)
+                if (COIN) {
+                    const bool counted = v.em & (v.type == 0 ? a.coin_p != nullptr : a.coin_d != nullptr);
+                    const unsigned hb = counted ? heads[v.mpe] : 0u;
+                    const int mo = v.type == 0 ? 0 : NDOIS * NY * NX;
+                    const unsigned ka = (unsigned)(mo + (v.doia * NY + v.ay) * NX + v.ax);
+                    const unsigned kb = (unsigned)(mo + (v.doib * NY + v.by) * NX + v.bx);
+#pragma unroll
+                    for (int h = 0; h < NHEADS; h++) {
+                        const bool on = (hb & (0x101u << h)) != 0;
+                        const unsigned long long bh = __ballot(on);
+                        if (on) *at_byte(cseg, 2u * lanes_below(bh, h * (CHUNK / 2) + cc[h])) = (unsigned short)((hb >> h) & 1 ? ka : kb);
+                        cc[h] += (unsigned)__popcll(bh);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);   // rows interleaved would hold their masks in spilled scalars
             }
         }
-        n_events += v.is_event;
-        n_rej += v.bad;
-        n_tx += v.tx;
-        const long long addr = v.binnable ? rebin(e, v.ay, v.by, zs, segs, a.nsino) : -1;
-        // coincidence maps (histogram_mp.cpp:1218-1222, ring stride of histogram_mp_fromarchive.cpp:1092):
-        // the event's two crystals, each an entry [map][layer][ring][x] in its head's segment of the
-        // chunk (the two heads of a module pair differ)
-        if (a.cseg) {
-            const bool cn = v.em && (v.type == 0 ? a.coin_p : a.coin_d) != nullptr;
-            const int ahead = cn ? (int)((MP_A >> (3 * v.mpe)) & 7) : -1;
-            const int bhead = cn ? (int)((MP_B >> (3 * v.mpe)) & 7) : -1;
-            const int mo = v.type == 0 ? 0 : NDOIS * NY * NX;
-            const unsigned short ka = (unsigned short)(mo + (v.doia * NY + v.ay) * NX + v.ax);
-            const unsigned short kb = (unsigned short)(mo + (v.doib * NY + v.by) * NX + v.bx);
+    }
+    if (c < nchunks) {
+        for (unsigned j = nk + lane; j < CHUNK / 2; j += 64) keys[j] = NOKEY;
+        if (COIN) {
+            unsigned n = 0;
 #pragma unroll
-            for (int h = 0; h < NHEADS; h++) {
-                const bool on = ahead == h || bhead == h;
-                const unsigned long long bh = __ballot(on);
-                if (on)
-                    cseg[h * (CHUNK / 2) + cc[h] +
-                         __builtin_amdgcn_mbcnt_hi((unsigned)(bh >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)bh, 0u))] =
-                        ahead == h ? ka : kb;
-                cc[h] += (unsigned)__popcll(bh);
+            for (int h = 0; h < NHEADS; h++) n = lane == h ? cc[h] : n;
+            if (lane < NHEADS) a.ccnt[c * NHEADS + lane] = n;
+        }
+        // the counters of the workgroup's waves, then one add per counter to the statistics
+        const unsigned mine = lane == 0 ? n_prompts : lane == 1 ? n_randoms : lane == 2 ? n_events : lane == 3 ? n_tags :
+                              lane == 4 ? n_time : lane == 5 ? n_rej : n_tx;
+        if (lane < 7 && mine) atomicAdd(&counts[lane], mine);
+        if (__ballot(last_time != 0)) {
+            for (int o = 32; o > 0; o >>= 1) {
+                const unsigned long long other = __shfl_xor(last_time, o);
+                last_time = other > last_time ? other : last_time;
             }
+            if (lane == 0) atomicMax(&a.st[ST_LAST_TIME], last_time);
         }
-        n_prompts += addr >= 0 && v.type == 0;
-        n_randoms += addr >= 0 && v.type == 1;
-        // trues mode counts prompt - delayed, mode 1 the two apart, mode 2 prompts only (the
-        // delayed events have no bin there): every mode keeps the delayed flag in bit 0
-        const bool has = addr >= 0;
-        const unsigned long long bal = __ballot(has);
-        if (has) {
-            const unsigned pre = __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0u));
-            keys[nk + pre] = (unsigned)(2 * addr + (v.type != 0 ? 1 : 0));
-        }
-        nk += (unsigned)__popcll(bal);
-    };
-    // The walk visits one position of each aligned word pair (2k, 2k + 1): the one of its
-    // parity, entry parity flipped by every out-of-sync word before 2k; an out-of-sync word is
-    // visited but not decoded, and when it is the pair's even word the walk goes on to the odd
-    // one.  Each lane takes a pair per row; rows of 64 pairs in groups of G: the next group's
-    // words are loaded and this group's LUT entries gathered before any of the group is processed.
-    constexpr int G = 4, NIT = CHUNK / 128;
-    static_assert(NIT % G == 0, "whole groups");
-    const unsigned short *sw = sws[wv];
-    auto load_words = [&](int i0, unsigned *x1, unsigned *x2, int *pp, bool *l) __attribute__((always_inline)) {
-#pragma unroll
-        for (int g = 0; g < G; g++) {
-            const int x = 2 * ((i0 + g) * 64 + lane);
-            int n = 0, m = nsw;   // out-of-sync words visited before x
-            while (n < m) {
-                const int mid = (n + m) >> 1;
-                if (sw[mid] < x) n = mid + 1;
-                else m = mid;
-            }
-            const int par = (entry + n) & 1;
-            int p = x + par;
-            if (n < nsw && sw[n] == p) p = (par == 0 && !(n + 1 < nsw && sw[n + 1] == x + 1)) ? x + 1 : -1;
-            const long long q = cs + p;
-            pp[g] = p;
-            l[g] = p >= 0 && q + 1 < pend && q >= lo && q < hi;
-            x1[g] = l[g] ? a.w[q] : 0u;
-            x2[g] = l[g] ? a.w[q + 1] : 0u;
-        }
-    };
-    unsigned w1[G], w2[G];
-    int pos[G];
-    bool lv[G];
-    load_words(0, w1, w2, pos, lv);
-    for (int i0 = 0; i0 < NIT; i0 += G) {
-        unsigned n1[G], n2[G];
-        int np[G];
-        bool nl[G];
-#pragma unroll
-        for (int g = 0; g < G; g++) n1[g] = n2[g] = 0u, np[g] = -1, nl[g] = false;
-        if (i0 + G < NIT) load_words(i0 + G, n1, n2, np, nl);
-        Ev v[G];
-        int3 e[G];
-#pragma unroll
-        for (int g = 0; g < G; g++) {
-            v[g] = decode(w1[g], w2[g], lv[g]);
-            e[g] = make_int3(-1, 0, 0);
-            if (v[g].binnable)
-                e[g] = a.sol[((v[g].mpe * NXD) + v[g].ax + NX * v[g].doia) * NXD + v[g].bx + NX * v[g].doib];
-        }
-#pragma unroll
-        for (int g = 0; g < G; g++) step(cs + pos[g], w1[g], w2[g], v[g], e[g]);
-#pragma unroll
-        for (int g = 0; g < G; g++) w1[g] = n1[g], w2[g] = n2[g], pos[g] = np[g], lv[g] = nl[g];
     }
-    no_keys_from(nk);
-    if (a.cseg) {
-        unsigned n = 0;
-#pragma unroll
-        for (int h = 0; h < NHEADS; h++) n = lane == h ? cc[h] : n;
-        if (lane < NHEADS) a.ccnt[c * NHEADS + lane] = n;
-    }
-    wave_flush(&a.st[ST_TAGS], n_tags, lane);
-    wave_flush(&a.st[ST_TIME_TAGS], n_time, lane);
-    wave_flush(&a.st[ST_EVENTS], n_events, lane);
-    wave_flush(&a.st[ST_REJECTED], n_rej, lane);
-    wave_flush(&a.st[ST_TX], n_tx, lane);
-    wave_flush(&a.st[ST_PROMPTS], n_prompts, lane);
-    wave_flush(&a.st[ST_RANDOMS], n_randoms, lane);
-    for (int o = 32; o > 0; o >>= 1) {
-        const unsigned long long other = __shfl_xor(last_time, o);
-        last_time = other > last_time ? other : last_time;
-    }
-    if (lane == 0 && last_time) atomicMax(&a.st[ST_LAST_TIME], last_time);
+    __syncthreads();
+    if (tid < 7 && counts[tid]) atomicAdd(&a.st[ST_LINE * tid], (unsigned long long)counts[tid]);
 }
+static_assert(ST_PROMPTS == 0 && ST_RANDOMS == ST_LINE && ST_EVENTS == 2 * ST_LINE && ST_TAGS == 3 * ST_LINE &&
+              ST_TIME_TAGS == 4 * ST_LINE && ST_REJECTED == 5 * ST_LINE && ST_TX == 6 * ST_LINE, "order of the counters");
 
 // tiles[t] = index of the first sorted key of tile t or later, for t in [0, ntiles] (NOKEY is
 // later than every tile): a binary search per tile.  The sort orders key bits TILE_BITS + 1 and
@@ -728,7 +761,8 @@ extern "C" int hrrt_lm_histogram(hrrt_delays *c, const uint32_t *d_words, long l
         lm_resolve_kernel<<<(unsigned)npackets, CHUNKS_PER_PACKET, 0, s>>>(a.chunks, nchunks);
         if (opt->start_ms > 0) lm_window_kernel<0><<<grid, WAVES * 64, 0, s>>>(a, nchunks);
         if (opt->end_ms > 0) lm_window_kernel<1><<<grid, WAVES * 64, 0, s>>>(a, nchunks);
-        lm_hist_kernel<<<grid, WAVES * 64, 0, s>>>(a, nchunks);
+        if (coin) lm_hist_kernel<true><<<grid, WAVES * 64, 0, s>>>(a, nchunks);
+        else lm_hist_kernel<false><<<grid, WAVES * 64, 0, s>>>(a, nchunks);
     }
     DTRY(hipGetLastError());
     // the key slots by tile: the tile bits (key bits 13 and up) sorted, through enough bits that
