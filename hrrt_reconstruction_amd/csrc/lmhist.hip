@@ -13,13 +13,13 @@
 //   lm_hist_kernel     every word pair the walk visits inside the frame: tags into the
 //                      statistics, events decoded and rebinned through the module-pair LUT with
 //                      the reference's float operations; each binned event written as a key
-//                      2*bin + delayed into its chunk's CHUNK/2 key slots (the unused slots hold
-//                      NOKEY), and each event's two crystals as 16-bit entries into the chunk's
-//                      per-head segments
-//   radix sort         the keys by 8192-bin tile (rocPRIM, key bits 14 and up; NOKEY sorts last)
-//   lm_tiles_kernel    the first key of every tile in the sorted keys
+//                      2*bin + delayed into its chunk's CHUNK/2 key slots, and each event's two
+//                      crystals as 16-bit entries into the chunk's per-head segments
+//   lm_count_kernel, lm_part_sums_kernel, lm_scatter_kernel  the keys into buckets of 2^20 bins
+//   lm_tile_count_kernel, lm_tile_scatter_kernel  the buckets' keys into their tiles of 8192 bins,
+//                      and the first key of every tile
 //   lm_tile_kernel     per tile: its keys counted in LDS, then the tile's int16 bins (wrapping)
-//                      and saturating uint8 delayed bins written in order, 16 per thread
+//                      and saturating uint8 delayed bins written in order
 //   lm_coin_kernel     per head and range of chunks: the head's crystal entries counted in LDS
 //   lm_coin_sum_kernel the ranges' counts summed into the coincidence maps
 // No global atomics touch a sinogram bin or a crystal counter: scattered device-scope atomics
@@ -33,8 +33,6 @@
 #include <cstring>
 #include <vector>
 
-#include <rocprim/device/device_radix_sort.hpp>
-
 #include "../../include/hrrt_lmhist.h"
 #include "delays.h"
 #include "kernels.h"
@@ -46,7 +44,10 @@ namespace {
 constexpr long long PACKET = HRRT_LM_PACKET_WORDS;
 constexpr int CHUNK = 2048;                          // words per chunk, one wave
 constexpr int TILE_BITS = 13, TILE = 1 << TILE_BITS;  // sinogram bins per histogram tile
-constexpr unsigned NOKEY = 0xffffffffu;               // an unused key slot
+constexpr int BUCKET_BITS = 20;                      // sinogram bins per bucket of the first partition
+constexpr int BUCKET_TILES = 1 << (BUCKET_BITS - TILE_BITS);
+constexpr int MAX_BUCKETS = 1 << (30 - BUCKET_BITS);  // the sinogram has at most 2^30 bins
+constexpr int MAX_PARTS = 512;                       // workgroups of the first partition
 constexpr int COIN_HEAD = 2 * NDOIS * NY * NX;        // coincidence counters of one head: [map][layer][ring][x]
 constexpr int COIN_RANGES = 32;                       // chunk ranges of the coincidence-map pass
 constexpr int CHUNKS_PER_PACKET = (int)(PACKET / CHUNK);
@@ -96,7 +97,8 @@ struct LmArgs {
     const int2 *seg;        // [128] by 2*(int)seg + (seg < 0) + 64: {first | last << 16, offset}
     int nsino;
     long long S;            // nplanes * nsino
-    unsigned *keys;         // [nchunks][CHUNK/2] binned events 2*bin + (delayed), then NOKEY
+    unsigned *keys;         // [nchunks][CHUNK/2] binned events 2*bin + (delayed)
+    unsigned *kcnt;         // [nchunks] keys of each chunk
     unsigned *coin_p, *coin_d;
     unsigned short *cseg;   // [nchunks][NHEADS][CHUNK/2] crystal entries (index in COIN_HEAD) by head
     unsigned *ccnt;         // [nchunks][NHEADS] entries per chunk and head
@@ -481,7 +483,7 @@ __global__ __launch_bounds__(WAVES * 64, 6) void lm_hist_kernel(LmArgs a, long l
         }
     }
     if (c < nchunks) {
-        for (unsigned j = nk + lane; j < CHUNK / 2; j += 64) keys[j] = NOKEY;
+        if (lane == 0) a.kcnt[c] = nk;
         if (COIN) {
             unsigned n = 0;
 #pragma unroll
@@ -506,37 +508,240 @@ __global__ __launch_bounds__(WAVES * 64, 6) void lm_hist_kernel(LmArgs a, long l
 static_assert(ST_PROMPTS == 0 && ST_RANDOMS == ST_LINE && ST_EVENTS == 2 * ST_LINE && ST_TAGS == 3 * ST_LINE &&
               ST_TIME_TAGS == 4 * ST_LINE && ST_REJECTED == 5 * ST_LINE && ST_TX == 6 * ST_LINE, "order of the counters");
 
-// tiles[t] = index of the first sorted key of tile t or later, for t in [0, ntiles] (NOKEY is
-// later than every tile): a binary search per tile.  The sort orders key bits TILE_BITS + 1 and
-// up, so key < t << (TILE_BITS + 1) is monotone along the sorted keys.
-__global__ void lm_tiles_kernel(const unsigned *__restrict__ keys, long long n, long long ntiles,
-                                unsigned *__restrict__ tiles) {
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t > ntiles) return;
-    const unsigned v = (unsigned)(t << (TILE_BITS + 1));
-    long long lo = 0, hi = n;
-    while (lo < hi) {
-        const long long mid = (lo + hi) >> 1;
-        if (keys[mid] < v) lo = mid + 1;
-        else hi = mid;
+// ---- the keys by tile.  The order within a tile does not matter (a tile counts its keys), so two
+// counting partitions do it: first into buckets of 2^BUCKET_BITS bins, by up to 512 workgroups with a
+// range of chunks each, then slices of the buckets into tiles.  Stores of single keys to their places
+// would bound both (each is a request of its own: 67 us for the first at 20 M keys, 44 this way), so a
+// batch of keys is put in order in LDS first and its runs are stored whole.
+constexpr int PART_THREADS = 1024;
+constexpr int CHUNK_KEYS = CHUNK / 2 / 64;   // key slots of a chunk per lane
+
+// the chunk's key slots, 16 bytes a lane; key u of the lane is valid below the returned count's position
+__device__ inline void load_chunk(const unsigned *__restrict__ keys, long long c, unsigned (&v)[CHUNK_KEYS]) {
+    const uint4 *src = reinterpret_cast<const uint4 *>(keys + c * (CHUNK / 2)) + (threadIdx.x & 63);
+#pragma unroll
+    for (int i = 0; i < CHUNK_KEYS / 4; i++) {
+        const uint4 x = src[64 * i];
+        v[4 * i] = x.x, v[4 * i + 1] = x.y, v[4 * i + 2] = x.z, v[4 * i + 3] = x.w;
     }
-    tiles[t] = (unsigned)lo;
+}
+__device__ inline unsigned chunk_slot(int u) { return 256 * (u >> 2) + 4 * (threadIdx.x & 63) + (u & 3); }
+
+// Exclusive sums of v[0 .. PART_THREADS) over the workgroup, one element per thread; total gets the sum.
+__device__ inline unsigned block_exclusive(unsigned v, unsigned *wave_sum, unsigned &total) {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    unsigned inc = v;
+    for (int o = 1; o < 64; o <<= 1) {
+        const unsigned up = __shfl_up(inc, o);
+        if (lane >= o) inc += up;
+    }
+    if (lane == 63) wave_sum[wv] = inc;
+    __syncthreads();
+    unsigned before = 0;
+    total = 0;
+    for (int w = 0; w < PART_THREADS / 64; w++) {
+        before += w < wv ? wave_sum[w] : 0u;
+        total += wave_sum[w];
+    }
+    return before + inc - v;
 }
 
-constexpr int TILE_THREADS = 512, TILE_PER_THREAD = TILE / TILE_THREADS;   // 16 bins per thread
-static_assert(TILE_PER_THREAD == 16, "the tile write-out packs 16 bins per thread");
+// Up to U keys per thread (those with ok) into their digits' places in out: next[d] is the index of the
+// next key of digit d, advanced by the workgroup's keys of it; reserve(n), called once by the thread of
+// each digit with the number of its keys, gives how many others have put there.  The keys go
+// through buf in the order of their digits.  Ends with a barrier.
+template <int U, typename Digit, typename Reserve>
+__device__ inline void partition_batch(const unsigned (&v)[U], const bool (&ok)[U], Digit digit, unsigned *next,
+                                       unsigned *cnt, unsigned *buf, unsigned *wave_sum, unsigned *__restrict__ out,
+                                       Reserve reserve) {
+    const int tid = threadIdx.x;
+    cnt[tid] = 0;
+    __syncthreads();
+    unsigned rank[U];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+        if (ok[u]) rank[u] = atomicAdd(&cnt[digit(v[u])], 1u);
+    __syncthreads();
+    unsigned total;
+    const unsigned n = cnt[tid], before = block_exclusive(n, wave_sum, total), others = reserve(n);
+    cnt[tid] = before;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < U; u++)
+        if (ok[u]) buf[cnt[digit(v[u])] + rank[u]] = v[u];
+    __syncthreads();
+    const unsigned place = next[tid];
+    next[tid] = place + n;
+    cnt[tid] = place + others - before;
+    __syncthreads();
+    for (unsigned i = tid; i < total; i += PART_THREADS) {
+        const unsigned k = buf[i];
+        out[cnt[digit(k)] + i] = k;
+    }
+    __syncthreads();
+}
+
+// counts[b * parts + part]: keys of bucket b in the part's chunks
+__global__ __launch_bounds__(PART_THREADS) void lm_count_kernel(const unsigned *__restrict__ keys,
+                                                                const unsigned *__restrict__ kcnt, long long nchunks,
+                                                                int nbuckets, unsigned *__restrict__ counts) {
+    __shared__ unsigned cnt[PART_THREADS];
+    cnt[threadIdx.x] = 0;
+    __syncthreads();
+    const long long per = (nchunks + gridDim.x - 1) / gridDim.x, c0 = blockIdx.x * per, c1 = min(nchunks, c0 + per);
+    for (long long c = c0 + (threadIdx.x >> 6); c < c1; c += PART_THREADS / 64) {
+        unsigned v[CHUNK_KEYS];
+        load_chunk(keys, c, v);
+        const unsigned n = kcnt[c];
+#pragma unroll
+        for (int u = 0; u < CHUNK_KEYS; u++)
+            if (chunk_slot(u) < n) atomicAdd(&cnt[v[u] >> (BUCKET_BITS + 1)], 1u);
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < nbuckets) counts[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = cnt[threadIdx.x];
+}
+static_assert(MAX_BUCKETS <= PART_THREADS && BUCKET_TILES <= PART_THREADS, "a thread per digit");
+
+// one wave per bucket: the parts' counts into their exclusive sums, the bucket's total, and its tiles'
+// counters cleared
+__global__ __launch_bounds__(64) void lm_part_sums_kernel(unsigned *__restrict__ counts, int parts,
+                                                          unsigned *__restrict__ totals, unsigned *__restrict__ tcount,
+                                                          unsigned *__restrict__ used) {
+    unsigned *row = counts + (size_t)blockIdx.x * parts;
+    const int lane = threadIdx.x;
+    for (int t = lane; t < BUCKET_TILES; t += 64) tcount[blockIdx.x * BUCKET_TILES + t] = used[blockIdx.x * BUCKET_TILES + t] = 0;
+    unsigned sum = 0;
+    for (int p0 = 0; p0 < parts; p0 += 64) {
+        const unsigned v = p0 + lane < parts ? row[p0 + lane] : 0u;
+        unsigned inc = v;
+        for (int o = 1; o < 64; o <<= 1) {
+            const unsigned up = __shfl_up(inc, o);
+            if (lane >= o) inc += up;
+        }
+        if (p0 + lane < parts) row[p0 + lane] = sum + inc - v;
+        sum += __shfl(inc, 63);
+    }
+    if (lane == 0) totals[blockIdx.x] = sum;
+}
+
+__global__ __launch_bounds__(PART_THREADS) void lm_scatter_kernel(const unsigned *__restrict__ keys,
+                                                                  const unsigned *__restrict__ kcnt, long long nchunks,
+                                                                  int nbuckets, const unsigned *__restrict__ counts,
+                                                                  const unsigned *__restrict__ totals,
+                                                                  unsigned *__restrict__ out) {
+    __shared__ unsigned next[PART_THREADS], cnt[PART_THREADS], wave_sum[PART_THREADS / 64], buf[CHUNK_KEYS * PART_THREADS];
+    const int b = threadIdx.x;
+    unsigned total;
+    const unsigned base = block_exclusive(b < nbuckets ? totals[b] : 0u, wave_sum, total);
+    next[b] = base + (b < nbuckets ? counts[(size_t)b * gridDim.x + blockIdx.x] : 0u);
+    const long long per = (nchunks + gridDim.x - 1) / gridDim.x, c0 = blockIdx.x * per, c1 = min(nchunks, c0 + per);
+    for (long long cb = c0; cb < c1; cb += PART_THREADS / 64) {      // a chunk per wave
+        const long long c = cb + (threadIdx.x >> 6);
+        unsigned v[CHUNK_KEYS];
+        bool ok[CHUNK_KEYS];
+        load_chunk(keys, min(c, c1 - 1), v);
+        const unsigned n = c < c1 ? kcnt[c] : 0u;
+#pragma unroll
+        for (int u = 0; u < CHUNK_KEYS; u++) ok[u] = chunk_slot(u) < n;
+        partition_batch(v, ok, [](unsigned k) { return k >> (BUCKET_BITS + 1); }, next, cnt, buf, wave_sum, out,
+                        [](unsigned) { return 0u; });
+    }
+}
+
+// A workgroup of the second partition takes a slice of up to SLICE keys of one bucket: a bucket has as
+// many slices as its keys need and at least one (planes at a segment's ends can hold ten times the mean:
+// with a workgroup per bucket the fullest one took 190 of 190 us).
+constexpr int SLICE_KEYS = 8, SLICE = SLICE_KEYS * PART_THREADS;
+struct Slice {
+    unsigned bucket, start, k0, k1;     // the bucket, its first key, the slice's keys
+    int first;                          // the bucket's first slice
+};
+__device__ inline bool find_slice(const unsigned *__restrict__ totals, int nbuckets, unsigned item, unsigned (*wave_sum)[PART_THREADS / 64],
+                                  Slice *found) {
+    const unsigned tid = threadIdx.x, n = (int)tid < nbuckets ? totals[tid] : 0u;
+    const unsigned slices = (int)tid < nbuckets ? max(1u, (n + SLICE - 1) / SLICE) : 0u;
+    unsigned keys, all;
+    const unsigned start = block_exclusive(n, wave_sum[0], keys), s0 = block_exclusive(slices, wave_sum[1], all);
+    if (item >= s0 && item < s0 + slices) {
+        const unsigned k0 = start + (item - s0) * SLICE;
+        *found = Slice{tid, start, k0, min(start + n, k0 + SLICE), item == s0};
+    }
+    __syncthreads();
+    return item < all;
+}
+__device__ inline unsigned tile_of(unsigned k) { return (k >> (TILE_BITS + 1)) & (BUCKET_TILES - 1); }
+__device__ inline void load_slice(const unsigned *__restrict__ keys, const Slice &sl, unsigned (&v)[SLICE_KEYS], bool (&ok)[SLICE_KEYS]) {
+#pragma unroll
+    for (int u = 0; u < SLICE_KEYS; u++) {
+        const unsigned i = sl.k0 + u * PART_THREADS + threadIdx.x;
+        ok[u] = i < sl.k1;
+        v[u] = ok[u] ? keys[i] : 0u;
+    }
+}
+
+// tcount[t]: keys of tile t, added up over the slices
+__global__ __launch_bounds__(PART_THREADS) void lm_tile_count_kernel(const unsigned *__restrict__ in,
+                                                                     const unsigned *__restrict__ totals, int nbuckets,
+                                                                     unsigned *__restrict__ tcount) {
+    __shared__ unsigned cnt[BUCKET_TILES], wave_sum[2][PART_THREADS / 64];
+    __shared__ Slice sl;
+    const int tid = threadIdx.x;
+    if (tid < BUCKET_TILES) cnt[tid] = 0;
+    if (!find_slice(totals, nbuckets, blockIdx.x, wave_sum, &sl)) return;
+    unsigned v[SLICE_KEYS];
+    bool ok[SLICE_KEYS];
+    load_slice(in, sl, v, ok);
+#pragma unroll
+    for (int u = 0; u < SLICE_KEYS; u++)
+        if (ok[u]) atomicAdd(&cnt[tile_of(v[u])], 1u);
+    __syncthreads();
+    if (tid < BUCKET_TILES && cnt[tid]) atomicAdd(&tcount[sl.bucket * BUCKET_TILES + tid], cnt[tid]);
+}
+
+// The slices' keys into their tiles, each slice behind what others have reserved of a tile (used[t]), and
+// tiles[t] = index of the first key of tile t (tiles[ntiles] = number of keys).
+__global__ __launch_bounds__(PART_THREADS) void lm_tile_scatter_kernel(const unsigned *__restrict__ in,
+                                                                       const unsigned *__restrict__ totals, int nbuckets,
+                                                                       const unsigned *__restrict__ tcount,
+                                                                       unsigned *__restrict__ used, long long ntiles,
+                                                                       unsigned *__restrict__ out,
+                                                                       unsigned *__restrict__ tiles) {
+    __shared__ unsigned next[PART_THREADS], cnt[PART_THREADS], wave_sum[2][PART_THREADS / 64], buf[SLICE];
+    __shared__ Slice sl;
+    const int tid = threadIdx.x;
+    if (!find_slice(totals, nbuckets, blockIdx.x, wave_sum, &sl)) return;
+    unsigned v[SLICE_KEYS], total;
+    bool ok[SLICE_KEYS];
+    load_slice(in, sl, v, ok);
+    const long long t = (long long)sl.bucket * BUCKET_TILES + tid;
+    const unsigned start = sl.start + block_exclusive(tid < BUCKET_TILES ? tcount[t] : 0u, wave_sum[0], total);
+    if (sl.first) {
+        if (tid < BUCKET_TILES && t < ntiles) tiles[t] = start;
+        if (tid == 0 && (int)sl.bucket == nbuckets - 1) tiles[ntiles] = sl.start + total;
+    }
+    next[tid] = start;
+    partition_batch(v, ok, tile_of, next, cnt, buf, wave_sum[1], out,
+                    [&](unsigned n) { return tid < BUCKET_TILES && n ? atomicAdd(&used[t], n) : 0u; });
+}
+
+constexpr int TILE_THREADS = 512, TILE_ROUNDS = TILE / (8 * TILE_THREADS);   // 8 bins per thread and round
 
 __device__ inline unsigned pack16(int lo, int hi) { return ((unsigned)lo & 0xffffu) | ((unsigned)hi << 16); }
-__device__ inline unsigned pack8(const int *v) {
-    return (unsigned)min(v[0], 255) | (unsigned)min(v[1], 255) << 8 | (unsigned)min(v[2], 255) << 16 |
-           (unsigned)min(v[3], 255) << 24;
+__device__ inline uint4 pack16x8(const int4 &u, const int4 &v) {
+    return make_uint4(pack16(u.x, u.y), pack16(u.z, u.w), pack16(v.x, v.y), pack16(v.z, v.w));
+}
+__device__ inline unsigned pack8(const int4 &v) {
+    return (unsigned)min(v.x, 255) | (unsigned)min(v.y, 255) << 8 | (unsigned)min(v.z, 255) << 16 |
+           (unsigned)min(v.w, 255) << 24;
 }
 
-// Tiles of TILE bins, grid-strided: a tile's keys counted per bin in LDS, then its bins in order,
-// 16 per thread: mode 0 int16(prompts - delayed), mode 2 int16(prompts), mode 1 (BOTH: the two
-// counted apart) int16(prompts) and min(delayed, 255) as bytes, or int16 delayed at sino[S + bin]
-// without a byte output.  int16 values wrap as the reference's short counters do.  vec: the
-// outputs take 16-byte stores (sino, and delayed or sino + S, 16-byte aligned).
+// Tiles of TILE bins, grid-strided: a tile's keys counted per bin in LDS, then its bins written in
+// order, 8 per thread and round, whole lines a wave: mode 0 int16(prompts - delayed), mode 2
+// int16(prompts), mode 1 (BOTH: the two counted apart) int16(prompts) and min(delayed, 255) as bytes, or
+// int16 delayed at sino[S + bin] without a byte output.  int16 values wrap as the reference's short
+// counters do.  The kernel is bound by its writes: the next tile's first keys are loaded while a tile is
+// written, and a thread clears the counters that it has read.  vec: the outputs take 16-byte stores (sino, and
+// delayed or sino + S, 16-byte aligned).
 template <bool BOTH>
 __global__ __launch_bounds__(TILE_THREADS) void lm_tile_kernel(const unsigned *__restrict__ keys,
                                                                const unsigned *__restrict__ tiles, long long ntiles,
@@ -545,56 +750,60 @@ __global__ __launch_bounds__(TILE_THREADS) void lm_tile_kernel(const unsigned *_
     constexpr int NC = BOTH ? 2 : 1;
     __shared__ int4 cnt4[NC * TILE / 4];
     int *cnt = reinterpret_cast<int *>(cnt4);
-    const int j0 = threadIdx.x * TILE_PER_THREAD;
-    for (long long t = blockIdx.x; t < ntiles; t += gridDim.x) {
-        for (int j = threadIdx.x; j < NC * TILE / 4; j += TILE_THREADS) cnt4[j] = make_int4(0, 0, 0, 0);
+    const int tid = threadIdx.x;
+    for (int j = tid; j < NC * TILE / 4; j += TILE_THREADS) cnt4[j] = make_int4(0, 0, 0, 0);
+    auto count = [&](unsigned k) {
+        const int bin = (int)((k >> 1) & (TILE - 1));
+        if (BOTH) atomicAdd(&cnt[(int)(k & 1) * TILE + bin], 1);
+        else atomicAdd(&cnt[bin], (mode == 0 && (k & 1)) ? -1 : 1);
+    };
+    // the ranges of this tile and the next, and this thread's first key of this tile
+    auto range = [&](long long t) { return t < ntiles ? make_uint2(tiles[t], tiles[t + 1]) : make_uint2(0, 0); };
+    auto first = [&](uint2 r) { return r.x + tid < r.y ? keys[r.x + tid] : 0u; };
+    long long t = blockIdx.x;
+    uint2 r = range(t), rn = range(t + gridDim.x);
+    unsigned k = first(r);
+    __syncthreads();
+    for (; t < ntiles; t += gridDim.x) {
+        if (r.x + tid < r.y) count(k);
+        for (unsigned i = r.x + TILE_THREADS + tid; i < r.y; i += TILE_THREADS) count(keys[i]);
+        r = rn;
+        k = first(r);
+        rn = range(t + 2 * gridDim.x);
         __syncthreads();
-        const unsigned a = tiles[t], b = tiles[t + 1];
-        for (unsigned i = a + threadIdx.x; i < b; i += TILE_THREADS) {
-            const unsigned k = keys[i];
-            const int bin = (int)((k >> 1) & (TILE - 1));
-            if (BOTH) atomicAdd(&cnt[(int)(k & 1) * TILE + bin], 1);
-            else atomicAdd(&cnt[bin], (mode == 0 && (k & 1)) ? -1 : 1);
-        }
-        __syncthreads();
-        const long long b0 = t * TILE + j0;
-        int p[TILE_PER_THREAD], d[TILE_PER_THREAD];
 #pragma unroll
-        for (int q = 0; q < TILE_PER_THREAD / 4; q++) {
-            const int4 v = cnt4[(j0 >> 2) + q];
-            p[4 * q] = v.x, p[4 * q + 1] = v.y, p[4 * q + 2] = v.z, p[4 * q + 3] = v.w;
+        for (int q = 0; q < TILE_ROUNDS; q++) {
+            const int j = 2 * (q * TILE_THREADS + tid);      // in fours of bins
+            const long long b0 = t * TILE + 4 * j;
+            const int4 p0 = cnt4[j], p1 = cnt4[j + 1];
+            int4 d0 = make_int4(0, 0, 0, 0), d1 = d0;
+            cnt4[j] = cnt4[j + 1] = make_int4(0, 0, 0, 0);
             if (BOTH) {
-                const int4 w = cnt4[((TILE + j0) >> 2) + q];
-                d[4 * q] = w.x, d[4 * q + 1] = w.y, d[4 * q + 2] = w.z, d[4 * q + 3] = w.w;
+                d0 = cnt4[TILE / 4 + j], d1 = cnt4[TILE / 4 + j + 1];
+                cnt4[TILE / 4 + j] = cnt4[TILE / 4 + j + 1] = make_int4(0, 0, 0, 0);
             }
-        }
-        if (vec && b0 + TILE_PER_THREAD <= S) {
-            uint4 *o = reinterpret_cast<uint4 *>(sino + b0);
-            o[0] = make_uint4(pack16(p[0], p[1]), pack16(p[2], p[3]), pack16(p[4], p[5]), pack16(p[6], p[7]));
-            o[1] = make_uint4(pack16(p[8], p[9]), pack16(p[10], p[11]), pack16(p[12], p[13]), pack16(p[14], p[15]));
-            if (BOTH) {
-                if (delayed) {
-                    *reinterpret_cast<uint4 *>(delayed + b0) = make_uint4(pack8(d), pack8(d + 4), pack8(d + 8), pack8(d + 12));
-                } else {
-                    uint4 *o2 = reinterpret_cast<uint4 *>(sino + S + b0);
-                    o2[0] = make_uint4(pack16(d[0], d[1]), pack16(d[2], d[3]), pack16(d[4], d[5]), pack16(d[6], d[7]));
-                    o2[1] = make_uint4(pack16(d[8], d[9]), pack16(d[10], d[11]), pack16(d[12], d[13]), pack16(d[14], d[15]));
+            if (vec && b0 + 8 <= S) {
+                *reinterpret_cast<uint4 *>(sino + b0) = pack16x8(p0, p1);
+                if (BOTH) {
+                    if (delayed) *reinterpret_cast<uint2 *>(delayed + b0) = make_uint2(pack8(d0), pack8(d1));
+                    else *reinterpret_cast<uint4 *>(sino + S + b0) = pack16x8(d0, d1);
                 }
-            }
-        } else {
+            } else {
+                const int p[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
+                const int d[8] = {d0.x, d0.y, d0.z, d0.w, d1.x, d1.y, d1.z, d1.w};
 #pragma unroll
-            for (int q = 0; q < TILE_PER_THREAD; q++) {
-                const long long i = b0 + q;
-                if (i < S) {
-                    sino[i] = (int16_t)(uint16_t)(unsigned)p[q];
-                    if (BOTH) {
-                        if (delayed) delayed[i] = (uint8_t)min(d[q], 255);
-                        else sino[S + i] = (int16_t)(uint16_t)(unsigned)d[q];
+                for (int i = 0; i < 8; i++) {
+                    if (b0 + i < S) {
+                        sino[b0 + i] = (int16_t)(uint16_t)(unsigned)p[i];
+                        if (BOTH) {
+                            if (delayed) delayed[b0 + i] = (uint8_t)min(d[i], 255);
+                            else sino[S + b0 + i] = (int16_t)(uint16_t)(unsigned)d[i];
+                        }
                     }
                 }
             }
         }
-        __syncthreads();   // the counters are cleared for the next tile
+        __syncthreads();   // the counters are clear for the next tile
     }
 }
 
@@ -673,24 +882,19 @@ int ensure_lm(hrrt_delays &c, long long nchunks, bool coin) {
         DTRY(hipMemcpy(c.d_sol, c.lut.data(), sizeof(int3) * c.lut.size(), hipMemcpyHostToDevice));
     }
     if (!c.d_lm_stats) DTRY(hipMalloc(&c.d_lm_stats, sizeof(unsigned long long) * ST_WORDS));
-    if (!c.d_lm_tiles) {
-        const long long S = (long long)c.nplanes * c.nsino;
-        DTRY(hipMalloc(&c.d_lm_tiles, sizeof(unsigned) * (size_t)((S + TILE - 1) / TILE + 1)));
+    if (!c.d_lm_tiles) {    // first keys of the tiles, then two counters per tile of whole buckets
+        const long long S = (long long)c.nplanes * c.nsino, nb = (S + (1ll << BUCKET_BITS) - 1) >> BUCKET_BITS;
+        DTRY(hipMalloc(&c.d_lm_tiles, sizeof(unsigned) * (size_t)((S + TILE - 1) / TILE + 1 + 2 * nb * BUCKET_TILES)));
     }
     const long long keys = nchunks * (CHUNK / 2);
     if (keys > c.lm_key_cap) {
         if (c.d_lm_keys) DTRY(hipFree(c.d_lm_keys));
-        if (c.d_lm_sort_tmp) DTRY(hipFree(c.d_lm_sort_tmp));
         c.d_lm_keys = nullptr;
-        c.d_lm_sort_tmp = nullptr;
         c.lm_key_cap = 0;
         DTRY(hipMalloc(&c.d_lm_keys, sizeof(unsigned) * 2 * (size_t)keys));
-        size_t bytes = 0;
-        DTRY(rocprim::radix_sort_keys(nullptr, bytes, c.d_lm_keys, c.d_lm_keys + keys, (size_t)keys, 0, 32));
-        DTRY(hipMalloc(&c.d_lm_sort_tmp, bytes));
-        c.lm_sort_bytes = bytes;
         c.lm_key_cap = keys;
     }
+    if (!c.d_lm_part) DTRY(hipMalloc(&c.d_lm_part, sizeof(unsigned) * (size_t)(MAX_BUCKETS * MAX_PARTS + MAX_BUCKETS)));
     if (coin && !c.d_lm_coin_part)
         DTRY(hipMalloc(&c.d_lm_coin_part, sizeof(unsigned) * (size_t)COIN_RANGES * NHEADS * COIN_HEAD));
     if (coin && nchunks > c.lm_coin_cap) {
@@ -706,7 +910,7 @@ int ensure_lm(hrrt_delays &c, long long nchunks, bool coin) {
     if (nchunks > c.lm_chunk_cap) {
         if (c.d_lm_chunks) DTRY(hipFree(c.d_lm_chunks));
         c.d_lm_chunks = nullptr;
-        DTRY(hipMalloc(&c.d_lm_chunks, sizeof(unsigned) * 65 * (size_t)nchunks));   // summaries, then masks
+        DTRY(hipMalloc(&c.d_lm_chunks, sizeof(unsigned) * 66 * (size_t)nchunks));   // summaries, masks, key counts
         c.lm_chunk_cap = nchunks;
     }
     return HRRT_OK;
@@ -750,6 +954,7 @@ extern "C" int hrrt_lm_histogram(hrrt_delays *c, const uint32_t *d_words, long l
     a.ccnt = coin ? c->d_lm_coin_cnt : nullptr;
     a.chunks = c->d_lm_chunks;
     a.cmask = c->d_lm_chunks + c->lm_chunk_cap;
+    a.kcnt = c->d_lm_chunks + 65 * c->lm_chunk_cap;
     a.w16 = (uintptr_t)d_words % 16 == 0;
     a.st = c->d_lm_stats;
     lm_stats_init_kernel<<<(ST_WORDS + 255) / 256, 256, 0, s>>>(a.st);
@@ -765,29 +970,27 @@ extern "C" int hrrt_lm_histogram(hrrt_delays *c, const uint32_t *d_words, long l
         else lm_hist_kernel<false><<<grid, WAVES * 64, 0, s>>>(a, nchunks);
     }
     DTRY(hipGetLastError());
-    // the key slots by tile: the tile bits (key bits 13 and up) sorted, through enough bits that
-    // NOKEY's exceed every tile's
     const long long ntiles = (S + TILE - 1) / TILE;
-    const long long nk = nchunks * (CHUNK / 2);
-    unsigned *sorted = c->d_lm_keys + c->lm_key_cap;
-    if (nk > 0) {
-        unsigned end_bit = TILE_BITS + 1;
-        while ((ntiles >> (end_bit - TILE_BITS - 1)) != 0) end_bit++;
-        size_t bytes = 0;
-        DTRY(rocprim::radix_sort_keys(nullptr, bytes, c->d_lm_keys, sorted, (size_t)nk, TILE_BITS + 1, end_bit, s));
-        if (bytes > c->lm_sort_bytes)
-            return hrrt_dl::fail(HRRT_ERR_HIP, "radix sort scratch of " + std::to_string(bytes) + " bytes exceeds its buffer");
-        DTRY(rocprim::radix_sort_keys(c->d_lm_sort_tmp, bytes, c->d_lm_keys, sorted, (size_t)nk, TILE_BITS + 1, end_bit, s));
-    }
-    lm_tiles_kernel<<<(unsigned)((ntiles + 1 + 255) / 256), 256, 0, s>>>(sorted, nk, ntiles, c->d_lm_tiles);
+    const int nbuckets = (int)((S + (1ll << BUCKET_BITS) - 1) >> BUCKET_BITS);
+    // a wave per chunk of a short stream, at most two workgroups per CU of a long one
+    const int parts = (int)std::min<long long>(std::max<long long>((nchunks + PART_THREADS / 64 - 1) / (PART_THREADS / 64), 1), MAX_PARTS);
+    unsigned *by_bucket = c->d_lm_keys + c->lm_key_cap, *by_tile = c->d_lm_keys, *totals = c->d_lm_part + MAX_BUCKETS * MAX_PARTS;
+    unsigned *tcount = c->d_lm_tiles + ntiles + 1, *used = tcount + (size_t)nbuckets * BUCKET_TILES;
+    const unsigned slices = (unsigned)(nbuckets + nchunks * (CHUNK / 2) / SLICE);    // at least as many as there are
+    lm_count_kernel<<<parts, PART_THREADS, 0, s>>>(a.keys, a.kcnt, nchunks, nbuckets, c->d_lm_part);
+    lm_part_sums_kernel<<<nbuckets, 64, 0, s>>>(c->d_lm_part, parts, totals, tcount, used);
+    lm_scatter_kernel<<<parts, PART_THREADS, 0, s>>>(a.keys, a.kcnt, nchunks, nbuckets, c->d_lm_part, totals, by_bucket);
+    lm_tile_count_kernel<<<slices, PART_THREADS, 0, s>>>(by_bucket, totals, nbuckets, tcount);
+    lm_tile_scatter_kernel<<<slices, PART_THREADS, 0, s>>>(by_bucket, totals, nbuckets, tcount, used, ntiles, by_tile, c->d_lm_tiles);
+    DTRY(hipGetLastError());
     const unsigned tgrid = (unsigned)std::min(ntiles, 1024ll);   // every workgroup resident (4 per CU)
     const bool both = opt->mode == 1;
     const int vec = (uintptr_t)d_sino % 16 == 0 &&
                     (!both || (d_delayed ? (uintptr_t)d_delayed % 16 == 0 : S % 8 == 0));
     if (both)
-        lm_tile_kernel<true><<<tgrid, TILE_THREADS, 0, s>>>(sorted, c->d_lm_tiles, ntiles, S, opt->mode, d_sino, d_delayed, vec);
+        lm_tile_kernel<true><<<tgrid, TILE_THREADS, 0, s>>>(by_tile, c->d_lm_tiles, ntiles, S, opt->mode, d_sino, d_delayed, vec);
     else
-        lm_tile_kernel<false><<<tgrid, TILE_THREADS, 0, s>>>(sorted, c->d_lm_tiles, ntiles, S, opt->mode, d_sino, d_delayed, vec);
+        lm_tile_kernel<false><<<tgrid, TILE_THREADS, 0, s>>>(by_tile, c->d_lm_tiles, ntiles, S, opt->mode, d_sino, d_delayed, vec);
     if (coin) {
         lm_coin_kernel<<<dim3(COIN_RANGES, NHEADS), 1024, 0, s>>>(a.cseg, a.ccnt, nchunks, c->d_lm_coin_part);
         lm_coin_sum_kernel<<<(2 * NCRYS + 255) / 256, 256, 0, s>>>(c->d_lm_coin_part, d_coin_p, d_coin_d);
