@@ -8,6 +8,14 @@
 
 namespace hrrt {
 
+// The batched rotation works on tiles of ROT_TILE x ROT_TILE voxel columns; their positions in a rotated
+// frame, with the upper neighbours, lie in a box of ROT_BOX columns a side: 7 * sqrt(2) = 9.9 apart.
+constexpr int ROT_TILE = 8, ROT_BOX = 12;
+struct RotBox {
+    int x, y;                            // first column
+    unsigned mask[6];                    // bit i: column {i / ROT_BOX, i % ROT_BOX} of the box is read
+};
+
 // Geometry tables resident on the device (uploaded once per context).
 struct DevGeom {
     int N, c, views, Z, Z4, NQ, S, th, K, GM, ZS, spp, sviews, subsets;
@@ -25,6 +33,9 @@ struct DevGeom {
     const int4 *bp_lut2;                 // [N][GM]: {zsa | zea << 16, LDS index of plane 0 of the shifted
                                          //  segment 2k, of segment 2k-1, bits(frac)}
     const float2 *rot;                   // [views/2][N][N] rotation sample positions (rotateimage2 order)
+    const int *rot_tiles;                // tiles {x | y << 16} of voxel columns, the rot_ntiles with FOV columns first
+    const RotBox *rot_box;               // [views/2][rot_ntiles]
+    int rot_ntiles;
     // forward-projector planes by (k, yr): {k | yr << 8 | planes << 16, bits(base plane), bits(tan),
     // delta | ymin << 16}; runs of one and of up to three middle planes of a group, and the end and
     // axial (k = 0) planes one by one

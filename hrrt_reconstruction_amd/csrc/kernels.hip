@@ -1004,35 +1004,132 @@ __device__ __forceinline__ float update1(float img, float corr, float nf, float 
     return image_max < t ? image_max : t;   // _mm_min_ps(image_max, .)
 }
 
-template <bool KAHAN>
-__global__ void __launch_bounds__(256) rot_update_kernel(const DevGeom g, const PairBatch b,
-                                                         const float4 *__restrict__ A, const float4 *__restrict__ B,
-                                                         float4 *__restrict__ image, const float4 *__restrict__ nf) {
-    int x, yg;
+__device__ __forceinline__ float invert1(float s, float eps1) { return fabsf(s) > eps1 ? (1.0f / s) : 0.0f; }
+
+// The rotation of a batch by tiles: a workgroup takes ROT_TILE x ROT_TILE voxel columns and ROT_Q chunks
+// of four planes of them.  Read from memory by each voxel, the eight neighbours (four of A, four of B) moved
+// 308 MB a view pair of a 256 x 256 x 207 image from L2 into the L1s (33 us a pair, the same
+// when both buffers lie in the last-level cache).  Here a tile's columns in the rotated frame are read
+// once per pair, summed as A + B, and kept in LDS, double buffered: the next pair's columns are
+// loaded while a pair is accumulated.  They lie in a box of 12 x 12 for a tile of 8 x 8; a mask says which
+// of the box a voxel touches (some 86 of 120).  Tiles and boxes come from the host (rot_tiles: those
+// with a FOV voxel first, strip by strip so that an XCD's share of them is compact; rot_box).
+// Nine pairs, 256 x 256 x 207: 300 -> 235 us; eight frames of eight pairs, 128 x 128: 310 -> 259 us, where
+// reading A and B once takes 264 at the rate of a copy.
+//   ROT_UPDATE  the image update with the sum;  ROT_SUM  the sum itself (rotate_image_buf into a zeroed
+//   correction, PJ:1701-1725);  ROT_SENS  its inverse, and zeros outside the FOV (all tiles)
+enum RotMode { ROT_UPDATE, ROT_SUM, ROT_SENS };
+constexpr int ROT_Q = 8, ROT_THREADS = ROT_TILE * ROT_TILE * ROT_Q, ROT_COLS = ROT_BOX * ROT_BOX;
+constexpr int ROT_LOADS = (ROT_COLS * ROT_Q + ROT_THREADS - 1) / ROT_THREADS;
+
+template <bool KAHAN, int MODE>
+__global__ void __launch_bounds__(ROT_THREADS) rot_tile_kernel(const DevGeom g, const PairBatch b,
+                                                               const float4 *__restrict__ A,
+                                                               const float4 *__restrict__ B, float4 *__restrict__ out,
+                                                               const float4 *__restrict__ nf, int nchunks) {
+    __shared__ float4 box[2][ROT_COLS * ROT_Q];
+    const int N = g.N, NQ = g.NQ, tid = threadIdx.x;
     const int frame = blockIdx.y;
     A += frame * b.buf_stride / 4;
     B += frame * b.buf_stride / 4;
-    image += frame * b.img_stride / 4;
-    rot_block(blockIdx.x, g.N, (g.N + 3) / 4, x, yg);
-    const int q = threadIdx.x, y = yg * blockDim.y + threadIdx.y;
-    if (q >= g.NQ || y < g.cyl_lo[x] || y >= g.cyl_hi[x]) return;
-    const float4 corr = rotate_accumulate<KAHAN>(g, b, A, B, x, y, q);
-    const size_t i = ((size_t)x * g.N + y) * g.NQ + q;
-    const float4 im = image[i], n = nf[i];
-    image[i] = make_float4(update1(im.x, corr.x, n.x, g.image_max), update1(im.y, corr.y, n.y, g.image_max),
-                           update1(im.z, corr.z, n.z, g.image_max), update1(im.w, corr.w, n.w, g.image_max));
-}
-
-// Rotation sum only (rotate_image_buf into a zeroed correction, PJ:1701-1725), for the
-// paths that filter the correction or the sensitivity before using it.
-__global__ void __launch_bounds__(256) rot_sum_kernel(const DevGeom g, const PairBatch b,
-                                                      const float4 *__restrict__ A, const float4 *__restrict__ B,
-                                                      float4 *__restrict__ corr) {
-    int x, yg;
-    rot_block(blockIdx.x, g.N, (g.N + 3) / 4, x, yg);
-    const int q = threadIdx.x, y = yg * blockDim.y + threadIdx.y;
-    if (q >= g.NQ || y < g.cyl_lo[x] || y >= g.cyl_hi[x]) return;
-    corr[((size_t)x * g.N + y) * g.NQ + q] = rotate_accumulate<false>(g, b, A, B, x, y, q);
+    out += frame * b.img_stride / 4;
+    // workgroups are dealt to the XCDs in turn: each takes a run of the FOV tiles, all chunks of a tile
+    const int per = (g.rot_ntiles + 7) >> 3;
+    int ti, chunk;
+    if ((int)blockIdx.x < 8 * per * nchunks) {
+        const int i = blockIdx.x >> 3;
+        ti = (blockIdx.x & 7) * per + i / nchunks;
+        chunk = i % nchunks;
+        if (i / nchunks >= per || ti >= g.rot_ntiles) return;
+    } else {
+        const int i = blockIdx.x - 8 * per * nchunks;
+        ti = g.rot_ntiles + i / nchunks;
+        chunk = i % nchunks;
+    }
+    const int tile = g.rot_tiles[ti];
+    const int col = tid / ROT_Q, ql = tid % ROT_Q, q = chunk * ROT_Q + ql;
+    const int x = (tile & 0xffff) * ROT_TILE + col / ROT_TILE, y = (tile >> 16) * ROT_TILE + col % ROT_TILE;
+    const bool inside = x < N && y < N && q < NQ, live = inside && y >= g.cyl_lo[x] && y < g.cyl_hi[x];
+    const size_t o = ((size_t)x * N + y) * NQ + q;
+    if (ti >= g.rot_ntiles) {       // ROT_SENS: no FOV voxel
+        if (inside) out[o] = f4(0.f);
+        return;
+    }
+    // this thread's columns of a box (col + 64 k): their byte offsets from the box's first column
+    unsigned off[ROT_LOADS];
+#pragma unroll
+    for (int k = 0; k < ROT_LOADS; k++) {
+        const int c = col + k * (ROT_TILE * ROT_TILE);
+        off[k] = (unsigned)(((c / ROT_BOX) * N + c % ROT_BOX) * NQ + q) * 16u;
+    }
+    const int half = __builtin_amdgcn_readfirstlane(tid >> 8);      // a wave's columns lie in one word of the mask
+    const unsigned bit = q < NQ ? 1u << (col & 31) : 0u;
+    const RotBox *boxes = g.rot_box + (size_t)b.view0 * g.rot_ntiles + ti;
+    const float2 *rt = g.rot + ((size_t)b.view0 * N + min(x, N - 1)) * N + min(y, N - 1);
+    const size_t vstride = (size_t)N * N * b.view_stride, bstride = (size_t)g.rot_ntiles * b.view_stride;
+    float4 va[ROT_LOADS], vb[ROT_LOADS];
+    auto load = [&](int lp, const RotBox &r) __attribute__((always_inline)) {
+        const size_t base = (size_t)lp * N * N * NQ + ((size_t)r.x * N + r.y) * NQ;
+        const char *pa = reinterpret_cast<const char *>(A + base), *pb = reinterpret_cast<const char *>(B + base);
+#pragma unroll
+        for (int k = 0; k < ROT_LOADS; k++) {
+            if ((half ? r.mask[2 * k + 1] : r.mask[2 * k]) & bit) {
+                va[k] = *reinterpret_cast<const float4 *>(pa + off[k]);
+                vb[k] = *reinterpret_cast<const float4 *>(pb + off[k]);
+            }
+        }
+    };
+    auto store = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < ROT_LOADS; k++)
+            if (tid + k * ROT_THREADS < ROT_COLS * ROT_Q) box[buf][tid + k * ROT_THREADS] = add4(va[k], vb[k]);
+    };
+#pragma unroll
+    for (int k = 0; k < ROT_LOADS; k++) va[k] = vb[k] = f4(0.f);
+    float4 corr = f4(0.f), comp = f4(0.f);
+    RotBox r = boxes[0];
+    float2 p = rt[0];
+    load(0, r);
+    store(0);
+    __syncthreads();
+    for (int lp = 0; lp < b.npairs; lp++) {
+        const bool more = lp + 1 < b.npairs;
+        const RotBox rn = boxes[more ? bstride * (lp + 1) : 0];
+        const float2 pn = rt[more ? vstride * (lp + 1) : 0];
+        if (more) load(lp + 1, rn);
+        const int xi = (int)p.x, yi = (int)p.y;
+        if (live && !(xi < 0 || xi > N - 2 || yi < 0 || yi > N - 2)) {
+            const float x1 = p.x - xi, y1 = p.y - yi;
+            const float w1 = (1 - x1) * (1 - y1), w2 = x1 * (1 - y1), w3 = y1 * (1 - x1), w4 = y1 * x1;
+            const float4 *m = &box[lp & 1][((xi - r.x) * ROT_BOX + yi - r.y) * ROT_Q + ql];
+            const float4 m1 = m[0], m2 = m[ROT_BOX * ROT_Q], m3 = m[ROT_Q], m4 = m[(ROT_BOX + 1) * ROT_Q];
+            const float4 v = add4(add4(mul4(m1, w1), mul4(m2, w2)), add4(mul4(m3, w3), mul4(m4, w4)));
+            if (KAHAN) {
+                kahan_add(corr.x, comp.x, v.x);
+                kahan_add(corr.y, comp.y, v.y);
+                kahan_add(corr.z, comp.z, v.z);
+                kahan_add(corr.w, comp.w, v.w);
+            } else {
+                corr = add4(corr, v);
+            }
+        }
+        if (more) store((lp + 1) & 1);
+        r = rn;
+        p = pn;
+        __syncthreads();
+    }
+    if (MODE == ROT_UPDATE) {
+        if (!live) return;
+        const float4 im = out[o], n = nf[o];
+        out[o] = make_float4(update1(im.x, corr.x, n.x, g.image_max), update1(im.y, corr.y, n.y, g.image_max),
+                             update1(im.z, corr.z, n.z, g.image_max), update1(im.w, corr.w, n.w, g.image_max));
+    } else if (MODE == ROT_SUM) {
+        if (live) out[o] = corr;
+    } else if (inside) {
+        const int z = 4 * q;
+        out[o] = make_float4(live && z + 0 < g.Z ? invert1(corr.x, g.eps1) : 0.0f, live && z + 1 < g.Z ? invert1(corr.y, g.eps1) : 0.0f,
+                             live && z + 2 < g.Z ? invert1(corr.z, g.eps1) : 0.0f, live && z + 3 < g.Z ? invert1(corr.w, g.eps1) : 0.0f);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1151,26 +1248,6 @@ __global__ void __launch_bounds__(256) flat_image_kernel(const DevGeom g, const 
             dst[((size_t)a * N + b) * g.Z4 + z] = (in && z < g.Z) ? tile[i][t] : 0.0f;
         }
     }
-}
-
-__device__ __forceinline__ float invert1(float s, float eps1) { return fabsf(s) > eps1 ? (1.0f / s) : 0.0f; }
-
-template <bool KAHAN>
-__global__ void __launch_bounds__(256) rot_sens_kernel(const DevGeom g, const PairBatch b,
-                                                       const float4 *__restrict__ A, const float4 *__restrict__ B,
-                                                       float4 *__restrict__ nf) {
-    int x, yg;
-    rot_block(blockIdx.x, g.N, (g.N + 3) / 4, x, yg);
-    const int q = threadIdx.x, y = yg * blockDim.y + threadIdx.y;
-    if (q >= g.NQ || y < g.cyl_lo[x] || y >= g.cyl_hi[x]) return;
-    const float4 s = rotate_accumulate<KAHAN>(g, b, A, B, x, y, q);
-    const int z = 4 * q;
-    float4 o;
-    o.x = z + 0 < g.Z ? invert1(s.x, g.eps1) : 0.0f;
-    o.y = z + 1 < g.Z ? invert1(s.y, g.eps1) : 0.0f;
-    o.z = z + 2 < g.Z ? invert1(s.z, g.eps1) : 0.0f;
-    o.w = z + 3 < g.Z ? invert1(s.w, g.eps1) : 0.0f;
-    nf[((size_t)x * g.N + y) * g.NQ + q] = o;
 }
 
 __global__ void __launch_bounds__(256) rot_add_kernel(const DevGeom g, int view, const float4 *__restrict__ A,
@@ -1299,11 +1376,6 @@ __global__ void end_iteration_kernel(const DevGeom g, float *__restrict__ image,
             float *v = image + ((size_t)x * g.N + y) * g.Z4 + z;
             if ((double)*v < 1e-16) *v = 0.0f;
         }
-}
-
-__global__ void fill_kernel(float4 *__restrict__ p, size_t n4) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (size_t)gridDim.x * blockDim.x)
-        p[i] = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
 __global__ void fill_u64_kernel(unsigned long long *__restrict__ p, int n) {
@@ -1899,24 +1971,31 @@ hipError_t launch_backproject_incremental(const DevGeom &g, const PairBatch &b, 
     return hipGetLastError();
 }
 
+template <bool KAHAN, int MODE>
+static void launch_rot_tile(const DevGeom &g, const PairBatch &b, const float4 *A, const float4 *B, float4 *out,
+                            const float4 *nf, hipStream_t s) {
+    const int nchunks = (g.NQ + ROT_Q - 1) / ROT_Q, side = (g.N + ROT_TILE - 1) / ROT_TILE;
+    const int ntiles = 8 * ((g.rot_ntiles + 7) / 8) + (MODE == ROT_SENS ? side * side - g.rot_ntiles : 0);
+    hipLaunchKernelGGL((rot_tile_kernel<KAHAN, MODE>), dim3(ntiles * nchunks, b.nframes), dim3(ROT_THREADS), 0, s, g, b, A, B,
+                       out, nf, nchunks);
+}
+
 hipError_t launch_rotate_update(const DevGeom &g, const PairBatch &b, const float *bufA, const float *bufB,
                                 float *image, const float *normfac, int kahan, hipStream_t s) {
     const float4 *A = reinterpret_cast<const float4 *>(bufA), *B = reinterpret_cast<const float4 *>(bufB);
     float4 *im = reinterpret_cast<float4 *>(image);
     const float4 *nf = reinterpret_cast<const float4 *>(normfac);
-    if (kahan) hipLaunchKernelGGL(rot_update_kernel<true>, rot_grid(g, b.nframes), dim3(64, 4), 0, s, g, b, A, B, im, nf);
-    else hipLaunchKernelGGL(rot_update_kernel<false>, rot_grid(g, b.nframes), dim3(64, 4), 0, s, g, b, A, B, im, nf);
+    if (kahan) launch_rot_tile<true, ROT_UPDATE>(g, b, A, B, im, nf, s);
+    else launch_rot_tile<false, ROT_UPDATE>(g, b, A, B, im, nf, s);
     return hipGetLastError();
 }
 
 hipError_t launch_rotate_sens(const DevGeom &g, const PairBatch &b, const float *bufA, const float *bufB,
                               float *normfac_out, int kahan, hipStream_t s) {
-    size_t n4 = (size_t)g.N * g.N * g.NQ;
-    hipLaunchKernelGGL(fill_kernel, dim3(1024), dim3(256), 0, s, reinterpret_cast<float4 *>(normfac_out), n4);
     const float4 *A = reinterpret_cast<const float4 *>(bufA), *B = reinterpret_cast<const float4 *>(bufB);
     float4 *o = reinterpret_cast<float4 *>(normfac_out);
-    if (kahan) hipLaunchKernelGGL(rot_sens_kernel<true>, rot_grid(g), dim3(64, 4), 0, s, g, b, A, B, o);
-    else hipLaunchKernelGGL(rot_sens_kernel<false>, rot_grid(g), dim3(64, 4), 0, s, g, b, A, B, o);
+    if (kahan) launch_rot_tile<true, ROT_SENS>(g, b, A, B, o, nullptr, s);
+    else launch_rot_tile<false, ROT_SENS>(g, b, A, B, o, nullptr, s);
     return hipGetLastError();
 }
 
@@ -1989,8 +2068,8 @@ hipError_t launch_update_image(const DevGeom &g, float *image, float *corr, cons
 
 hipError_t launch_rotate_sum(const DevGeom &g, const PairBatch &b, const float *bufA, const float *bufB, float *corr,
                              hipStream_t s) {
-    hipLaunchKernelGGL(rot_sum_kernel, rot_grid(g), dim3(64, 4), 0, s, g, b, reinterpret_cast<const float4 *>(bufA),
-                       reinterpret_cast<const float4 *>(bufB), reinterpret_cast<float4 *>(corr));
+    launch_rot_tile<false, ROT_SUM>(g, b, reinterpret_cast<const float4 *>(bufA), reinterpret_cast<const float4 *>(bufB),
+                                    reinterpret_cast<float4 *>(corr), nullptr, s);
     return hipGetLastError();
 }
 
