@@ -90,7 +90,7 @@ struct hrrt_ctx {
     // that voxels outside the FOV, which the blur never writes, read as zero
     bool psf_on = false;
     std::vector<float> psf_k[3], psf_normz;
-    float *d_psf = nullptr;          // [taps x][taps y][normz]
+    float *d_psf = nullptr;          // [normz][taps x][taps y]
     float *psf_img = nullptr, *psf_corr = nullptr, *psf_buf = nullptr;
     float *flat = nullptr;           // [z_pixels][N][N] staging of the flat image files
     int ensure_psf_scratch() {
@@ -100,10 +100,11 @@ struct hrrt_ctx {
         if ((r = zalloc((void **)&psf_buf, sizeof(float) * vol_floats()))) return r;
         return HRRT_OK;
     }
-    hipError_t convolve3d(const float *in, float *out, hipStream_t s) const {
+    // with normfac, out is an image and takes the update with the blurred volume
+    hipError_t convolve3d(const float *in, float *out, hipStream_t s, const float *normfac = nullptr) const {
         const int hx = ((int)psf_k[0].size() - 1) / 2, hy = ((int)psf_k[1].size() - 1) / 2;
-        return hrrt::launch_convolve3d(dg, in, out, psf_buf, d_psf, hx, d_psf + psf_k[0].size(), hy,
-                                       d_psf + psf_k[0].size() + psf_k[1].size(), geo.z_min, geo.z_max, s);
+        const float *taps = d_psf + psf_normz.size();
+        return hrrt::launch_convolve3d(dg, in, out, psf_buf, taps, hx, taps + psf_k[0].size(), hy, d_psf, geo.z_min, geo.z_max, normfac, s);
     }
     // optional per-kernel timing of hrrt_osem_subset (HIP events on the launch stream)
     bool timing = false;
@@ -1012,8 +1013,7 @@ extern "C" int hrrt_osem_subset(hrrt_ctx *ctx, float *d_image, const float *d_no
     ctx->mark(2, S(stream));
     if (ctx->psf_on) {   // the correction is blurred before the update (S3:4229)
         HIP_TRY(hrrt::launch_rotate_sum(ctx->dg, b, ctx->bufA, ctx->bufB, ctx->psf_corr, S(stream)));
-        HIP_TRY(ctx->convolve3d(ctx->psf_corr, ctx->psf_corr, S(stream)));
-        HIP_TRY(hrrt::launch_update_image(ctx->dg, d_image, ctx->psf_corr, d_normfac_subset, S(stream)));
+        HIP_TRY(ctx->convolve3d(ctx->psf_corr, d_image, S(stream), d_normfac_subset));
     } else {
         HIP_TRY(hrrt::launch_rotate_update(ctx->dg, b, ctx->bufA, ctx->bufB, d_image, d_normfac_subset, 0,
                                            S(stream)));
@@ -1045,8 +1045,7 @@ extern "C" int hrrt_osem_subset_w012(hrrt_ctx *ctx, float *d_image, const float 
     ctx->mark(2, S(stream));
     if (ctx->psf_on) {
         HIP_TRY(hrrt::launch_rotate_sum(ctx->dg, b, ctx->bufA, ctx->bufB, ctx->psf_corr, S(stream)));
-        HIP_TRY(ctx->convolve3d(ctx->psf_corr, ctx->psf_corr, S(stream)));
-        HIP_TRY(hrrt::launch_update_image(ctx->dg, d_image, ctx->psf_corr, d_normfac_subset, S(stream)));
+        HIP_TRY(ctx->convolve3d(ctx->psf_corr, d_image, S(stream), d_normfac_subset));
     } else {
         HIP_TRY(hrrt::launch_rotate_update(ctx->dg, b, ctx->bufA, ctx->bufB, d_image, d_normfac_subset, 0,
                                            S(stream)));
@@ -1445,9 +1444,9 @@ extern "C" int hrrt_set_psf(hrrt_ctx *ctx, int enable, float fwhm1, float fwhm2,
         }
     for (int z = 0; z < G.z4; z++)
         if (normz[z] > 0) normz[z] = 1 / normz[z];
-    std::vector<float> packed(k[0]);
+    std::vector<float> packed(normz);
+    packed.insert(packed.end(), k[0].begin(), k[0].end());
     packed.insert(packed.end(), k[1].begin(), k[1].end());
-    packed.insert(packed.end(), normz.begin(), normz.end());
     if (ctx->d_psf) (void)hipFree(ctx->d_psf);
     ctx->d_psf = nullptr;
     if (hipMalloc((void **)&ctx->d_psf, sizeof(float) * packed.size()) != hipSuccess)

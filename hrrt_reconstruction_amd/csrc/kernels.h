@@ -126,10 +126,12 @@ hipError_t launch_flat_image(const DevGeom &g, const float *src, float *dst, int
 // rotation of the batch's pairs summed into corr (FOV voxels), no update
 hipError_t launch_rotate_sum(const DevGeom &g, const PairBatch &b, const float *bufA, const float *bufB, float *corr,
                              hipStream_t s);
-// PSF blur convolve3d: x pass in -> buf, y/z pass buf -> out (out may be in); taps of the x and
+// PSF blur convolve3d: x pass in -> buf, y/z pass buf -> out (out may be in), or, with normfac, the image
+// update of out with the blurred volume as its correction; taps of the x and
 // y kernels with half-widths hx, hy; normz [Z4]; the z pass keeps planes inside [z_min, z_max)
 hipError_t launch_convolve3d(const DevGeom &g, const float *in, float *out, float *buf, const float *taps_x, int hx,
-                             const float *taps_y, int hy, const float *normz, int z_min, int z_max, hipStream_t s);
+                             const float *taps_y, int hy, const float *normz, int z_min, int z_max,
+                             const float *normfac, hipStream_t s);
 hipError_t launch_init_image(const DevGeom &g, float *image, int z_min, int z_max, hipStream_t s);
 hipError_t launch_end_iteration(const DevGeom &g, float *image, int z_min, int z_max, hipStream_t s);
 // Segments [th0, th0 + nth) (their file blocks must be in place), written to the padded planes

@@ -1141,65 +1141,162 @@ __global__ void __launch_bounds__(ROT_THREADS) rot_tile_kernel(const DevGeom g, 
 // the planes z + mask inside [z_min, z_max), and is scaled by normz(z) * (1/sum
 // of the y taps).  Only FOV voxels are written, as in the reference.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) psf_x_kernel(const DevGeom g, const float4 *__restrict__ in,
-                                                    float4 *__restrict__ out, const float *__restrict__ taps, int h) {
-    int x, yg;
-    rot_block(blockIdx.x, g.N, (g.N + 3) / 4, x, yg);
-    const int q = threadIdx.x, y = yg * blockDim.y + threadIdx.y;
-    if (q >= g.NQ || y < g.cyl_lo[x] || y >= g.cyl_hi[x]) return;
-    const int lo = g.cyl_lo[y], hi = g.cyl_hi[y];
-    float4 acc = f4(0.f);
-    float norm = 0.0f;
-    for (int mask = -h; mask < h; mask++) {
-        const int m2 = x + mask;
-        if (m2 < lo || m2 >= hi) continue;
-        const float f = taps[mask + h];
-        norm = norm + f;
-        acc = add4(acc, mul4(in[((size_t)m2 * g.N + y) * g.NQ + q], f));
+// Both passes were bound by their loads (a float4 per tap and output) and the z pass by its LDS reads and
+// tests (a float per tap and plane).  A wave now makes PSF_R outputs that follow each other along the axis of its
+// taps from one walk over their inputs, and a lane makes four planes from whole float4s of the column.
+// 256 x 256 x 207, 13 taps: x pass 45 -> 30 us, y/z pass 88 -> 48 us (60 with the update).
+constexpr int PSF_R = 4;
+
+// acc[j] += in * tap and norm[j] += tap for every output first + j and input m in [m0, m1) with a tap m - (first + j)
+// in [-h, h), taps ascending; at(m) is the input of position m (wave-uniform).  Four inputs at a time, the next
+// four in flight; inputs and outputs the same distance apart share their tap, so it is tested and read once
+// for them (an output still meets its inputs in order).
+__device__ __forceinline__ void psf_tap(float f, const float4 &v, float4 &acc, float &norm) {
+    norm = norm + f;
+    acc = add4(acc, mul4(v, f));
+}
+template <typename At>
+__device__ __forceinline__ void psf_walk(int first, int m0, int m1, const float *__restrict__ taps, int h, At at,
+                                         float4 (&acc)[PSF_R], float (&norm)[PSF_R]) {
+    float4 v[PSF_R], vn[PSF_R];
+#pragma unroll
+    for (int j = 0; j < PSF_R; j++) acc[j] = f4(0.f), norm[j] = 0.0f;
+    if (m0 >= m1) return;
+    auto load = [&](int m) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < PSF_R; i++) vn[i] = at(min(m + i, m1 - 1));
+    };
+    load(m0);
+    for (int m = m0; m < m1; m += PSF_R) {
+#pragma unroll
+        for (int i = 0; i < PSF_R; i++) v[i] = vn[i];
+        if (m + PSF_R < m1) load(m + PSF_R);
+        if (m + PSF_R <= m1) {
+#pragma unroll
+            for (int d = 1 - PSF_R; d < PSF_R; d++) {
+                const int t = m + d - first + h;
+                if (t < 0 || t >= 2 * h) continue;
+                const float f = taps[t];
+#pragma unroll
+                for (int j = 0; j < PSF_R; j++)
+                    if (j + d >= 0 && j + d < PSF_R) psf_tap(f, v[(j + d) & (PSF_R - 1)], acc[j], norm[j]);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < PSF_R; i++) {
+                if (m + i >= m1) break;
+#pragma unroll
+                for (int j = 0; j < PSF_R; j++) {
+                    const int t = m + i - (first + j) + h;
+                    if (t >= 0 && t < 2 * h) psf_tap(taps[t], v[i], acc[j], norm[j]);
+                }
+            }
+        }
     }
-    if (norm != 1.0f && norm != 0.0f) acc = mul4(acc, 1.0f / norm);
-    out[((size_t)x * g.N + y) * g.NQ + q] = acc;
 }
 
+// workgroup -> (line, run of PSF_R outputs along it): an XCD gets a band of lines, run after run
+__device__ __forceinline__ bool psf_block(int bid, int nlines, int nruns, int &line, int &run) {
+    const int per = (nlines + 7) >> 3, r = bid >> 3;
+    line = (bid & 7) * per + r / nruns;
+    run = r % nruns;
+    return r / nruns < per && line < nlines;
+}
+
+// a workgroup's four waves take four rows y
+__global__ void __launch_bounds__(256) psf_x_kernel(const DevGeom g, const float4 *__restrict__ in,
+                                                    float4 *__restrict__ out, const float *__restrict__ taps, int h) {
+    int yg, run;
+    if (!psf_block(blockIdx.x, (g.N + 3) / 4, (g.N + PSF_R - 1) / PSF_R, yg, run)) return;
+    const int q = threadIdx.x, y = yg * 4 + __builtin_amdgcn_readfirstlane(threadIdx.y), x0 = run * PSF_R;
+    if (q >= g.NQ || y >= g.N) return;
+    float4 acc[PSF_R];
+    float norm[PSF_R];
+    psf_walk(x0, max(x0 - h, g.cyl_lo[y]), min(x0 + PSF_R - 1 + h, g.cyl_hi[y]), taps, h,
+             [&](int m) { return in[((size_t)m * g.N + y) * g.NQ + q]; }, acc, norm);
+#pragma unroll
+    for (int j = 0; j < PSF_R; j++) {
+        const int x = x0 + j;
+        if (x >= g.N || y < g.cyl_lo[x] || y >= g.cyl_hi[x]) continue;
+        if (norm[j] != 1.0f && norm[j] != 0.0f) acc[j] = mul4(acc[j], 1.0f / norm[j]);
+        out[((size_t)x * g.N + y) * g.NQ + q] = acc[j];
+    }
+}
+
+// UPDATE: the blurred column is the correction of the image update of `out` (pt_cal_updateimage
+// S3:2033-2056) instead of the result.  Dynamic LDS: PSF_R columns a wave with pad zero quads at each end.
+template <bool UPDATE>
 __global__ void __launch_bounds__(256) psf_yz_kernel(const DevGeom g, const float4 *__restrict__ in,
-                                                     float *__restrict__ out, const float *__restrict__ taps, int h,
+                                                     float4 *__restrict__ out, const float4 *__restrict__ nf,
+                                                     const float *__restrict__ taps, int h, int pad,
                                                      const float *__restrict__ normz, int z_min, int z_max) {
-    __shared__ float col[4][256];
-    int x, yg;
-    rot_block(blockIdx.x, g.N, (g.N + 3) / 4, x, yg);
-    const int q = threadIdx.x, ty = threadIdx.y, y = yg * blockDim.y + ty;
-    const int lo = g.cyl_lo[x], hi = g.cyl_hi[x];
-    const bool fov = y >= lo && y < hi;
-    float norm = 0.0f;
-    if (fov) {
-        float4 acc = f4(0.f);
-        for (int mask = -h; mask < h; mask++) {
-            const int m2 = y + mask;
-            if (m2 < lo || m2 >= hi) continue;
-            const float f = taps[mask + h];
-            norm = norm + f;
-            if (q < g.NQ) acc = add4(acc, mul4(in[((size_t)x * g.N + m2) * g.NQ + q], f));
-        }
-        if (q < g.NQ) {
-            col[ty][4 * q + 0] = acc.x;
-            col[ty][4 * q + 1] = acc.y;
-            col[ty][4 * q + 2] = acc.z;
-            col[ty][4 * q + 3] = acc.w;
-        }
+    extern __shared__ float4 cols[];
+    int x, run;
+    if (!psf_block(blockIdx.x, g.N, (g.N + 4 * PSF_R - 1) / (4 * PSF_R), x, run)) return;
+    const int q = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int y0 = (run * 4 + wv) * PSF_R, lo = g.cyl_lo[x], hi = g.cyl_hi[x], len = g.NQ + 2 * pad;
+    float4 *col = cols + wv * PSF_R * len;
+    float norm[PSF_R];
+    if (q < g.NQ) {
+        float4 acc[PSF_R];
+        psf_walk(y0, max(y0 - h, lo), min(y0 + PSF_R - 1 + h, hi), taps, h,
+                 [&](int m) { return in[((size_t)x * g.N + m) * g.NQ + q]; }, acc, norm);
+        // planes outside [z_min, z_max) take no part in the z sums: zeros there (adding a zero leaves a sum
+        // that began at +0 as it is)
+        const int z = 4 * q;
+#pragma unroll
+        for (int j = 0; j < PSF_R; j++)
+            col[j * len + pad + q] = make_float4(z + 0 >= z_min && z + 0 < z_max ? acc[j].x : 0.0f, z + 1 >= z_min && z + 1 < z_max ? acc[j].y : 0.0f,
+                                                 z + 2 >= z_min && z + 2 < z_max ? acc[j].z : 0.0f, z + 3 >= z_min && z + 3 < z_max ? acc[j].w : 0.0f);
+    }
+    for (int i = q; i < 2 * pad * PSF_R; i += 64) {
+        const int j = i / (2 * pad), k = i % (2 * pad);
+        col[j * len + (k < pad ? k : g.NQ + k)] = f4(0.f);
     }
     __syncthreads();
-    if (!fov) return;
-    float *o = out + ((size_t)x * g.N + y) * g.Z4;
-    for (int z = q; z < g.Z4; z += 64) {
-        float v = 0.0f;
-        if (norm != 0.0f) {
-            for (int mask = -h; mask < h; mask++) {
-                const int zz = z + mask;
-                if (z < g.Z && zz >= z_min && zz < z_max) v = v + col[ty][zz] * taps[mask + h];
-            }
-            v = v * (normz[z] * (1.0f / norm));
+    if (q >= g.NQ) return;
+    // the z sums of all columns, a tap (the same for planes the same distance apart) tested and read once
+    float v[PSF_R][4];
+#pragma unroll
+    for (int j = 0; j < PSF_R; j++) v[j][0] = v[j][1] = v[j][2] = v[j][3] = 0.0f;
+    for (int i = -pad; i <= pad; i++) {
+        float w[PSF_R][4];
+#pragma unroll
+        for (int j = 0; j < PSF_R; j++) {
+            const float4 c = col[j * len + pad + q + i];
+            w[j][0] = c.x, w[j][1] = c.y, w[j][2] = c.z, w[j][3] = c.w;
         }
-        o[z] = v;
+#pragma unroll
+        for (int d = -3; d < 4; d++) {
+            const int t = 4 * i + d + h;
+            if (t < 0 || t >= 2 * h) continue;
+            const float f = taps[t];
+#pragma unroll
+            for (int j = 0; j < PSF_R; j++)
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if (k + d >= 0 && k + d < 4) v[j][k] = v[j][k] + w[j][(k + d) & 3] * f;
+        }
+    }
+    const float4 nz = reinterpret_cast<const float4 *>(normz)[q];
+    const int z = 4 * q;
+#pragma unroll
+    for (int j = 0; j < PSF_R; j++) {
+        const int y = y0 + j;
+        if (y < lo || y >= hi) continue;
+        float4 r = f4(0.f);
+        if (norm[j] != 0.0f) {
+            const float in1 = 1.0f / norm[j];
+            r = make_float4((z + 0 < g.Z ? v[j][0] : 0.0f) * (nz.x * in1), (z + 1 < g.Z ? v[j][1] : 0.0f) * (nz.y * in1),
+                            (z + 2 < g.Z ? v[j][2] : 0.0f) * (nz.z * in1), (z + 3 < g.Z ? v[j][3] : 0.0f) * (nz.w * in1));
+        }
+        const size_t o = ((size_t)x * g.N + y) * g.NQ + q;
+        if (UPDATE) {
+            const float4 im = out[o], n = nf[o];
+            r = make_float4(update1(im.x, r.x, n.x, g.image_max), update1(im.y, r.y, n.y, g.image_max),
+                            update1(im.z, r.z, n.z, g.image_max), update1(im.w, r.w, n.w, g.image_max));
+        }
+        out[o] = r;
     }
 }
 
@@ -1340,42 +1437,58 @@ __global__ void ratio_w012_kernel(const DevGeom g, float *__restrict__ est, cons
     }
 }
 
-__global__ void update_image_kernel(const DevGeom g, float *__restrict__ image, float *__restrict__ corr,
-                                    const float *__restrict__ nf) {
-    const int x = blockIdx.x;
-    for (int y = g.cyl_lo[x] + threadIdx.y; y < g.cyl_hi[x]; y += blockDim.y)
-        for (int z = threadIdx.x; z < g.Z4; z += blockDim.x) {
-            const size_t i = ((size_t)x * g.N + y) * g.Z4 + z;
-            image[i] = update1(image[i], corr[i], nf[i], g.image_max);
-            corr[i] = 0.0f;
-        }
+// The voxelwise image kernels take four columns a workgroup, a wave each, four planes a lane (a
+// workgroup per x left 3/4 of the chip's wavefronts empty: 121 us for the update of a 256 x 256 x 207 image,
+// 35 us for the end of an iteration at 128 x 128).
+__device__ __forceinline__ bool image_voxels(const DevGeom &g, int &x, int &y, size_t &i) {
+    int yg;
+    rot_block(blockIdx.x, g.N, (g.N + 3) / 4, x, yg);
+    y = yg * 4 + threadIdx.y;
+    i = ((size_t)x * g.N + y) * g.NQ + threadIdx.x;
+    return y < g.N;
 }
 
-__global__ void normfac_invert_kernel(const DevGeom g, const float *__restrict__ sens, float *__restrict__ out) {
-    const int x = blockIdx.x;
-    for (int y = g.cyl_lo[x] + threadIdx.y; y < g.cyl_hi[x]; y += blockDim.y)
-        for (int z = threadIdx.x; z < g.Z; z += blockDim.x) {
-            const size_t i = ((size_t)x * g.N + y) * g.Z4 + z;
-            out[i] = invert1(sens[i], g.eps1);
-        }
+__global__ void __launch_bounds__(256) update_image_kernel(const DevGeom g, float4 *__restrict__ image,
+                                                           float4 *__restrict__ corr, const float4 *__restrict__ nf) {
+    int x, y;
+    size_t i;
+    if (!image_voxels(g, x, y, i) || y < g.cyl_lo[x] || y >= g.cyl_hi[x]) return;
+    for (int q = threadIdx.x; q < g.NQ; q += 64, i += 64) {
+        const float4 im = image[i], c = corr[i], n = nf[i];
+        image[i] = make_float4(update1(im.x, c.x, n.x, g.image_max), update1(im.y, c.y, n.y, g.image_max),
+                               update1(im.z, c.z, n.z, g.image_max), update1(im.w, c.w, n.w, g.image_max));
+        corr[i] = f4(0.f);
+    }
 }
 
-__global__ void init_image_kernel(const DevGeom g, float *__restrict__ image, int z_min, int z_max) {
-    const int x = blockIdx.x;
-    for (int y = threadIdx.y; y < g.N; y += blockDim.y)
-        for (int z = threadIdx.x; z < g.Z4; z += blockDim.x) {
-            const bool in = y >= g.cyl_lo[x] && y < g.cyl_hi[x] && z >= z_min && z < z_max;
-            image[((size_t)x * g.N + y) * g.Z4 + z] = in ? 1.0f : 0.0f;
-        }
+__global__ void __launch_bounds__(256) normfac_invert_kernel(const DevGeom g, const float *__restrict__ sens,
+                                                             float *__restrict__ out) {
+    int x, y;
+    size_t i;
+    if (!image_voxels(g, x, y, i) || y < g.cyl_lo[x] || y >= g.cyl_hi[x]) return;
+    const size_t o = ((size_t)x * g.N + y) * g.Z4;
+    for (int z = threadIdx.x; z < g.Z; z += 64) out[o + z] = invert1(sens[o + z], g.eps1);
 }
 
-__global__ void end_iteration_kernel(const DevGeom g, float *__restrict__ image, int z_min, int z_max) {
-    const int x = blockIdx.x;
-    for (int y = g.cyl_lo[x] + threadIdx.y; y < g.cyl_hi[x]; y += blockDim.y)
-        for (int z = z_min + (int)threadIdx.x; z < z_max; z += blockDim.x) {
-            float *v = image + ((size_t)x * g.N + y) * g.Z4 + z;
-            if ((double)*v < 1e-16) *v = 0.0f;
-        }
+__global__ void __launch_bounds__(256) init_image_kernel(const DevGeom g, float *__restrict__ image, int z_min,
+                                                         int z_max) {
+    int x, y;
+    size_t i;
+    if (!image_voxels(g, x, y, i)) return;
+    const bool fov = y >= g.cyl_lo[x] && y < g.cyl_hi[x];
+    for (int z = threadIdx.x; z < g.Z4; z += 64)
+        image[((size_t)x * g.N + y) * g.Z4 + z] = fov && z >= z_min && z < z_max ? 1.0f : 0.0f;
+}
+
+__global__ void __launch_bounds__(256) end_iteration_kernel(const DevGeom g, float *__restrict__ image, int z_min,
+                                                            int z_max) {
+    int x, y;
+    size_t i;
+    if (!image_voxels(g, x, y, i) || y < g.cyl_lo[x] || y >= g.cyl_hi[x]) return;
+    for (int z = z_min + (int)threadIdx.x; z < z_max; z += 64) {
+        float *v = image + ((size_t)x * g.N + y) * g.Z4 + z;
+        if ((double)*v < 1e-16) *v = 0.0f;
+    }
 }
 
 __global__ void fill_u64_kernel(unsigned long long *__restrict__ p, int n) {
@@ -2062,7 +2175,8 @@ hipError_t launch_ratio_w012(const DevGeom &g, float *est, const float *data, hi
 }
 
 hipError_t launch_update_image(const DevGeom &g, float *image, float *corr, const float *nf, hipStream_t s) {
-    hipLaunchKernelGGL(update_image_kernel, dim3(g.N), dim3(64, 4), 0, s, g, image, corr, nf);
+    hipLaunchKernelGGL(update_image_kernel, rot_grid(g), dim3(64, 4), 0, s, g, reinterpret_cast<float4 *>(image),
+                       reinterpret_cast<float4 *>(corr), reinterpret_cast<const float4 *>(nf));
     return hipGetLastError();
 }
 
@@ -2074,14 +2188,21 @@ hipError_t launch_rotate_sum(const DevGeom &g, const PairBatch &b, const float *
 }
 
 hipError_t launch_convolve3d(const DevGeom &g, const float *in, float *out, float *buf, const float *taps_x, int hx,
-                             const float *taps_y, int hy, const float *normz, int z_min, int z_max, hipStream_t s) {
+                             const float *taps_y, int hy, const float *normz, int z_min, int z_max,
+                             const float *normfac, hipStream_t s) {
     if (g.Z4 > 256 || g.NQ > 64 || z_min < 0 || z_max > g.Z) return hipErrorInvalidValue;   // one z column per wave
-    hipLaunchKernelGGL(psf_x_kernel, rot_grid(g), dim3(64, 4), 0, s, g, reinterpret_cast<const float4 *>(in),
-                       reinterpret_cast<float4 *>(buf), taps_x, hx);
+    const int runs = (g.N + PSF_R - 1) / PSF_R, runs4 = (g.N + 4 * PSF_R - 1) / (4 * PSF_R);
+    hipLaunchKernelGGL(psf_x_kernel, dim3(8 * (((g.N + 3) / 4 + 7) / 8) * runs), dim3(64, 4), 0, s, g,
+                       reinterpret_cast<const float4 *>(in), reinterpret_cast<float4 *>(buf), taps_x, hx);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(psf_yz_kernel, rot_grid(g), dim3(64, 4), 0, s, g, reinterpret_cast<const float4 *>(buf), out,
-                       taps_y, hy, normz, z_min, z_max);
+    const int pad = std::min((hy + 3) / 4, g.NQ);      // quads further off lie outside the column
+    const size_t lds = sizeof(float4) * 4 * PSF_R * (g.NQ + 2 * pad);
+    const dim3 grid(8 * ((g.N + 7) / 8) * runs4), block(64, 4);
+    const float4 *b4 = reinterpret_cast<const float4 *>(buf), *nf = reinterpret_cast<const float4 *>(normfac);
+    float4 *o4 = reinterpret_cast<float4 *>(out);
+    if (normfac) hipLaunchKernelGGL(psf_yz_kernel<true>, grid, block, lds, s, g, b4, o4, nf, taps_y, hy, pad, normz, z_min, z_max);
+    else hipLaunchKernelGGL(psf_yz_kernel<false>, grid, block, lds, s, g, b4, o4, nf, taps_y, hy, pad, normz, z_min, z_max);
     return hipGetLastError();
 }
 
@@ -2093,17 +2214,17 @@ hipError_t launch_flat_image(const DevGeom &g, const float *src, float *dst, int
 }
 
 hipError_t launch_normfac_invert(const DevGeom &g, const float *sens, float *out, hipStream_t s) {
-    hipLaunchKernelGGL(normfac_invert_kernel, dim3(g.N), dim3(64, 4), 0, s, g, sens, out);
+    hipLaunchKernelGGL(normfac_invert_kernel, rot_grid(g), dim3(64, 4), 0, s, g, sens, out);
     return hipGetLastError();
 }
 
 hipError_t launch_init_image(const DevGeom &g, float *image, int z_min, int z_max, hipStream_t s) {
-    hipLaunchKernelGGL(init_image_kernel, dim3(g.N), dim3(64, 4), 0, s, g, image, z_min, z_max);
+    hipLaunchKernelGGL(init_image_kernel, rot_grid(g), dim3(64, 4), 0, s, g, image, z_min, z_max);
     return hipGetLastError();
 }
 
 hipError_t launch_end_iteration(const DevGeom &g, float *image, int z_min, int z_max, hipStream_t s) {
-    hipLaunchKernelGGL(end_iteration_kernel, dim3(g.N), dim3(64, 4), 0, s, g, image, z_min, z_max);
+    hipLaunchKernelGGL(end_iteration_kernel, rot_grid(g), dim3(64, 4), 0, s, g, image, z_min, z_max);
     return hipGetLastError();
 }
 
