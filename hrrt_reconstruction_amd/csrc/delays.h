@@ -86,6 +86,7 @@ struct hrrt_delays {
                                              // entry parity, its 64 out-of-sync mask words, its key count
     long long lm_chunk_cap = 0;
     unsigned long long *d_lm_stats = nullptr;
+    unsigned long long *h_lm_stats = nullptr;   // pinned copy of the last call's statistics
 
     // calc_det_to_phy geometry_info.cpp:137-163: block/crystal offsets in float, the head
     // rotation in double, stored as float (constants geometry_info.h:51-55 are floats)

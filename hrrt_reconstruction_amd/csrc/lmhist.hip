@@ -191,7 +191,10 @@ __device__ int chunk_walk(unsigned mask, int entry, unsigned short *sw, int &nsw
     return p & 1;
 }
 
+// Also clears the statistics (workgroup 0), which only later kernels of the call add to.
 __global__ __launch_bounds__(WAVES * 64) void lm_summary_kernel(LmArgs a, long long nchunks) {
+    if (blockIdx.x == 0)
+        for (int i = threadIdx.x; i < ST_WORDS; i += WAVES * 64) a.st[i] = (i == ST_START || i == ST_END) ? NONE : 0ull;
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const long long c = (long long)blockIdx.x * WAVES + wv;
     if (c >= nchunks) return;
@@ -292,7 +295,8 @@ __device__ inline Event decode(const LmArgs &a, unsigned ew1, unsigned ew2) {
     v.bx = (int)(ew2 & 0xff), v.by = (int)((ew2 & 0xff00) >> 8);
     v.doia = a.doi ? (int)((ew1 & 0x01C00000u) >> 22) : 1;
     v.doib = a.doi ? (int)((ew2 & 0x01C00000u) >> 22) : 1;
-    v.bad = v.is_event & ((v.mpe < 1) | (v.mpe > NMP) | (max(v.ax, v.bx) >= NX) | (max(v.ay, v.by) >= NY));
+    const int outside = (int)((unsigned)(v.mpe - 1) >= (unsigned)NMP) | (int)(max(v.ax, v.bx) >= NX) | (int)(max(v.ay, v.by) >= NY);
+    v.bad = v.is_event & (outside != 0);
     const bool ok = v.is_event & !v.bad;
     v.tx = ok & ((v.doia == 7) | (v.doib == 7));
     v.em = ok & !v.tx & (max(v.doia, v.doib) <= 1);
@@ -863,11 +867,6 @@ __global__ void lm_coin_sum_kernel(const unsigned *__restrict__ part, unsigned *
     out[k] = sum;
 }
 
-__global__ void lm_stats_init_kernel(unsigned long long *st) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < ST_WORDS) st[i] = (i == ST_START || i == ST_END) ? NONE : 0ull;
-}
-
 // The module-pair LUT by (module pair, A crystal, B crystal) on the device, and the counts.
 int ensure_lm(hrrt_delays &c, long long nchunks, bool coin) {
     int r = upload(c);
@@ -882,6 +881,7 @@ int ensure_lm(hrrt_delays &c, long long nchunks, bool coin) {
         DTRY(hipMemcpy(c.d_sol, c.lut.data(), sizeof(int3) * c.lut.size(), hipMemcpyHostToDevice));
     }
     if (!c.d_lm_stats) DTRY(hipMalloc(&c.d_lm_stats, sizeof(unsigned long long) * ST_WORDS));
+    if (!c.h_lm_stats) DTRY(hipHostMalloc((void **)&c.h_lm_stats, sizeof(unsigned long long) * ST_WORDS));
     if (!c.d_lm_tiles) {    // first keys of the tiles, then two counters per tile of whole buckets
         const long long S = (long long)c.nplanes * c.nsino, nb = (S + (1ll << BUCKET_BITS) - 1) >> BUCKET_BITS;
         DTRY(hipMalloc(&c.d_lm_tiles, sizeof(unsigned) * (size_t)((S + TILE - 1) / TILE + 1 + 2 * nb * BUCKET_TILES)));
@@ -957,12 +957,10 @@ extern "C" int hrrt_lm_histogram(hrrt_delays *c, const uint32_t *d_words, long l
     a.kcnt = c->d_lm_chunks + 65 * c->lm_chunk_cap;
     a.w16 = (uintptr_t)d_words % 16 == 0;
     a.st = c->d_lm_stats;
-    lm_stats_init_kernel<<<(ST_WORDS + 255) / 256, 256, 0, s>>>(a.st);
-    DTRY(hipGetLastError());
+    const unsigned grid = (unsigned)std::max((nchunks + WAVES - 1) / WAVES, 1ll);
+    lm_summary_kernel<<<grid, WAVES * 64, 0, s>>>(a, nchunks);
     if (nchunks > 0) {
-        const unsigned grid = (unsigned)((nchunks + WAVES - 1) / WAVES);
         const long long npackets = (nchunks + CHUNKS_PER_PACKET - 1) / CHUNKS_PER_PACKET;
-        lm_summary_kernel<<<grid, WAVES * 64, 0, s>>>(a, nchunks);
         lm_resolve_kernel<<<(unsigned)npackets, CHUNKS_PER_PACKET, 0, s>>>(a.chunks, nchunks);
         if (opt->start_ms > 0) lm_window_kernel<0><<<grid, WAVES * 64, 0, s>>>(a, nchunks);
         if (opt->end_ms > 0) lm_window_kernel<1><<<grid, WAVES * 64, 0, s>>>(a, nchunks);
@@ -997,8 +995,8 @@ extern "C" int hrrt_lm_histogram(hrrt_delays *c, const uint32_t *d_words, long l
     }
     DTRY(hipGetLastError());
     if (stats) {
-        std::vector<unsigned long long> h(ST_WORDS);
-        DTRY(hipMemcpyAsync(h.data(), a.st, sizeof(unsigned long long) * ST_WORDS, hipMemcpyDeviceToHost, s));
+        const unsigned long long *h = c->h_lm_stats;
+        DTRY(hipMemcpyAsync(c->h_lm_stats, a.st, sizeof(unsigned long long) * ST_WORDS, hipMemcpyDeviceToHost, s));
         DTRY(hipStreamSynchronize(s));
         memset(stats, 0, sizeof(*stats));
         stats->prompts = (long long)h[ST_PROMPTS];

@@ -519,6 +519,7 @@ extern "C" void hrrt_delays_destroy(hrrt_delays *c) {
                     (void *)c->d_lm_coin_seg, (void *)c->d_lm_coin_cnt, (void *)c->d_lm_coin_part, (void *)c->d_lm_chunks,
                     (void *)c->d_lm_stats})
         if (p) (void)hipFree(p);
+    if (c->h_lm_stats) (void)hipHostFree(c->h_lm_stats);
     delete c;
 }
 
