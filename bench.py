@@ -125,7 +125,7 @@ def write_traffic(fetch_dir, write_dir, launches):
         return rows
 
     kinds = {"fp_ratio": "fp_kernel<3, 2, 1, true>", "backproject": "bp_inc_kernel",
-             "rotate_update": "rot_update_kernel<false>"}
+             "rotate_update": "rot_tile_kernel<false, 0>"}
     cal_bytes = 256 << 20
     out = {}
     scale = {}
@@ -395,7 +395,7 @@ def listmode_leg(torch, events, steps, seed, cpu_events, span):
     log(f"list mode: {events} events in {ms:.2f} ms ({events / ms / 1e6:.2f} G events/s)")
     res = {"events": events, "words": int(words.size), "ms_per_histogram": round(ms, 3),
            "events_per_s": round(events / (ms * 1e-3), 1), "prompts_binned": st["prompts"], "span": span,
-           "note": "whole stream per call: chunk walk, event keys, radix sort by sinogram tile, per-tile counts into int16 bins, statistics", "cpu_baseline": None}
+           "note": "whole stream per call: chunk walk, event keys, partition by sinogram tile, per-tile counts into int16 bins, statistics", "cpu_baseline": None}
     del sino, cp, cd, d
     torch.cuda.empty_cache()
     if cpu_events:
