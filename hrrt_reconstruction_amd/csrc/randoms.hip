@@ -146,8 +146,9 @@ __device__ inline unsigned abs_diff(unsigned a, unsigned b) {
 // thread that stores it.  Columns go bin-major into scratch and through column_transpose_kernel:
 // stores straight into the plane-major output, one 4-byte request each, took 0.35 ms longer at
 // span 9 (2209 planes) and 1 ms at span 3 with maxrd 25.
-// 73728 bins of 6367 planes, 0.41 M LORs: 2.42 ms, the layout by B ring and two-halves conversion
-// 2.78 ms; a pair takes 17 vector instructions (31 before).
+// 73728 bins of 6367 planes, 0.29 M LORs: 2.36 ms (2.42 with a group's segment reads behind the adds of the
+// group before, 2.78 with the layout by B ring and two-halves conversion); a pair takes 17 vector
+// instructions (31 before).  72 registers, for the 7 waves a SIMD of two workgroups per CU.
 constexpr int COL_ROWS = 8, COL_STEPS = NY / COL_ROWS, COL_THREADS = NY * COL_ROWS;
 static_assert(COL_STEPS * COL_ROWS == NY && COL_THREADS % 64 == 0, "rings split evenly");
 constexpr int COL_BINS = 8;     // bins per workgroup (the bin count is a multiple of 8)
@@ -158,7 +159,15 @@ constexpr int MID_PLANE = NY - 1;   // 103
 // Planes of the LDS column (span 3 at maxrd up to 68 has 6367).
 constexpr int COLUMN_PLANES = 6400;
 
-__global__ __launch_bounds__(COL_THREADS) void delays_column_kernel(Tables t, const float *__restrict__ sings,
+template <int NI>
+struct Group {      // pairs between their two stages
+    static constexpr int N = NI;
+    unsigned plane[NI];
+    int2 ent[NI];
+    float b[NI];
+};
+
+__global__ __launch_bounds__(COL_THREADS, 7) void delays_column_kernel(Tables t, const float *__restrict__ sings,
                                                                     const int *__restrict__ scale, float tauftime,
                                                                     float *__restrict__ cols, int cstride) {
     __shared__ int2 seg[128];
@@ -183,7 +192,7 @@ __global__ __launch_bounds__(COL_THREADS) void delays_column_kernel(Tables t, co
     }
     const bool mid = t.window >= MID_WINDOW;
     // this thread's LOR of the first eight of a bin, and its singles
-    int k0 = t.lor_off[first], k1 = t.lor_off[first + 1];
+    int k0 = t.lor_off[first], k1 = t.lor_off[first + 1], n1 = t.lor_off[min(first + 2, end)], sc = scale[first];
     int4 L = make_int4(0, 0, 0, 0);
     float a = 0.0f, b = 0.0f;
     auto load_lor = [&](int k, int kend) { if (k < kend) L = t.lor[k]; };
@@ -191,9 +200,10 @@ __global__ __launch_bounds__(COL_THREADS) void delays_column_kernel(Tables t, co
     load_lor(k0 + row, k1);
     load_sings(k0 + row, k1);
     for (int bin = first; bin < end; bin++) {
-        const int sc = scale[bin], kexp = sc >= 128 ? sc - 256 : sc;
+        const int kexp = sc >= 128 ? sc - 256 : sc;
         const float up = ldexpf(1.0f, kexp);
-        const int n0 = k1, n1 = bin + 1 < end ? t.lor_off[bin + 2] : k1;    // the next bin's LORs
+        // the next bin's LORs are [k1, n1); what the bin after it needs is on its way (beyond the last bin: none)
+        const int n0 = k1, n2 = t.lor_off[min(bin + 3, end)], sc_next = scale[min(bin + 1, end - 1)];
         auto sum = [&](auto finite) __attribute__((always_inline)) {
             for (int kb = k0; kb < k1; kb += COL_ROWS) {
                 if (kb > k0) {
@@ -207,31 +217,38 @@ __global__ __launch_bounds__(COL_THREADS) void delays_column_kernel(Tables t, co
                 sA[row][ay] = a * tauftime;
                 if (ay == 0) sL[row] = make_float2(__int_as_float(L.z), __int_as_float(L.w));
                 __syncthreads();
-                if (kb + COL_ROWS >= k1) {
-                    load_lor(n0 + row, n1);
-                    load_sings(n0 + row, n1);
-                }
+                if (kb + COL_ROWS >= k1) load_lor(n0 + row, n1);
                 const int n = min(COL_ROWS, k1 - kb);
                 for (int k = 0; k < n; k++) {
                     const float sd = sL[k].x, sz = sL[k].y, awt = sA[k][ay];
                     const float *bk = &sB[k][ay + row];
-                    auto steps = [&](auto lo, auto hi) __attribute__((always_inline)) {
-                        constexpr int I0 = decltype(lo)::value, NI = decltype(hi)::value - I0;
+                    // A pair in two stages: its plane, segment entry and B single, then its add.  A group's reads are
+                    // issued before the adds of the group before it, since LDS answers in order.
+                    auto first_stage = [&](auto i0, auto &g) __attribute__((always_inline)) {
+                        constexpr int I0 = decltype(i0)::value;
+#pragma unroll
+                        for (int i = 0; i < g.N; i++) {
+                            const float dzi = dz[I0 + i];
+                            g.plane[i] = (unsigned)(int)(za.y + sz * dzi);
+                            const float s = 0.5f + dzi * sd;
+                            const unsigned j = (unsigned)fminf(fabsf(s), 63.5f);
+                            // byte offset of entry 2 |(int)s| + (s < 0)
+                            const unsigned e8 = __builtin_amdgcn_alignbit(j, __float_as_uint(s), 28) & ~7u;
+                            g.ent[i] = *reinterpret_cast<const int2 *>(reinterpret_cast<const char *>(seg) + e8);
+                            g.b[i] = bk[COL_ROWS * (I0 + i)];
+                        }
+                        asm volatile("" ::: "memory");
+                    };
+                    auto second_stage = [&](auto &g) __attribute__((always_inline)) {
+                        constexpr int NI = std::remove_reference_t<decltype(g)>::N;
                         bool ok[NI];
                         int idx8[NI];
                         unsigned long long q[NI];
 #pragma unroll
                         for (int i = 0; i < NI; i++) {
-                            const float dzi = dz[I0 + i];
-                            const unsigned plane = (unsigned)(int)(za.y + sz * dzi);
-                            const float s = 0.5f + dzi * sd;
-                            const unsigned j = (unsigned)fminf(fabsf(s), 63.5f);
-                            // byte offset of entry 2 |(int)s| + (s < 0)
-                            const unsigned e8 = __builtin_amdgcn_alignbit(j, __float_as_uint(s), 28) & ~7u;
-                            const int2 ent = *reinterpret_cast<const int2 *>(reinterpret_cast<const char *>(seg) + e8);
-                            ok[i] = abs_diff(plane, MID_PLANE) < (unsigned)ent.x;
-                            idx8[i] = (int)(plane << 3) + ent.y;
-                            q[i] = to_fixed<decltype(finite)::value>(bk[COL_ROWS * (I0 + i)] * awt);
+                            ok[i] = abs_diff(g.plane[i], MID_PLANE) < (unsigned)g.ent[i].x;
+                            idx8[i] = (int)(g.plane[i] << 3) + g.ent[i].y;
+                            q[i] = to_fixed<decltype(finite)::value>(g.b[i] * awt);
                         }
                         // whole groups before their adds, or each add would wait for its own chain
 #pragma unroll
@@ -239,28 +256,41 @@ __global__ __launch_bounds__(COL_THREADS) void delays_column_kernel(Tables t, co
 #pragma unroll
                         for (int i = 0; i < NI; i++)
                             if (ok[i]) atomicAdd(reinterpret_cast<unsigned long long *>(reinterpret_cast<char *>(col) + idx8[i]), q[i]);
+                        asm volatile("" ::: "memory");
                     };
-                    steps(std::integral_constant<int, 0>(), std::integral_constant<int, MID_LO>());
-                    if (mid) steps(std::integral_constant<int, MID_LO>(), std::integral_constant<int, MID_HI>());
-                    steps(std::integral_constant<int, MID_HI>(), std::integral_constant<int, COL_STEPS>());
+                    Group<2> ga, gb, gd, ge, gf;
+                    Group<3> gc;
+                    first_stage(std::integral_constant<int, 0>(), ga);
+                    first_stage(std::integral_constant<int, 2>(), gb);
+                    second_stage(ga);
+                    if (mid) {
+                        first_stage(std::integral_constant<int, MID_LO>(), gc);
+                        second_stage(gb);
+                        first_stage(std::integral_constant<int, MID_LO + 3>(), gd);
+                        second_stage(gc);
+                        first_stage(std::integral_constant<int, MID_HI>(), ge);
+                        second_stage(gd);
+                    } else {
+                        first_stage(std::integral_constant<int, MID_HI>(), ge);
+                        second_stage(gb);
+                    }
+                    first_stage(std::integral_constant<int, MID_HI + 2>(), gf);
+                    second_stage(ge);
+                    second_stage(gf);
                 }
             }
         };
-        if (k0 == k1) {
-            load_lor(n0 + row, n1);
-            load_sings(n0 + row, n1);
-        } else if (sc < 128) {
-            sum(std::true_type());
-        } else {
-            sum(std::false_type());
-        }
+        if (k0 == k1) load_lor(n0 + row, n1);
+        else if (sc < 128) sum(std::true_type());
+        else sum(std::false_type());
+        load_sings(n0 + row, n1);       // the LOR has arrived; these arrive while the column is stored
         __syncthreads();
         const double down = ldexp(1.0, -kexp);
         for (int i = tid; i < t.nplanes; i += COL_THREADS) {
             cols[(size_t)bin * cstride + i] = (float)((double)(long long)col[i] * down);
             col[i] = 0ull;
         }
-        k0 = n0, k1 = n1;
+        k0 = n0, k1 = n1, n1 = n2, sc = sc_next;
     }
 }
 
