@@ -94,7 +94,7 @@ __global__ __launch_bounds__(256) void bin_scale_kernel(Tables t, const float *_
         const float a = sings[NCRYS + L.x / NY], b = sings[NCRYS + L.y / NY];
         m = fmaxf(m, a * b);
         mb = fmaxf(mb, b);
-        finite &= a <= 3.0e38f;
+        finite &= a * tauftime <= 3.0e38f;      // the factor itself, and no infinite a (a NaN product counts as not finite)
     }
     m *= tauftime;
     const int k = fixed_point_exponent(m, max(k1 - k0, 1));
