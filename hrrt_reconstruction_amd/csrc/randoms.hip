@@ -449,8 +449,9 @@ int group_lors(hrrt_delays &c) {
                 e.x = ((al * NHEADS + ahead) * NX + ax) * NY;
                 e.y = ((bl * NHEADS + bhead) * NX + bx) * NY;
                 // a slope of zero (a record of zeros in a LUT file) becomes one that leaves 0.5 + dz*d at
-                // 0.5 for every ring difference but not for a pair outside the window
-                const float d = std::fabs(s.d) < 1e-30f ? std::copysign(1e-30f, s.d) : s.d;
+                // 0.5 for every ring difference but not for a pair outside the window; so does one that is no
+                // number, which names segment 0 too
+                const float d = std::fabs(s.d) >= 1e-30f ? s.d : std::copysign(1e-30f, s.d);
                 memcpy(&e.z, &d, 4);
                 memcpy(&e.w, &s.z, 4);
                 lor[fill[s.nsino]++] = e;

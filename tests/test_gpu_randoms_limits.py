@@ -1,5 +1,8 @@
 """Smoothed randoms at the limits of float."""
+import numpy as np
 import pytest
+
+from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -14,3 +17,22 @@ def test_overflowing_factor_of_silent_crystals():
     g = GenDelays(span=9, lr_type=2)
     out = g.smooth(s.reshape(-1), 1e10)                 # tau * T = 60
     assert not out.any().item()
+
+def test_lut_slope_not_a_number(tmp_path):
+    """A record whose slope is NaN names segment 0, as one of slope zero does."""
+    import torch
+    from hrrt_reconstruction_amd.randoms import GenDelays
+    print("randoms NaN slopes", flush=True)
+    rng = np.random.default_rng(4)
+    s = torch.from_numpy(rng.uniform(20.0, 200.0, O.NCRYS).astype(np.float32)).cuda()
+    path = tmp_path / "lut"
+    GenDelays(span=9, lr_type=2).save_lut(str(path))
+    raw = np.fromfile(path, np.float32)
+    slopes = raw[1:20 * 144 * 144 * 3:3]
+    chosen = rng.random(slopes.size) < 0.01
+    out = []
+    for value in (0.0, np.nan):
+        slopes[chosen] = value
+        raw.tofile(path)
+        out.append(GenDelays(span=9, lr_type=2, lut_file=str(path)).smooth(s, 60.0))
+    assert torch.equal(out[0], out[1])
