@@ -645,6 +645,16 @@ extern "C" int hrrt_delays_smooth(hrrt_delays *c, const float *d_singles, float 
     if (r != HRRT_OK) return r;
     DTRY(hipGetDevice(&dev));
     if (dev != c->device) return hrrt_dl::fail(HRRT_ERR_ARG, "context tables live on another device");
+    const int cstride = (c->nplanes + 63) & ~63;
+    if (!c->d_cols) {
+        // The first smoothing may be recorded into a graph (a histogram has uploaded the tables): the allocation
+        // belongs to the context, not to the graph, so it is made whatever the thread's capture mode.
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        DTRY(hipThreadExchangeStreamCaptureMode(&mode));
+        const hipError_t e = hipMalloc(&c->d_cols, sizeof(float) * (size_t)c->nsino * cstride);
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        DTRY(e);
+    }
     const float ftime = scan_duration > 0.0f ? scan_duration : 1.0f;
     const float tauftime = c->tau * ftime;
     Tables t{c->d_lor, c->d_lor_off, c->d_seg_col, c->d_z, c->nsino, c->nplanes, c->maxrd + 5};
@@ -652,8 +662,6 @@ extern "C" int hrrt_delays_smooth(hrrt_delays *c, const float *d_singles, float 
     bin_scale_kernel<<<(c->nsino + 255) / 256, 256, 0, s>>>(t, c->d_sings, tauftime, c->d_scale);
     DTRY(hipGetLastError());
     const unsigned grid = 8 * ((c->nsino / 8 + COL_BINS - 1) / COL_BINS);
-    const int cstride = (c->nplanes + 63) & ~63;
-    if (!c->d_cols) DTRY(hipMalloc(&c->d_cols, sizeof(float) * (size_t)c->nsino * cstride));
     delays_column_kernel<<<grid, COL_THREADS, 0, s>>>(t, c->d_sings, c->d_scale, tauftime, c->d_cols, cstride);
     DTRY(hipGetLastError());
     column_transpose_kernel<<<dim3((c->nplanes + 64 * TT - 1) / (64 * TT), (c->nsino + 63) / 64), 256, 0, s>>>(c->d_cols, d_delays,
