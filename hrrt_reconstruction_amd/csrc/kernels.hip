@@ -2106,7 +2106,9 @@ hipError_t launch_backproject_incremental(const DevGeom &g, const PairBatch &b, 
     // Both bins of a ray in one workgroup share the breakpoints' work (9 pairs at 256 x 256, span 3: 0.346 ms
     // against 0.408 with a bin each); below two such workgroups per CU a bin each fills the chip better (one
     // view pair of that size, forward to image: 0.318 ms against 0.324; a 16-ring subset: 50.6 us against 51.9).
-    if ((long long)g.c * 2 * npf >= 512)
+    // Two bins also take twice the LDS: where a CU's 160 KB hold a single such workgroup, its four waves are too few
+    // (128 rings, 97 ring differences, 83 KB, nine pairs at 256 x 256: 1.20 ms against 0.88 with a bin each).
+    if ((long long)g.c * 2 * npf >= 512 && 2 * g.inc_shm <= 160 * 1024)
         hipLaunchKernelGGL(bp_inc_kernel<2>, dim3(g.c, 2, npf), block, g.inc_shm, s, g, b, src, src_global, apply_rescale,
                            bufA, bufB);
     else
