@@ -186,7 +186,7 @@ struct hrrt_ctx {
                    stream == o.stream && mixed == o.mixed && inv == o.inv && ll == o.ll;
         }
     } gkey;
-    double *ll_part = nullptr;           // FP64 partial sums (log-likelihood, count moments)
+    double *ll_part = nullptr;           // partial sums (LlSum of the log-likelihood, FP64 count moments)
     size_t ll_cap = 0;
     int ensure_ll_part(size_t n) {
         if (n <= ll_cap) return HRRT_OK;
@@ -1085,14 +1085,14 @@ static int frames_subset_launch(hrrt_ctx *ctx, int nframes, float *d_images, con
     io.add = d_adds;
     if (pr.mixed && pr.loglik) {
         io.invnorm = pr.invnorm16;
-        io.ll_part = ctx->ll_part;
+        io.ll_part = reinterpret_cast<hrrt::LlSum *>(ctx->ll_part);
     }
     ctx->mark(0, s);
     HIP_TRY(hrrt::launch_forward(ctx->dg, b, d_images, ctx->f_ratio, io, pr.mixed ? hrrt::FP_RATIO16 : hrrt::FP_RATIO, s));
     if (pr.mixed && pr.loglik) {
         int run, nsplit, threads;
         hrrt::forward_shape(ctx->dg, b.npairs * nframes, run, nsplit, threads);
-        HIP_TRY(hrrt::launch_ll_reduce(ctx->ll_part, ctx->dg.c * nsplit * b.npairs, nframes, pr.loglik, s));
+        HIP_TRY(hrrt::launch_ll_reduce(io.ll_part, ctx->dg.c * nsplit * b.npairs, nframes, pr.loglik, s));
     }
     // the subset update back-projects under the schedule in both forms (incremental by default);
     // the precision form sums the view pairs of the rotation with compensation
@@ -1116,7 +1116,7 @@ static int frames_check(hrrt_ctx *ctx, int nframes, const void *a, const void *b
     if ((r = ctx->ensure_frame_scratch(nframes))) return r;
     int run, nsplit, threads;
     hrrt::forward_shape(ctx->dg, ctx->npairs() * nframes, run, nsplit, threads);
-    return ctx->ensure_ll_part((size_t)ctx->dg.c * nsplit * ctx->npairs() * nframes);
+    return ctx->ensure_ll_part((size_t)ctx->dg.c * nsplit * ctx->npairs() * nframes * (sizeof(hrrt::LlSum) / sizeof(double)));
 }
 
 extern "C" int hrrt_osem_subset_frames(hrrt_ctx *ctx, int nframes, float *d_images, const float *d_normfac_subset,

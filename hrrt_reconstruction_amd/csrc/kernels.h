@@ -73,6 +73,14 @@ struct PairBatch {
     long long buf_stride = 0;            // floats between frames' rotated-frame buffers
 };
 
+// Sum of FP64 log-likelihood terms that is the same in any order, so it depends neither on the launch shape nor on
+// the number of frames: terms below 2^32 as whole parts and fractions in units of 2^-46 (an error of at most
+// 2^-47 a term, that of a term's own rounding at 32), larger ones and those not finite in double.
+struct LlSum {
+    long long whole, frac;
+    double large;
+};
+
 // Per-bin inputs of the forward projector's epilogue.
 //   FP_PLAIN  : projection only (out = scaled estimate)
 //   FP_RATIO  : OP ratio with float additive term (bit-exact path)
@@ -84,7 +92,7 @@ struct FpIO {
     const int16_t *prompt = nullptr;
     const void *add = nullptr;           // float (FP_RATIO, FP_RATIO_W012) or FP16 bits (FP_RATIO16)
     const uint16_t *invnorm = nullptr;   // FP16 1/(N*A) (FP_RATIO16 log-likelihood)
-    double *ll_part = nullptr;           // one partial sum per workgroup (FP_RATIO16)
+    LlSum *ll_part = nullptr;            // one partial sum per workgroup (FP_RATIO16)
 };
 
 hipError_t launch_forward(const DevGeom &g, const PairBatch &b, const float *image, float *out_paircol,
@@ -103,7 +111,7 @@ hipError_t launch_rotate_update(const DevGeom &g, const PairBatch &b, const floa
 hipError_t launch_rotate_sens(const DevGeom &g, const PairBatch &b, const float *bufA, const float *bufB,
                               float *normfac_out, int kahan, hipStream_t s);
 // per-frame sums of the forward projector's log-likelihood partials (fixed order, deterministic)
-hipError_t launch_ll_reduce(const double *part, int per_frame, int nframes, double *out, hipStream_t s);
+hipError_t launch_ll_reduce(const LlSum *part, int per_frame, int nframes, double *out, hipStream_t s);
 hipError_t launch_to_half(const float *in, uint16_t *out, size_t n, hipStream_t s);
 // the same, counting inputs that overflow to +-inf ([0]) and non-zero inputs that become FP16
 // subnormals or zero ([1]) into counts (cleared first by a kernel, so it may be captured)

@@ -34,6 +34,41 @@ __device__ __forceinline__ void kahan_add(float &s, float &c, float x) {
     s = t;
 }
 
+__device__ __forceinline__ void ll_add(LlSum &s, double t) {
+    constexpr double M = 0x1.8p52;                          // v + M holds v, rounded to a whole number, in its low bits
+    constexpr long long MB = 0x4338000000000000ll;
+    if (fabs(t) < 0x1p32) {
+        const double w = t + M;
+        s.whole += __double_as_longlong(w) - MB;
+        s.frac += __double_as_longlong((t - (w - M)) * 0x1p46 + M) - MB;
+    } else {
+        s.large += t;
+    }
+}
+
+// The workgroup's sum, in thread 0 (red: one element per wave)
+__device__ __forceinline__ LlSum ll_block_sum(LlSum s, LlSum *red) {
+    auto add = [&](const LlSum &o) {
+        s.whole += o.whole;
+        s.frac += o.frac;
+        s.large += o.large;
+    };
+    auto carry = [&] {
+        s.whole += s.frac >> 46;
+        s.frac &= (1ll << 46) - 1;
+    };
+    carry();
+    for (int o = 32; o > 0; o >>= 1) add(LlSum{__shfl_xor(s.whole, o), __shfl_xor(s.frac, o), __shfl_xor(s.large, o)});
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < (int)(blockDim.x >> 6); w++) add(red[w]);
+        carry();
+    }
+    return s;
+}
+
 // f(0), f(1), ..., f(N - 1) with the index as a constant
 template <int N, int I = 0, typename F>
 __device__ __forceinline__ void unroll(F &&f) {
@@ -280,7 +315,7 @@ __device__ __forceinline__ void fp_bins_load(const DevGeom &g, int pidx, int cnt
 template <int MODE, int RL>
 __device__ __forceinline__ void fp_bins_write(const DevGeom &g, const float4 (&acc)[RL], float sc, float resc, int pidx,
                                               int cnt, int x, int lp, float *__restrict__ out, const FpIO &io,
-                                              const FpBins<MODE, RL> &b, double &ll) {
+                                              const FpBins<MODE, RL> &b, LlSum &ll) {
 #pragma unroll
     for (int l = 0; l < 4; l++) {
         if ((l & 1) && x == g.c) continue;   // at x == N/2 lanes 1/3 duplicate lanes 0/2
@@ -304,7 +339,7 @@ __device__ __forceinline__ void fp_bins_write(const DevGeom &g, const float4 (&a
                     const float w = __half2float(__ushort_as_half(b.wn[l][j]));
                     if (w > 0.0f && den > g.eps3) {
                         const double mu = (double)den * (double)w;
-                        ll += (pr > 0 ? (double)pr * log(mu) : 0.0) - mu;
+                        ll_add(ll, (pr > 0 ? (double)pr * log(mu) : 0.0) - mu);
                     }
                 }
                 v = q * resc;
@@ -341,12 +376,12 @@ __global__ void __launch_bounds__(1024) fp_kernel(const DevGeom g, const PairBat
     if (MODE == FP_RATIO || MODE == FP_RATIO16) io.prompt += frame * b.sino_stride;
     if (MODE == FP_RATIO || MODE == FP_RATIO_W012) io.add = static_cast<const float *>(io.add) + frame * b.sino_stride;
     else if (MODE == FP_RATIO16) io.add = static_cast<const uint16_t *>(io.add) + frame * b.sino_stride;
-    double ll = 0.0;
+    LlSum ll{};
     const int x = g.c - ray;
     const int view = b.view0 + b.view_stride * lp;
     const int N = g.N, c = g.c;
     if (g.cyl_lo[x] == g.cyl_hi[x] || g.nzmask[view * (c + 1) + x] == 0) {
-        if (MODE == FP_RATIO16 && io.ll_part && threadIdx.x == 0) io.ll_part[L0] = 0.0;
+        if (MODE == FP_RATIO16 && io.ll_part && threadIdx.x == 0) io.ll_part[L0] = LlSum{};
         return;
     }
     const float cosv = g.cos_psi[view], sinv = g.sin_psi[view];
@@ -482,17 +517,8 @@ __global__ void __launch_bounds__(1024) fp_kernel(const DevGeom g, const PairBat
         }
     }
     if (MODE == FP_RATIO16 && io.ll_part) {
-        // workgroup sum of the log-likelihood in a fixed order (waves, then lanes)
-        for (int o = 32; o > 0; o >>= 1) ll += __shfl_xor(ll, o);
-        __syncthreads();
-        double *red = reinterpret_cast<double *>(lds);
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ll;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            double t = 0.0;
-            for (int w = 0; w < (int)(blockDim.x >> 6); w++) t += red[w];
-            io.ll_part[L0] = t;
-        }
+        const LlSum t = ll_block_sum(ll, reinterpret_cast<LlSum *>(lds));
+        if (threadIdx.x == 0) io.ll_part[L0] = t;
     }
 }
 
@@ -1930,7 +1956,7 @@ __global__ void nzmask_kernel(const DevGeom g, const int *__restrict__ colmask, 
 
 // ---------------------------------------------------------------------------
 // FP64 reductions (log-likelihood, count normalisation) and FP16 conversion.
-// Every sum runs in a fixed order, so results are reproducible run to run.
+// Every sum runs in a fixed order or is the same in any, so results are reproducible run to run.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ double block_sum_fixed(double v, double *red) {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
@@ -1943,13 +1969,17 @@ __device__ __forceinline__ double block_sum_fixed(double v, double *red) {
     return t;   // valid in thread 0
 }
 
-__global__ void __launch_bounds__(256) ll_reduce_kernel(const double *__restrict__ part, int per, double *__restrict__ out) {
-    __shared__ double red[4];
-    const double *p = part + (size_t)blockIdx.x * per;
-    double v = 0.0;
-    for (int i = threadIdx.x; i < per; i += blockDim.x) v += p[i];
-    const double t = block_sum_fixed(v, red);
-    if (threadIdx.x == 0) out[blockIdx.x] = t;
+__global__ void __launch_bounds__(256) ll_reduce_kernel(const LlSum *__restrict__ part, int per, double *__restrict__ out) {
+    __shared__ LlSum red[4];
+    const LlSum *p = part + (size_t)blockIdx.x * per;
+    LlSum v{};
+    for (int i = threadIdx.x; i < per; i += blockDim.x) {
+        v.whole += p[i].whole;
+        v.frac += p[i].frac;
+        v.large += p[i].large;
+    }
+    const LlSum t = ll_block_sum(v, red);
+    if (threadIdx.x == 0) out[blockIdx.x] = t.large + ((double)t.whole + (double)t.frac * 0x1p-46);
 }
 
 __global__ void to_half_kernel(const float *__restrict__ in, uint16_t *__restrict__ out, size_t n) {
@@ -2145,7 +2175,7 @@ hipError_t launch_rotate_sens(const DevGeom &g, const PairBatch &b, const float 
     return hipGetLastError();
 }
 
-hipError_t launch_ll_reduce(const double *part, int per_frame, int nframes, double *out, hipStream_t s) {
+hipError_t launch_ll_reduce(const LlSum *part, int per_frame, int nframes, double *out, hipStream_t s) {
     hipLaunchKernelGGL(ll_reduce_kernel, dim3(nframes), dim3(256), 0, s, part, per_frame, out);
     return hipGetLastError();
 }

@@ -233,7 +233,8 @@ int hrrt_calculate_normfac_mixed(hrrt_ctx *ctx, const uint16_t *d_invnorm16, flo
 /* hrrt_osem_subset with FP16 additive term.  When d_loglik is not NULL, *d_loglik
  * (device double) receives sum over the subset's bins of y*log(mu) - mu with
  * mu = (est + add) * w, w = FP16 1/(N*A) (d_invnorm16, shared by all frames), at the
- * image before the update, summed in FP64 in a fixed order. */
+ * image before the update, each term in FP64, their sum the same in any order: it depends neither on
+ * the launch shape nor on the frames beside it. */
 int hrrt_osem_subset_mixed(hrrt_ctx *ctx, float *d_image, const float *d_normfac_subset, const int16_t *d_prompt,
                            const uint16_t *d_add16, const uint16_t *d_invnorm16, int isubset, double *d_loglik,
                            void *stream);
