@@ -154,6 +154,21 @@ struct hrrt_ctx {
         HIP_TRY(hipMemset(*p, 0, bytes));
         return HRRT_OK;
     }
+    // d.rot_box, once d's positions and tiles are on the device
+    int rotation_boxes() {
+        const size_t n = (size_t)(geo.views / 2) * dg.rot_ntiles;
+        hrrt::RotBox *p = nullptr;
+        if (hipMalloc(&p, sizeof(hrrt::RotBox) * (n + 1)) != hipSuccess)
+            return fail(HRRT_ERR_NOMEM, "hipMalloc of a geometry table failed");
+        allocs.push_back(p);
+        int *wide = &p[n].x, view = 0;      // behind the boxes: 1 + a view with a tile too large for its box
+        HIP_TRY(hipMemset(wide, 0, sizeof(int)));
+        HIP_TRY(hrrt::launch_rot_boxes(dg, p, wide, nullptr));
+        HIP_TRY(hipMemcpy(&view, wide, sizeof(int), hipMemcpyDeviceToHost));
+        if (view) return fail(HRRT_ERR_ARG, "rotated tile larger than its box (view %d)", view - 1);
+        dg.rot_box = p;
+        return HRRT_OK;
+    }
     size_t vol_floats() const { return (size_t)geo.N * geo.N * geo.z4; }
     size_t col_floats() const { return (size_t)2 * geo.N * geo.spp; }
     int npairs() const { return geo.sviews / 2; }
@@ -377,8 +392,8 @@ extern "C" int hrrt_create(const hrrt_params *params, hrrt_ctx **out) {
             }
         }
     }
-    // tiles of the batched rotation, four rows of them at a time so that a run of the list is compact, and the
-    // box of each FOV tile's sample positions
+    // tiles of the batched rotation, four rows of them at a time so that a run of the list is compact (the box of
+    // each FOV tile's sample positions is found on the device, from the uploaded positions)
     std::vector<int> rtiles, rempty;
     const int side = (N + hrrt::ROT_TILE - 1) / hrrt::ROT_TILE;
     for (int t0 = 0; t0 < side; t0 += 4)
@@ -389,34 +404,7 @@ extern "C" int hrrt_create(const hrrt_params *params, hrrt_ctx **out) {
                     fov |= std::max(G.cyl_lo[x], ty * hrrt::ROT_TILE) < std::min(G.cyl_hi[x], (ty + 1) * hrrt::ROT_TILE);
                 (fov ? rtiles : rempty).push_back(tx | ty << 16);
             }
-    const int rot_ntiles = (int)rtiles.size();
-    std::vector<hrrt::RotBox> rbox((size_t)(G.views / 2) * rot_ntiles, hrrt::RotBox{});
-    for (int v = 0; v < G.views / 2; v++)
-        for (int t = 0; t < rot_ntiles; t++) {
-            hrrt::RotBox &r = rbox[(size_t)v * rot_ntiles + t];
-            const int x0 = (rtiles[t] & 0xffff) * hrrt::ROT_TILE, y0 = (rtiles[t] >> 16) * hrrt::ROT_TILE;
-            auto each = [&](auto f) {       // the positions whose neighbours the kernel reads
-                for (int x = x0; x < std::min(N, x0 + hrrt::ROT_TILE); x++)
-                    for (int y = std::max(G.cyl_lo[x], y0); y < std::min(G.cyl_hi[x], y0 + hrrt::ROT_TILE); y++) {
-                        const float2 p = rot[((size_t)v * N + x) * N + y];
-                        const int xi = (int)p.x, yi = (int)p.y;
-                        if (xi >= 0 && xi <= N - 2 && yi >= 0 && yi <= N - 2) f(xi, yi);
-                    }
-            };
-            int xhi = 0, yhi = 0;
-            r.x = r.y = N;
-            each([&](int x, int y) { r.x = std::min(r.x, x), r.y = std::min(r.y, y), xhi = std::max(xhi, x + 1), yhi = std::max(yhi, y + 1); });
-            if (xhi - r.x >= hrrt::ROT_BOX || yhi - r.y >= hrrt::ROT_BOX) {
-                delete ctx;
-                return fail(HRRT_ERR_ARG, "rotated tile larger than its box (view %d)", v);
-            }
-            each([&](int x, int y) {
-                for (int i : {0, 1, hrrt::ROT_BOX, hrrt::ROT_BOX + 1}) {
-                    const int c = (x - r.x) * hrrt::ROT_BOX + y - r.y + i;
-                    r.mask[c >> 5] |= 1u << (c & 31);
-                }
-            });
-        }
+    d.rot_ntiles = (int)rtiles.size();
     rtiles.insert(rtiles.end(), rempty.begin(), rempty.end());
     // forward-projector planes.  A plane's axial sample positions for row y are
     // base + (y - c) * tan and base + (c - y) * tan, truncated, plus delta: end planes use
@@ -657,8 +645,8 @@ extern "C" int hrrt_create(const hrrt_params *params, hrrt_ctx **out) {
         (r = ctx->upload(G.seg_data, d.seg_data)) || (r = ctx->upload(G.segment_offset, d.segment_offset)) ||
         (r = ctx->upload(file_seg, d.file_seg)) || (r = ctx->upload(G.bp_rescale, d.bp_rescale)) ||
         (r = ctx->upload(resc, d.rescalearray)) || (r = ctx->upload(blut, d.bp_lut)) ||
-        (r = ctx->upload(rot, d.rot)) || (r = ctx->upload(rtiles, d.rot_tiles)) || (r = ctx->upload(rbox, d.rot_box)) ||
-         (r = ctx->upload(fruns[0], d.fp_runs[0])) ||
+        (r = ctx->upload(rot, d.rot)) || (r = ctx->upload(rtiles, d.rot_tiles)) || (r = ctx->rotation_boxes()) ||
+        (r = ctx->upload(fruns[0], d.fp_runs[0])) ||
         (r = ctx->upload(fruns[1], d.fp_runs[1])) || (r = ctx->upload(fsingle, d.fp_single)) || (r = ctx->upload(pseg, d.pseg)) ||
         (r = ctx->upload(stage_plane, d.stage_plane)) || (r = ctx->upload(bp_src, d.bp_src)) ||
         (r = ctx->upload(blut2, d.bp_lut2)) || (r = ctx->upload(ichunk, d.inc_chunk)) ||
@@ -669,7 +657,6 @@ extern "C" int hrrt_create(const hrrt_params *params, hrrt_ctx **out) {
     }
     for (int n = 0; n < 2; n++) d.fp_nr[n] = (int)fruns[n].size();
     d.fp_ns = (int)fsingle.size();
-    d.rot_ntiles = rot_ntiles;
     d.fp_fast = fp_fast;
     d.fp_maxt = 0;
     d.fp_nsplit = 0;

@@ -140,6 +140,9 @@ hipError_t launch_rotate_sum(const DevGeom &g, const PairBatch &b, const float *
 hipError_t launch_convolve3d(const DevGeom &g, const float *in, float *out, float *buf, const float *taps_x, int hx,
                              const float *taps_y, int hy, const float *normz, int z_min, int z_max,
                              const float *normfac, hipStream_t s);
+// boxes [views/2][rot_ntiles] of the FOV tiles' sample positions from g.rot and g.rot_tiles; *wide becomes 1 + a view
+// with a tile that does not fit its box, if there is one
+hipError_t launch_rot_boxes(const DevGeom &g, RotBox *boxes, int *wide, hipStream_t s);
 hipError_t launch_init_image(const DevGeom &g, float *image, int z_min, int z_max, hipStream_t s);
 hipError_t launch_end_iteration(const DevGeom &g, float *image, int z_min, int z_max, hipStream_t s);
 // Segments [th0, th0 + nth) (their file blocks must be in place), written to the padded planes
