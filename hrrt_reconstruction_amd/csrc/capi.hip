@@ -1253,7 +1253,7 @@ extern "C" int hrrt_count_moments(hrrt_ctx *ctx, const float *d_image, const int
 
 extern "C" int hrrt_set_launch_shape(hrrt_ctx *ctx, int fp_tasks_per_thread, int fp_workgroups_per_ray) {
     if (!ctx) return fail(HRRT_ERR_ARG, "null context");
-    if (fp_tasks_per_thread < 1 || fp_tasks_per_thread > 4 || fp_workgroups_per_ray < 0 || fp_workgroups_per_ray > 64)
+    if (fp_tasks_per_thread < 0 || fp_tasks_per_thread > 4 || fp_workgroups_per_ray < 0 || fp_workgroups_per_ray > 64)
         return fail(HRRT_ERR_ARG, "launch shape out of range");
     ctx->dg.fp_maxt = fp_tasks_per_thread;
     ctx->dg.fp_nsplit = fp_workgroups_per_ray;

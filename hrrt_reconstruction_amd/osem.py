@@ -450,6 +450,7 @@ class Osem3D(Layout):
     KERNELS = ("fp_ratio", "backproject", "rotate_update")
 
     def set_launch_shape(self, tasks_per_thread: int, workgroups_per_ray: int = 0):
+        """The forward projector's launch shape; (0, 0) leaves it to each launch, as in a new context."""
         _lib.call("hrrt_set_launch_shape", self.ctx, int(tasks_per_thread), int(workgroups_per_ray))
 
     def set_backproject_shape(self, waves_per_workgroup: int):

@@ -264,8 +264,8 @@ int hrrt_count_moments(hrrt_ctx *ctx, const float *d_image, const int16_t *d_pro
  * by the autotuner): the planes of one ray column are split over
  * `fp_workgroups_per_ray` workgroups (0 = as many as the number of rays asks for, at most
  * 1024 threads each), and a thread takes one middle plane (`fp_tasks_per_thread` 1
- * or 2) or a run of three (3 or 4).  Until this is called the library chooses by the
- * number of rays and planes.  Results do not depend on the shape. */
+ * or 2) or a run of three (3 or 4).  0 tasks, as before any call: each launch takes what
+ * suits its number of rays and planes.  Results do not depend on the shape. */
 int hrrt_set_launch_shape(hrrt_ctx *ctx, int fp_tasks_per_thread, int fp_workgroups_per_ray);
 /* Workgroup size of the back projector in 64-lane waves (1..16; no counterpart in
  * the reference).  Each wave evaluates one voxel row of the column the
