@@ -953,75 +953,10 @@ __global__ void __launch_bounds__(256, NB == 2 ? 3 : 6) bp_inc_kernel(const DevG
 }
 
 // ---------------------------------------------------------------------------
-// Rotation (rotateimage2 PJ:1137-1186) of R = A + B of every pair of the
+// Rotation (rotateimage2 PJ:1137-1186) of R = A + B of every pair of a
 // batch, accumulated in pair order, fused with the image update
-// (pt_cal_updateimage S3:2033-2056).  Block (64, 4): x lanes over z chunks of 4.
+// (pt_cal_updateimage S3:2033-2056); a single pair added to an image further down.
 // ---------------------------------------------------------------------------
-// One pair's bilinear neighbourhood of R = A + B at the rotated position of (x, y):
-// the eight loads are issued here and consumed one pair later.
-struct RotTap {
-    float4 a1, a2, a3, a4, b1, b2, b3, b4;
-    float x1, y1;
-    bool ok;
-};
-
-__device__ __forceinline__ void rot_issue(const DevGeom &g, const float4 *__restrict__ A,
-                                          const float4 *__restrict__ B, int lp, float2 pnt, int q, RotTap &t) {
-    const int N = g.N, NQ = g.NQ;
-    const int xi = (int)pnt.x, yi = (int)pnt.y;
-    t.ok = !(xi < 0 || xi > N - 2 || yi < 0 || yi > N - 2);
-    t.x1 = pnt.x - xi;
-    t.y1 = pnt.y - yi;
-    const int xc = t.ok ? xi : 0, yc = t.ok ? yi : 0;      // in-bounds reads for a skipped pair
-    const size_t base = (size_t)lp * N * N * NQ + q;
-    const size_t i1 = base + ((size_t)xc * N + yc) * NQ, i2 = base + ((size_t)(xc + 1) * N + yc) * NQ;
-    t.a1 = A[i1]; t.b1 = B[i1];
-    t.a2 = A[i2]; t.b2 = B[i2];
-    t.a3 = A[i1 + NQ]; t.b3 = B[i1 + NQ];
-    t.a4 = A[i2 + NQ]; t.b4 = B[i2 + NQ];
-}
-
-// Sum over the batch's pairs, in pair order, of the bilinear interpolation of R = A + B
-// at the position the reference's rotation table gives (x, y) for the pair's view.
-// Software-pipelined: the table entry two pairs ahead and the neighbourhood one pair
-// ahead are in flight while a pair is accumulated.
-template <bool KAHAN>
-__device__ __forceinline__ float4 rotate_accumulate(const DevGeom &g, const PairBatch &b,
-                                                    const float4 *__restrict__ A, const float4 *__restrict__ B,
-                                                    int x, int y, int q) {
-    const int N = g.N;
-    const size_t vstride = (size_t)N * N * b.view_stride;
-    const float2 *rt = g.rot + ((size_t)b.view0 * N + x) * N + y;
-    float4 corr = f4(0.f), comp = f4(0.f);
-    RotTap cur, nxt;
-    float2 pn = b.npairs > 1 ? rt[vstride] : make_float2(0.f, 0.f);
-    rot_issue(g, A, B, 0, rt[0], q, cur);
-    for (int lp = 0; lp < b.npairs; lp++) {
-        if (lp + 1 < b.npairs) {
-            const float2 p = pn;
-            if (lp + 2 < b.npairs) pn = rt[vstride * (lp + 2)];
-            rot_issue(g, A, B, lp + 1, p, q, nxt);
-        }
-        if (cur.ok) {
-            const float x1 = cur.x1, y1 = cur.y1;
-            const float w1 = (1 - x1) * (1 - y1), w2 = x1 * (1 - y1), w3 = y1 * (1 - x1), w4 = y1 * x1;
-            const float4 m1 = add4(cur.a1, cur.b1), m2 = add4(cur.a2, cur.b2);
-            const float4 m3 = add4(cur.a3, cur.b3), m4 = add4(cur.a4, cur.b4);
-            const float4 v = add4(add4(mul4(m1, w1), mul4(m2, w2)), add4(mul4(m3, w3), mul4(m4, w4)));
-            if (KAHAN) {
-                kahan_add(corr.x, comp.x, v.x);
-                kahan_add(corr.y, comp.y, v.y);
-                kahan_add(corr.z, comp.z, v.z);
-                kahan_add(corr.w, comp.w, v.w);
-            } else {
-                corr = add4(corr, v);
-            }
-        }
-        cur = nxt;
-    }
-    return corr;
-}
-
 __device__ __forceinline__ float update1(float img, float corr, float nf, float image_max) {
     const float amin = 0.01f, amax = 100.00f;
     float cl = amin > corr ? amin : corr;   // _mm_max_ps(amin, corr)
@@ -1412,15 +1347,27 @@ __global__ void __launch_bounds__(256) flat_image_kernel(const DevGeom g, const 
     }
 }
 
+// ima += the rotation of one view pair's R = A + B: the bilinear interpolation at the position that the reference's
+// rotation table gives (x, y) for the view.  Block (64, 4): x lanes over z chunks of 4.
 __global__ void __launch_bounds__(256) rot_add_kernel(const DevGeom g, int view, const float4 *__restrict__ A,
                                                       const float4 *__restrict__ B, float4 *__restrict__ ima) {
     int x, yg;
-    rot_block(blockIdx.x, g.N, (g.N + 3) / 4, x, yg);
+    const int N = g.N, NQ = g.NQ;
+    rot_block(blockIdx.x, N, (N + 3) / 4, x, yg);
     const int q = threadIdx.x, y = yg * blockDim.y + threadIdx.y;
-    if (q >= g.NQ || y < g.cyl_lo[x] || y >= g.cyl_hi[x]) return;
-    PairBatch b{view, 0, 1};
-    const float4 r = rotate_accumulate<false>(g, b, A, B, x, y, q);
-    const size_t i = ((size_t)x * g.N + y) * g.NQ + q;
+    if (q >= NQ || y < g.cyl_lo[x] || y >= g.cyl_hi[x]) return;
+    const float2 p = g.rot[((size_t)view * N + x) * N + y];
+    const int xi = (int)p.x, yi = (int)p.y;
+    float4 r = f4(0.f);
+    if (!(xi < 0 || xi > N - 2 || yi < 0 || yi > N - 2)) {
+        const float x1 = p.x - xi, y1 = p.y - yi;
+        const float w1 = (1 - x1) * (1 - y1), w2 = x1 * (1 - y1), w3 = y1 * (1 - x1), w4 = y1 * x1;
+        const size_t i1 = ((size_t)xi * N + yi) * NQ + q, i2 = i1 + (size_t)N * NQ;
+        const float4 m1 = add4(A[i1], B[i1]), m2 = add4(A[i2], B[i2]);
+        const float4 m3 = add4(A[i1 + NQ], B[i1 + NQ]), m4 = add4(A[i2 + NQ], B[i2 + NQ]);
+        r = add4(r, add4(add4(mul4(m1, w1), mul4(m2, w2)), add4(mul4(m3, w3), mul4(m4, w4))));
+    }
+    const size_t i = ((size_t)x * N + y) * NQ + q;
     ima[i] = add4(ima[i], r);
 }
 
