@@ -169,11 +169,20 @@ __device__ unsigned chunk_mask_word(const unsigned *__restrict__ w, long long cs
 // (may be null), their number to nsw; returns the parity it leaves with.  All of it is scalar: a
 // ballot says which mask words hold any, so a chunk without them costs a few instructions (one
 // lane searching the 32 words of its parity in LDS took 40 us of a 40 M word stream's 80).
-__device__ int chunk_walk(unsigned mask, int entry, unsigned short *sw, int &nsw, int lane) {
+// RUNS: the chunk has 64 out-of-sync words in a row from a multiple of 64 (a stream's zero tail), which are
+// taken at once (8 M zero words: 0.38 ms, 1.51 one by one).
+template <bool RUNS>
+__device__ __forceinline__ int chunk_steps(unsigned mask, unsigned runs, int entry, unsigned short *sw, int &nsw, int lane) {
     const unsigned long long some = __ballot(mask != 0);
     int p = entry;
     nsw = 0;
     while (p < CHUNK) {
+        if (RUNS && (p & 63) == 0 && (runs >> (p >> 6)) & 1) {
+            if (sw) sw[nsw + lane] = (unsigned short)(p + lane);
+            nsw += 64;
+            p += 64;
+            continue;
+        }
         const int par = p & 1, k = p >> 1;
         int wi = k >> 5;
         unsigned m = (unsigned)__builtin_amdgcn_readlane((int)mask, par * 32 + wi) & (~0u << (k & 31));
@@ -189,6 +198,11 @@ __device__ int chunk_walk(unsigned mask, int entry, unsigned short *sw, int &nsw
         p = pos + 1;
     }
     return p & 1;
+}
+__device__ int chunk_walk(unsigned mask, int entry, unsigned short *sw, int &nsw, int lane) {
+    const unsigned long long full = __ballot(mask == ~0u);
+    const unsigned runs = (unsigned)full & (unsigned)(full >> 32);      // bit w: words 64 w .. 64 w + 63
+    return runs ? chunk_steps<true>(mask, runs, entry, sw, nsw, lane) : chunk_steps<false>(mask, 0u, entry, sw, nsw, lane);
 }
 
 // Also clears the statistics (workgroup 0), which only later kernels of the call add to.
