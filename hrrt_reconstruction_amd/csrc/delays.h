@@ -62,6 +62,7 @@ struct hrrt_delays {
     int nlor = 0, device = 0;
     std::vector<int4> h_lor;                 // LORs grouped by bin (device copy d_lor)
     std::vector<int> h_lor_off;
+    bool uploaded = false;                   // every table of hrrt_dl::upload is on the device
     int4 *d_lor = nullptr;
     int *d_lor_off = nullptr;
     int2 *d_seg = nullptr;

@@ -925,6 +925,7 @@ int ensure_lm(hrrt_delays &c, long long nchunks, bool coin) {
     if (nchunks > c.lm_chunk_cap) {
         if (c.d_lm_chunks) DTRY(hipFree(c.d_lm_chunks));
         c.d_lm_chunks = nullptr;
+        c.lm_chunk_cap = 0;
         DTRY(hipMalloc(&c.d_lm_chunks, sizeof(unsigned) * 66 * (size_t)nchunks));   // summaries, masks, key counts
         c.lm_chunk_cap = nchunks;
     }

@@ -487,7 +487,7 @@ int hrrt_dl::fail(int code, const std::string &msg) { return hrrt::set_last_erro
 
 // Device copies of the tables, on the current device, at the first smoothing.
 int hrrt_dl::upload(hrrt_delays &c) {
-    if (c.d_lor) return HRRT_OK;
+    if (c.uploaded) return HRRT_OK;
     const std::vector<int4> &lor = c.h_lor;
     const std::vector<int> &count = c.h_lor_off;
     // segment entries by e = 2*(int)seg + (seg < 0) + 64 (the kernel's index): e - 64 even and
@@ -502,19 +502,22 @@ int hrrt_dl::upload(hrrt_delays &c) {
     for (int code = 0; code < c.nsegs; code++) seg_col[code] = make_int2(MID_PLANE + 1 - c.segz0[code], 8 * c.segoff[code]);
     std::vector<float2> z(NY);
     for (int i = 0; i < NY; i++) z[i] = make_float2(c.zpos[i], c.zpos2[i]);
-    DTRY(hipGetDevice(&c.device));
-    DTRY(hipMalloc(&c.d_lor, sizeof(int4) * lor.size()));
-    DTRY(hipMalloc(&c.d_lor_off, sizeof(int) * count.size()));
-    DTRY(hipMalloc(&c.d_seg, sizeof(int2) * 128));
-    DTRY(hipMalloc(&c.d_seg_col, sizeof(int2) * 128));
-    DTRY(hipMalloc(&c.d_scale, sizeof(int) * c.nsino));
-    DTRY(hipMalloc(&c.d_z, sizeof(float2) * NY));
-    DTRY(hipMalloc(&c.d_sings, sizeof(float) * (NCRYS + NCOLS)));
-    DTRY(hipMemcpy(c.d_lor, lor.data(), sizeof(int4) * lor.size(), hipMemcpyHostToDevice));
-    DTRY(hipMemcpy(c.d_lor_off, count.data(), sizeof(int) * count.size(), hipMemcpyHostToDevice));
-    DTRY(hipMemcpy(c.d_seg, seg.data(), sizeof(int2) * 128, hipMemcpyHostToDevice));
-    DTRY(hipMemcpy(c.d_seg_col, seg_col.data(), sizeof(int2) * 128, hipMemcpyHostToDevice));
-    DTRY(hipMemcpy(c.d_z, z.data(), sizeof(float2) * NY, hipMemcpyHostToDevice));
+    int dev = -1;
+    DTRY(hipGetDevice(&dev));
+    if (c.d_lor && dev != c.device) return hrrt_dl::fail(HRRT_ERR_ARG, "context tables live on another device");
+    c.device = dev;
+    auto table = [](auto *&dst, size_t bytes, const void *src) {     // a table that an earlier, failed upload left is kept
+        const hipError_t e = dst ? hipSuccess : hipMalloc(&dst, bytes);
+        return e == hipSuccess && src ? hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice) : e;
+    };
+    DTRY(table(c.d_lor, sizeof(int4) * lor.size(), lor.data()));
+    DTRY(table(c.d_lor_off, sizeof(int) * count.size(), count.data()));
+    DTRY(table(c.d_seg, sizeof(int2) * 128, seg.data()));
+    DTRY(table(c.d_seg_col, sizeof(int2) * 128, seg_col.data()));
+    DTRY(table(c.d_scale, sizeof(int) * c.nsino, nullptr));
+    DTRY(table(c.d_z, sizeof(float2) * NY, z.data()));
+    DTRY(table(c.d_sings, sizeof(float) * (NCRYS + NCOLS), nullptr));
+    c.uploaded = true;
     return HRRT_OK;
 }
 
