@@ -110,7 +110,7 @@ hipError_t launch_rotate_update(const DevGeom &g, const PairBatch &b, const floa
                                 float *image, const float *normfac, int kahan, hipStream_t s);
 hipError_t launch_rotate_sens(const DevGeom &g, const PairBatch &b, const float *bufA, const float *bufB,
                               float *normfac_out, int kahan, hipStream_t s);
-// per-frame sums of the forward projector's log-likelihood partials (fixed order, deterministic)
+// per-frame sums of the forward projector's log-likelihood partials
 hipError_t launch_ll_reduce(const LlSum *part, int per_frame, int nframes, double *out, hipStream_t s);
 hipError_t launch_to_half(const float *in, uint16_t *out, size_t n, hipStream_t s);
 // the same, counting inputs that overflow to +-inf ([0]) and non-zero inputs that become FP16

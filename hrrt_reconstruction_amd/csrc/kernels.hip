@@ -236,8 +236,8 @@ __device__ __forceinline__ void rot_block(int bid, int N, int NYG, int &x, int &
 // 4 (RL + 1) LDS reads of 16 bytes in place of 8 RL.  End planes and axial
 // planes go one per thread (single).
 //
-// What bounds it: LDS reads and FP32 VALU, about equally (span 3, 9 view pairs at 256 x 256: 16 runs
-// and 5 singles of 64 lanes per row).  With one plane per thread slot and 8 reads per plane the LDS alone
+// What bounds it: LDS reads and FP32 VALU, about equally (span 3, 9 view pairs at 256 x 256: 16 runs and 5 singles
+// of 64 lanes per row; LDS busy for 52 % of the time, VALU for 54 % at 2.2 cycles an instruction).  With one plane per thread slot and 8 reads per plane the LDS alone
 // took 2 of the 2.9 thousand cycles of a row.  RL = 3 is odd, so the 16 lanes of a quarter-wave read
 // 16 different bank groups, and its sums fit 128 registers with 16 waves in a CU: 0.69 -> 0.586 ms for
 // such a subset.  The samples of a step are loaded a whole step ahead and stored at its beginning,
@@ -676,10 +676,10 @@ __global__ void __launch_bounds__(1024) bp_kernel(const DevGeom g, const PairBat
 // hit the window's zero cells and add +0.
 //
 // What bounds it (9 pairs at 256 x 256, span 3, 0.346 ms; 0.435 with one bin per workgroup, scalar loads of the
-// records and table-driven staging): VALU issue (149 M wave instructions, 78 % of the SIMDs' time at
-// four cycles each), then the 0.7 GB of halves written, which alone take 0.11 ms. Two bins per thread share a
-// breakpoint's record, addresses and reads; its cells are read while the one before is applied, across the
-// rows; the longest columns start first.
+// records and table-driven staging): the chains of sums of the three waves a SIMD holds (149 M vector instructions, one
+// per 5.7 cycles and SIMD where independent additions go one per 2.2; LDS busy for 18 % of the time), then the 0.7 GB
+// of halves written, which alone take 0.11 ms. Two bins per thread share a breakpoint's record, addresses and
+// reads; its cells are read while the one before is applied, across the rows; the longest columns start first.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
@@ -973,10 +973,10 @@ __device__ __forceinline__ float invert1(float s, float eps1) { return fabsf(s) 
 // when both buffers lie in the last-level cache).  Here a tile's columns in the rotated frame are read
 // once per pair, summed as A + B, and kept in LDS, double buffered: the next pair's columns are
 // loaded while a pair is accumulated.  They lie in a box of 12 x 12 for a tile of 8 x 8; a mask says which
-// of the box a voxel touches (some 86 of 120).  Tiles and boxes come from the host (rot_tiles: those
-// with a FOV voxel first, strip by strip so that an XCD's share of them is compact; rot_box).
-// Nine pairs, 256 x 256 x 207: 300 -> 235 us; eight frames of eight pairs, 128 x 128: 310 -> 259 us, where
-// reading A and B once takes 264 at the rate of a copy.
+// of the box a voxel touches (at most 91 of the 144, 79 on average).  The tiles come from the host (rot_tiles: those
+// with a FOV voxel first, strip by strip so that an XCD's share of them is compact), the boxes from rot_box_kernel.
+// Nine pairs, 256 x 256 x 207: 300 -> 235 us for 0.81 GB (the FOV of A, B, image and factors once each); eight
+// frames of four pairs, 128 x 128: 310 -> 259 us for 0.78 GB.
 //   ROT_UPDATE  the image update with the sum;  ROT_SUM  the sum itself (rotate_image_buf into a zeroed
 //   correction, PJ:1701-1725);  ROT_SENS  its inverse, and zeros outside the FOV (all tiles)
 enum RotMode { ROT_UPDATE, ROT_SUM, ROT_SENS };
@@ -1489,8 +1489,8 @@ __global__ void ratio_w012_kernel(const DevGeom g, float *__restrict__ est, cons
     }
 }
 
-// The voxelwise image kernels take four columns a workgroup, a wave each, four planes a lane (a
-// workgroup per x left 3/4 of the chip's wavefronts empty: 121 us for the update of a 256 x 256 x 207 image,
+// The voxelwise image kernels take four columns a workgroup, a wave each; a lane takes the 16 bytes of a quad at a
+// time in the update, a plane at a time in the others (a workgroup per x left 3/4 of the chip's wavefronts empty: 121 us for the update of a 256 x 256 x 207 image,
 // 35 us for the end of an iteration at 128 x 128).
 __device__ __forceinline__ bool image_voxels(const DevGeom &g, int &x, int &y, size_t &i) {
     int yg;

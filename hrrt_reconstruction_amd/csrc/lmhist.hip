@@ -997,7 +997,8 @@ extern "C" int hrrt_lm_histogram(hrrt_delays *c, const uint32_t *d_words, long l
     lm_tile_count_kernel<<<slices, PART_THREADS, 0, s>>>(by_bucket, totals, nbuckets, tcount);
     lm_tile_scatter_kernel<<<slices, PART_THREADS, 0, s>>>(by_bucket, totals, nbuckets, tcount, used, ntiles, by_tile, c->d_lm_tiles);
     DTRY(hipGetLastError());
-    const unsigned tgrid = (unsigned)std::min(ntiles, 1024ll);   // every workgroup resident (4 per CU)
+    // four workgroups per CU, all resident (two are in mode 1, whose counters take twice the LDS; the others follow)
+    const unsigned tgrid = (unsigned)std::min(ntiles, 1024ll);
     const bool both = opt->mode == 1;
     const int vec = (uintptr_t)d_sino % 16 == 0 &&
                     (!both || (d_delayed ? (uintptr_t)d_delayed % 16 == 0 : S % 8 == 0));
