@@ -18,7 +18,7 @@ from __future__ import annotations
 
 # (0, 0) leaves both numbers to each launch's count of rays and planes; the others fix them for every call
 CANDIDATES = [(0, 0), (1, 0), (1, 3), (1, 4), (1, 6), (3, 0), (3, 2), (3, 3)]
-BY_RULE_MARGIN = 0.02
+BY_RULE_MARGIN = 0.05
 
 
 def _choose(results):
@@ -74,64 +74,46 @@ def tune_backproject(g, image, normfac, prompt, add, subsets=(0, 8), repeats=2, 
     return best_w, results
 
 
+def _forward_times(g, step, subsets, repeats, candidates):
+    """{shape: ms per forward launch}, the least of `repeats` rounds over all candidates (the first ones meet a GPU whose
+    clock still rises: one after the other, two shapes of the same kernel came out 10 % apart)."""
+    import torch
+    results = {}
+    for _ in range(repeats):
+        for shape in candidates:
+            try:
+                g.set_launch_shape(*shape)
+            except Exception:
+                continue
+            step(subsets[0])                      # warm-up / first launch of this variant
+            torch.cuda.synchronize()
+            g.timing_enable(True)
+            for s in subsets:
+                step(s)
+            ms, n = g.timing_read()["fp_ratio"]
+            g.timing_enable(False)
+            results[shape] = min(results.get(shape, float("inf")), ms / max(n, 1))
+    return results
+
+
 def tune_forward(g, image, normfac, prompt, add, subsets=(0, 8), repeats=2, candidates=CANDIDATES):
     """Return ((tasks_per_thread, workgroups_per_ray), {shape: ms per forward launch})."""
-    import torch
     work = image.clone()
-    results = {}
-    for shape in candidates:
-        try:
-            g.set_launch_shape(*shape)
-        except Exception:
-            continue
-        g.osem_subset(work, normfac, prompt, add, subsets[0])      # warm-up / first launch of this variant
-        torch.cuda.synchronize()
-        g.timing_enable(True)
-        for _ in range(repeats):
-            for s in subsets:
-                g.osem_subset(work, normfac, prompt, add, s)
-        kt = g.timing_read()
-        g.timing_enable(False)
-        ms, n = kt["fp_ratio"]
-        results[shape] = ms / max(n, 1)
+    results = _forward_times(g, lambda s: g.osem_subset(work, normfac, prompt, add, s), subsets, repeats, candidates)
     best = _choose(results)
     g.set_launch_shape(*best)
-    del work
     return best, results
 
 
 def tune_frames(g, images, normfac, prompts, adds, mixed=False, subsets=(0, 8), repeats=2, candidates=CANDIDATES):
     """Forward launch shape for the batched path (hrrt_osem_subset_frames, or the FP16-input
-    form with mixed=True): every candidate timed on one subset update of all frames, the
+    form with mixed=True): every candidate timed on subset updates of all frames, the
     fastest kept on the context.  Shapes give bit-identical results; a new shape drops the
     context's captured iteration graphs, which the next iteration call captures again.
     Returns ((tasks_per_thread, workgroups_per_ray), {shape: ms per forward launch})."""
-    import torch
     work = images.clone()
-    results = {}
-
-    def run(s):
-        if mixed:
-            g.osem_subset_frames_mixed(work, normfac, prompts, adds, s)
-        else:
-            g.osem_subset_frames(work, normfac, prompts, adds, s)
-
-    for shape in candidates:
-        try:
-            g.set_launch_shape(*shape)
-        except Exception:
-            continue
-        run(subsets[0])                       # warm-up / first launch of this variant
-        torch.cuda.synchronize()
-        g.timing_enable(True)
-        for _ in range(repeats):
-            for s in subsets:
-                run(s)
-        kt = g.timing_read()
-        g.timing_enable(False)
-        ms, n = kt["fp_ratio"]
-        results[shape] = ms / max(n, 1)
+    update = g.osem_subset_frames_mixed if mixed else g.osem_subset_frames
+    results = _forward_times(g, lambda s: update(work, normfac, prompts, adds, s), subsets, repeats, candidates)
     best = _choose(results)
     g.set_launch_shape(*best)
-    del work
     return best, results
