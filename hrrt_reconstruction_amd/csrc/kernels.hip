@@ -1432,10 +1432,10 @@ __global__ void __launch_bounds__(256) paircol_to_estimate_kernel(const DevGeom 
 
 // estimate [2S][N] -> pair-column with the back-projection rescale; the
 // estimate itself is rescaled in place as back_proj3d2 does (PJ:1496-1507).  A small scanner has few tiles and
-// then the latency of a thread's loads is what counts: a thread takes four elements, and every load is unconditional (a guard,
-// or a bin or plane past the end, reads an element inside) so that they are in flight together.  Direct back
-// projection of a view pair, 48 rings at 92 x 92: 33.8 -> 29.1 us (sixteen elements, each behind its tests); 104 rings
-// at 256 x 256: 205 -> 202.
+// then the latency of a thread's loads is what counts: a thread takes four elements, and no load waits for the test of
+// another (the tables are read for guards and planes past the end too, at an index inside).  Direct back
+// projection of a view pair, 48 rings at 92 x 92: 33.8 -> 28.2 us (sixteen elements, each behind its tests); 104 rings
+// at 256 x 256: 205 -> 200.
 constexpr int EP = 4;
 __global__ void __launch_bounds__(64 * LT / EP) estimate_to_paircol_kernel(const DevGeom g, float *__restrict__ prj,
                                                                          float *__restrict__ pc) {
@@ -1450,15 +1450,19 @@ __global__ void __launch_bounds__(64 * LT / EP) estimate_to_paircol_kernel(const
 #pragma unroll
     for (int i = 0; i < EP; i++) {
         const int sg = max(s[i], 0);
-        p[i] = s[i] < 0 ? 0 : g.segment_offset[sg] + min(q0 + w + ROWS * i, g.spp - 1) - g.seg_data[sg];
+        p[i] = g.segment_offset[sg] + min(q0 + w + ROWS * i, g.spp - 1) - g.seg_data[sg];
         r[i] = g.bp_rescale[sg];
     }
 #pragma unroll
-    for (int i = 0; i < EP; i++) v[i] = prj[((size_t)h * g.S + p[i]) * N + min(col, N - 1)];
+    for (int i = 0; i < EP; i++) {
+        if (col >= N || q0 + w + ROWS * i >= g.spp) s[i] = -1;
+        v[i] = 0.0f;
+        if (s[i] >= 0) v[i] = prj[((size_t)h * g.S + p[i]) * N + col];
+    }
 #pragma unroll
     for (int i = 0; i < EP; i++) {
         const float e = v[i] * r[i];
-        if (s[i] >= 0 && col < N && q0 + w + ROWS * i < g.spp) prj[((size_t)h * g.S + p[i]) * N + col] = e;
+        if (s[i] >= 0) prj[((size_t)h * g.S + p[i]) * N + col] = e;
         tile[w + ROWS * i][t] = e;
     }
     __syncthreads();
